@@ -2744,19 +2744,24 @@ grs_status grs_distance_from_mask(grs_ctx *c) {
   if (c->mnz < 1) return fail(c, GRS_ERR_STATE, "no mask: render or set one first");
   HIPCHK(c, hipSetDevice(c->device));
   const int64_t nz = c->mnz, ny = c->mny, nr = c->mnrot, n = nz * ny * nr;
-  ENSURE(c, c->d_g1, sizeof(int32_t) * n);
   ENSURE(c, c->d_keys, sizeof(float) * n);
-  HIPCHK(c, grs_launch_edt_cols(P<uint8_t>(c->d_mask), nz, ny * nr, P<int32_t>(c->d_g1), c->st));
-  int64_t per_slice = nz * ny * (int64_t)(sizeof(int32_t) + sizeof(double));
-  int64_t ns = ((int64_t)1536 << 20) / (per_slice > 0 ? per_slice : 1);
-  if (ns < 1) ns = 1;
-  if (ns > nr) ns = nr;
-  ENSURE(c, c->d_edt_v, sizeof(int32_t) * (size_t)(nz * ny * ns));
-  ENSURE(c, c->d_edt_z, sizeof(double) * (size_t)(nz * ny * ns));
-  for (int64_t s0 = 0; s0 < nr; s0 += ns) {
-    int64_t k = nr - s0 < ns ? nr - s0 : ns;
-    HIPCHK(c, grs_launch_edt_rows(P<int32_t>(c->d_g1), nz, ny, s0, k, P<int32_t>(c->d_edt_v),
-                                  P<double>(c->d_edt_z), P<float>(c->d_keys), c->st));
+  if (grs_edt_tile_width(nz, ny, nr) > 0) {
+    ENSURE(c, c->d_g1, (size_t)grs_edt_work_bytes(nz, ny * nr));
+    HIPCHK(c, grs_launch_edt(P<uint8_t>(c->d_mask), nz, ny, nr, c->d_g1.p, P<float>(c->d_keys), c->st));
+  } else {
+    ENSURE(c, c->d_g1, sizeof(int32_t) * n);
+    HIPCHK(c, grs_launch_edt_cols(P<uint8_t>(c->d_mask), nz, ny * nr, P<int32_t>(c->d_g1), c->st));
+    int64_t per_slice = nz * ny * (int64_t)(sizeof(int32_t) + sizeof(double));
+    int64_t ns = ((int64_t)1536 << 20) / (per_slice > 0 ? per_slice : 1);
+    if (ns < 1) ns = 1;
+    if (ns > nr) ns = nr;
+    ENSURE(c, c->d_edt_v, sizeof(int32_t) * (size_t)(nz * ny * ns));
+    ENSURE(c, c->d_edt_z, sizeof(double) * (size_t)(nz * ny * ns));
+    for (int64_t s0 = 0; s0 < nr; s0 += ns) {
+      int64_t k = nr - s0 < ns ? nr - s0 : ns;
+      HIPCHK(c, grs_launch_edt_rows(P<int32_t>(c->d_g1), nz, ny, s0, k, P<int32_t>(c->d_edt_v),
+                                    P<double>(c->d_edt_z), P<float>(c->d_keys), c->st));
+    }
   }
   HIPCHK(c, hipStreamSynchronize(c->st));
   c->snz = nz;

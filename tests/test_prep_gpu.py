@@ -38,6 +38,28 @@ def test_edt_matches_scipy_bitwise(engine):
             assert np.isinf(d[:, :, i]).all()
 
 
+@pytest.mark.parametrize("nz, ny", [(1, 1), (63, 16), (64, 17), (65, 33), (129, 250), (20, 1203), (70, 1204), (33, 2409),
+                                    (17, 4817), (4096, 18), (4097, 18)])
+def test_edt_at_tile_edges(engine, nz, ny):
+    """Tile widths, partial tiles, row counts around the steps and the sides
+    where another kernel takes over; few spots (long searches), many, none."""
+    rng = np.random.default_rng(nz * 10007 + ny)
+    mask = np.zeros((nz, ny, 4), bool)
+    mask[rng.integers(nz), rng.integers(ny), 0] = True
+    mask[:, :, 1] = rng.random((nz, ny)) < 3.0 / (nz * ny)
+    mask[:, :, 2] = rng.random((nz, ny)) < 0.02
+    mask[0, 0, 2] = True
+    engine.set_binary_stack(mask)
+    engine.distance_from_mask()
+    d = engine.get_distance_stack(mask.shape)
+    for i in range(4):
+        if mask[:, :, i].any():
+            ref = ndimage.distance_transform_edt(~mask[:, :, i]).astype(np.float32)
+        else:
+            ref = np.full((nz, ny), np.inf, np.float32)
+        assert np.array_equal(d[:, :, i].view(np.uint32), ref.view(np.uint32)), i
+
+
 def test_rendered_scene_scores_one_at_truth(engine):
     s = scenes.make_scene(seed=73, ngrains=3, dilate=1)
     engine.set_geometry(s.geo, s.hkl, s.rot)
