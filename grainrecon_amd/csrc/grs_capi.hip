@@ -1292,9 +1292,9 @@ grs_status grs_spot_residual(grs_ctx *c, const double *geo7, const double *grain
                                      P<int32_t>(c->f_grain), P<double>(c->f_gr6), d_up, P<double>(c->f_res),
                                      d_contrib, d_jac, c->st));
   if (grad7) {
-    ENSURE(c, c->f_out, sizeof(double) * (7 + 6 * G));
+    ENSURE(c, c->f_out, sizeof(double) * (7 + 6 * G + grs_grad_part_doubles()));
     HIPCHK(c, grs_launch_grad_reduce(d_contrib, n, P<int64_t>(c->f_goff), G, P<double>(c->f_out),
-                                     P<double>(c->f_out) + 7, c->st));
+                                     P<double>(c->f_out) + 7, P<double>(c->f_out) + 7 + 6 * G, c->st));
   }
   if (c->timing) HIPCHK(c, timing_end(c));
   HIPCHK(c, hipMemcpyAsync(resid, c->f_res.p, sizeof(double) * 2 * n, hipMemcpyDeviceToHost, c->st));

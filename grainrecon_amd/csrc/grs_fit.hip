@@ -273,32 +273,45 @@ __global__ void k_spot_residual(grs_fitc f, int64_t n, const double *hkl, const 
   }
 }
 
-/* per-grain sums of the 6 grain components (spots sorted by grain) */
-__global__ void k_grain_reduce(const double *contrib, const int64_t *goff, int64_t G, double *out6) {
-  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= G * 6) return;
-  int64_t gidx = t / 6;
-  int k = (int)(t - gidx * 6);
-  double acc = 0.0;
-  for (int64_t i = goff[gidx]; i < goff[gidx + 1]; i++) acc += contrib[13 * i + 7 + k];
-  out6[t] = acc;
+/* Gradient sums, one wave per output block: block g < G adds the 6 grain
+ * components of grain g's spots, block G + b the 7 geometry components of
+ * spots b, b + nb, ... (nb blocks).  Lane l takes every 64th spot and the lanes are added
+ * by halves: a fixed order, so the sums are reproducible.  Bound: reading the
+ * 13 doubles per spot once from L2; a thread per (grain, component) walking its
+ * spots and one block for the geometry took 100 + 97 us for 75,000 spots of
+ * 300 grains, latency of the serial chains; this takes 6 us + 4 us. */
+#define GRS_GEO_BLOCKS 256
+
+__global__ __launch_bounds__(64) void k_grad_reduce(const double *contrib, int64_t n, const int64_t *goff, int64_t G,
+                                                    double *out6, double *part7) {
+  const int lane = threadIdx.x;
+  const int64_t b = blockIdx.x;
+  const bool grain = b < G;
+  const int64_t i0 = grain ? goff[b] + lane : (b - G) * 64 + lane;
+  const int64_t i1 = grain ? goff[b + 1] : n, step = grain ? 64 : (int64_t)GRS_GEO_BLOCKS * 64;
+  const double *c = contrib + (grain ? 7 : 0);
+  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+  for (int64_t i = i0; i < i1; i += step)
+#pragma unroll
+    for (int k = 0; k < 7; k++)
+      if (k < 6 || !grain) acc[k] += c[13 * i + k];
+#pragma unroll
+  for (int k = 0; k < 7; k++)
+    for (int off = 32; off >= 1; off >>= 1) acc[k] += __shfl_xor(acc[k], off, 64);
+  if (lane == 0) {
+    double *o = grain ? out6 + 6 * b : part7 + 7 * (b - G);
+    for (int k = 0; k < (grain ? 6 : 7); k++) o[k] = acc[k];
+  }
 }
 
-/* the 7 geometry components, fixed-order reduction in one block */
-__global__ __launch_bounds__(256) void k_geo_reduce(const double *contrib, int64_t n, double *out7) {
-  __shared__ double part[7][256];
-  int tid = threadIdx.x;
-  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-  for (int64_t i = tid; i < n; i += 256)
-    for (int k = 0; k < 7; k++) acc[k] += contrib[13 * i + k];
-  for (int k = 0; k < 7; k++) part[k][tid] = acc[k];
-  __syncthreads();
-  for (int w = 128; w >= 1; w >>= 1) {
-    if (tid < w)
-      for (int k = 0; k < 7; k++) part[k][tid] += part[k][tid + w];
-    __syncthreads();
-  }
-  if (tid < 7) out7[tid] = part[tid][0];
+/* out[j] = sum over i of part[ncol * i + j]: block j, 64 partial sums added by
+ * halves.  One thread per column walking 300 rows took 72 us, this takes 4 us. */
+__global__ __launch_bounds__(64) void k_column_sum(const double *part, int64_t n, int32_t ncol, double *out) {
+  const int lane = threadIdx.x, j = blockIdx.x;
+  double acc = 0.0;
+  for (int64_t i = lane; i < n; i += 64) acc += part[ncol * i + j];
+  for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if (lane == 0) out[j] = acc;
 }
 
 /* Gauss-Newton normal equations of the block-arrow system, one block per grain
@@ -390,15 +403,6 @@ __global__ __launch_bounds__(GRS_NE_T) void k_spot_normal(grs_fitc f, const doub
     partial[37 * g + (t - 69)] = acc;
 }
 
-/* the grains' shares of Agg, bg and the two sums added in grain order */
-__global__ void k_normal_sum(const double *partial, int64_t G, double *out37) {
-  const int j = threadIdx.x;
-  if (j >= 37) return;
-  double acc = 0.0;
-  for (int64_t g = 0; g < G; g++) acc += partial[37 * g + j];
-  out37[j] = acc;
-}
-
 hipError_t grs_launch_spot_normal(const void *fitc, int64_t G, const double *hkl, const double *omega,
                                   const double *meas, const int64_t *goff, const double *gr6, double delta,
                                   double *pergrain, double *partial, double *out37, hipStream_t st) {
@@ -406,7 +410,7 @@ hipError_t grs_launch_spot_normal(const void *fitc, int64_t G, const double *hkl
   const grs_fitc &f = *static_cast<const grs_fitc *>(fitc);
   hipLaunchKernelGGL(k_spot_normal, dim3((unsigned)G), dim3(GRS_NE_T), 0, st, f, hkl, omega, meas, goff, gr6, delta,
                      pergrain, partial);
-  hipLaunchKernelGGL(k_normal_sum, dim3(1), dim3(64), 0, st, partial, G, out37);
+  hipLaunchKernelGGL(k_column_sum, dim3(37), dim3(64), 0, st, partial, G, 37, out37);
   return hipGetLastError();
 }
 
@@ -420,12 +424,13 @@ hipError_t grs_launch_spot_residual(const void *fitc, int64_t n, const double *h
   return hipGetLastError();
 }
 
+int64_t grs_grad_part_doubles(void) { return 7 * GRS_GEO_BLOCKS; }
+
 hipError_t grs_launch_grad_reduce(const double *contrib, int64_t n, const int64_t *goff, int64_t G, double *out7,
-                                  double *out6, hipStream_t st) {
-  hipLaunchKernelGGL(k_geo_reduce, dim3(1), dim3(256), 0, st, contrib, n, out7);
-  if (G > 0)
-    hipLaunchKernelGGL(k_grain_reduce, dim3((unsigned)((G * 6 + 127) / 128)), dim3(128), 0, st, contrib, goff, G,
-                       out6);
+                                  double *out6, double *part7, hipStream_t st) {
+  hipLaunchKernelGGL(k_grad_reduce, dim3((unsigned)(G + GRS_GEO_BLOCKS)), dim3(64), 0, st, contrib, n, goff, G, out6,
+                     part7);
+  hipLaunchKernelGGL(k_column_sum, dim3(7), dim3(64), 0, st, part7, (int64_t)GRS_GEO_BLOCKS, 7, out7);
   return hipGetLastError();
 }
 
