@@ -97,7 +97,7 @@ struct grs_ctx {
   DevBuf v_vol[4], r_rows, r_counts, r_acc_lin, r_acc_C;
   int64_t v_dim[3] = {0, 0, 0};
   /* G-vector matching score buffers */
-  DevBuf t_pos, t_proj, t_units, t_fam, t_dposs, t_glen, t_scratch, t_out, t_skey, t_su, t_bst, t_slen, t_sorig;
+  DevBuf t_pos, t_proj, t_band, t_units, t_fam, t_dposs, t_glen, t_scratch, t_out, t_skey, t_su, t_bst, t_slen, t_sorig;
   DevBuf v_lin, v_out; /* grs_get_volume_at */
   /* grain centre-of-mass fit buffers */
   DevBuf m_rows, m_rptr, m_nm, m_cs, m_dis;
@@ -317,7 +317,7 @@ void grs_destroy(grs_ctx *c) {
                     &c->r_rows, &c->r_counts, &c->r_acc_lin, &c->r_acc_C, &c->t_pos, &c->t_proj, &c->t_units,
                     &c->t_fam, &c->t_dposs, &c->t_glen, &c->t_scratch, &c->t_out, &c->m_rows, &c->m_rptr,
                     &c->m_nm, &c->t_skey, &c->t_su, &c->t_bst, &c->t_slen, &c->t_sorig, &c->v_lin,
-                    &c->v_out, &c->f_in, &c->f_cnt, &c->m_cs, &c->m_dis};
+                    &c->v_out, &c->f_in, &c->f_cnt, &c->m_cs, &c->m_dis, &c->t_band};
   if (c->g_exec) hipGraphExecDestroy(c->g_exec);
   for (auto &kv : c->gi_cache) hipGraphExecDestroy(kv.second);
   for (hipEvent_t e : c->tev) hipEventDestroy(e);
@@ -2460,6 +2460,7 @@ grs_status grs_forward_gt(grs_ctx *c, const double *pos, const double *q, int64_
   const int64_t wslots = ((waves + 3) / 4) * 4;
   ENSURE(c, c->t_pos, sizeof(double) * 3);
   ENSURE(c, c->t_proj, sizeof(double) * 18 * (size_t)c->nrot);
+  ENSURE(c, c->t_band, sizeof(double) * 2 * (size_t)c->nrot);
   ENSURE(c, c->t_units, sizeof(double) * 12 * (size_t)(nsp > 0 ? nsp : 1));
   ENSURE(c, c->t_fam, sizeof(int32_t) * (size_t)c->H);
   ENSURE(c, c->t_dposs, sizeof(double) * 4);
@@ -2496,9 +2497,11 @@ grs_status grs_forward_gt(grs_ctx *c, const double *pos, const double *q, int64_
     HIPCHK(c, grs_launch_gt_sort(P<int64_t>(c->p_fptr), c->nrot, P<double>(c->t_units), nsp, c->p_maxframe,
                                  P<double>(c->t_skey), P<double>(c->t_su), P<int32_t>(c->t_sorig),
                                  P<int32_t>(c->t_bst), P<int32_t>(c->t_slen), c->st));
-  HIPCHK(c, grs_launch_gt_score(P<grs_dgeo>(c->d_geo), P<double>(c->d_hkl), P<int32_t>(c->t_fam),
+  HIPCHK(c, grs_launch_gt_band(P<double>(c->t_proj), P<int64_t>(c->p_fptr), c->nrot, P<double>(c->t_units), F,
+                               P<double>(c->t_band), c->st));
+  HIPCHK(c, grs_launch_gt_score(P<grs_dgeo>(c->d_geo), P<double>(c->d_hkl), c->H, P<int32_t>(c->t_fam),
                                 P<double>(c->t_glen), P<double>(c->d_sub), P<int32_t>(c->d_valid), N,
-                                P<double>(c->t_proj), P<int64_t>(c->p_fptr), P<double>(c->t_units),
+                                P<double>(c->t_proj), P<double>(c->t_band), P<int64_t>(c->p_fptr), P<double>(c->t_units),
                                 sorted ? P<double>(c->t_skey) : nullptr, sorted ? P<double>(c->t_su) : nullptr,
                                 sorted ? P<int32_t>(c->t_sorig) : nullptr, sorted ? P<int32_t>(c->t_bst) : nullptr,
                                 sorted ? P<int32_t>(c->t_slen) : nullptr, nsp, semantics == GRS_GT_MATCH ? 1 : 0,

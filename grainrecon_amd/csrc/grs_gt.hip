@@ -44,6 +44,7 @@
 #include <hip/hip_runtime.h>
 
 #include "grs_internal.h"
+#include "grs_resolve.h"
 
 #define GT_PROJ_DOUBLES 18
 #define GT_SORT_MAX 4096 /* spots per projection up to which k_gt_sort keeps them in LDS */
@@ -229,22 +230,105 @@ __device__ __forceinline__ uint64_t gt_lanes_below(uint64_t m, int lane) {
   return lane == 0 ? 0ull : (m & (~0ull >> (64 - lane)));
 }
 
-/* 4 blocks per CU (128 VGPRs): the kernel waits on the window loads, and
- * 4 waves per SIMD hide more of that than 3 unspilled ones (33 vs 50 ms for
- * 8192 orientations x 124k spots) */
+/* lane l's x, l the same in every lane */
+__device__ __forceinline__ double gt_lane(double x, int l) {
+  const uint64_t b = (uint64_t)__double_as_longlong(x);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, l);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+/* band[2 i], band[2 i + 1]: smallest and largest w . u of projection i over its
+ * spots' unit vectors w of the nfam families (u: the incoming beam); +Inf,
+ * -Inf without a finite one */
+__global__ __launch_bounds__(64) void k_gt_band(const double *proj, const int64_t *fptr, const double *units,
+                                                int32_t nfam, double *band) {
+  const int32_t i = blockIdx.x;
+  const double *P = proj + GT_PROJ_DOUBLES * i;
+  double lo = __builtin_inf(), hi = -__builtin_inf();
+  for (int64_t s = fptr[i] + threadIdx.x; s < fptr[i + 1]; s += 64) {
+    for (int32_t j = 0; j < nfam; j++) {
+      const double *w = units + 12 * s + 3 * j;
+      const double d = (P[5] * w[0] + P[6] * w[1]) + P[7] * w[2];
+      lo = d < lo ? d : lo;
+      hi = d > hi ? d : hi;
+    }
+  }
+  for (int off = 32; off >= 1; off >>= 1) {
+    const double a = __shfl_xor(lo, off, 64), b = __shfl_xor(hi, off, 64);
+    lo = a < lo ? a : lo;
+    hi = b > hi ? b : hi;
+  }
+  if (threadIdx.x == 0) {
+    band[2 * i] = lo;
+    band[2 * i + 1] = hi;
+  }
+}
+
+/* the terms of projection i for the exact event pipeline */
+__device__ __forceinline__ void gt_vw(const double *P, grs_vw *v) {
+  v->c = P[0];
+  v->s = P[1];
+  v->SW1 = P[3];
+  v->SW2 = P[4];
+  v->u0 = P[5];
+  v->u1 = P[6];
+  v->u2 = P[7];
+  v->ctr1 = P[8];
+  v->ctr2 = P[9];
+  v->cu1 = P[10];
+  v->cu2 = P[11];
+  v->L2 = P[12];
+  v->k0 = P[13];
+  v->tnum = P[14];
+  v->ov1 = P[15];
+  v->ov2 = P[16];
+}
+
+#define GT_RING 128     /* candidate events queued per wave */
+#define GT_TAB_MAX 1024 /* reflections up to which a wave keeps its G table in LDS (36 bytes each) */
+
+/* One wave per orientation.  About 10% of the (projection, reflection) events
+ * can do anything: the expected count needs cos(beta) and lambda inside the
+ * selection windows, and a match needs the reflection's unit vector n within
+ * GT_WIN of a spot's, so u . n within GT_WIN of the projection's band of
+ * u . w (the spots of a projection lie in the thin shell that diffracts).
+ * Phase A tests both with a dozen operations, lanes over a projection's
+ * reflections, and queues the events that pass (the margins are those of
+ * k_fast's phase A, 1e-12 on cos(beta) and 1e-9 lambda_max, and 1e-6 on the
+ * band; a NaN neither counts nor matches); 64 queued events at a time run the exact
+ * event and the spot search, in (projection, reflection) order (the event
+ * decided by b1_classify, by the exact pipeline where that leaves it open).  Bound: the
+ * dependent loads of the spot search and FP64 arithmetic.  8192 orientations,
+ * 86 reflections, 181 projections, 124,000 spots: 3.3 ms against 28.7 ms
+ * with both run for every event, where a wave always held some lane that
+ * passed a test.  4 blocks per CU (128 VGPRs). */
+template <bool TAB>
 __global__ __launch_bounds__(256, 4) void k_gt_score(const grs_dgeo *g, const double *hkl, const int32_t *famidx,
                                                   const double *glen_poss, const double *SUB, const int32_t *valid,
-                                                  int64_t N, const double *proj, const int64_t *fptr,
+                                                  int64_t N, const double *proj, const double *band,
+                                                  const int64_t *fptr,
                                                   const double *units, const double *skey, const double *su,
                                                   const int32_t *sorig, const int32_t *bst, const int32_t *slen,
                                                   int64_t nsp, int32_t cost_mode, double *scratch, int64_t cap,
                                                   double *out) {
   GRS_NO_CONTRACT
+  extern __shared__ double gts[];
+  __shared__ double thr[12];
+  if (threadIdx.x == 0) b1_thresholds(g, thr);
+  __syncthreads();
   const int32_t H = g->H, nrot = g->nrot;
-  const int lane = threadIdx.x & 63;
-  const int64_t gwave = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, wib = threadIdx.x >> 6;
+  /* per wave: G and 1/|G| of each reflection (4 doubles), the ring, the families */
+  const int32_t Ht = TAB ? H : 0;
+  double *tab = gts + (int64_t)wib * (4 * Ht + GT_RING / 2 + (Ht + 1) / 2);
+  uint32_t *ring = (uint32_t *)(tab + 4 * Ht);
+  int32_t *tfam = (int32_t *)(ring + GT_RING);
+  const int64_t gwave = (int64_t)blockIdx.x * (blockDim.x >> 6) + wib;
   const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x >> 6);
   double *list = scratch + gwave * cap;
+  const double cb_lo = g->cos_beta_max - 1e-12, lm = 1e-9 * g->lambda_max;
+  const double lam_lo = g->lambda_min - lm, lam_hi = g->lambda_max + lm;
   for (int64_t u = gwave; u < N; u += nwaves) {
     double *o = out + 4 * u;
     if (!valid[u]) {
@@ -256,92 +340,118 @@ __global__ __launch_bounds__(256, 4) void k_gt_score(const grs_dgeo *g, const do
     /* calc_Gt_match's cost sums: sum over the matches, in their order, of
      * (n_k - w_k)^2 per component k (ForwardCalc_OR_space_Gt.m:195-197) */
     double c0 = 0.0, c1 = 0.0, c2 = 0.0;
-    for (int32_t i = 0; i < nrot; i++) {
-      const double *P = proj + GT_PROJ_DOUBLES * i;
-      grs_vw v;
-      v.c = P[0];
-      v.s = P[1];
-      v.SW1 = P[3];
-      v.SW2 = P[4];
-      v.u0 = P[5];
-      v.u1 = P[6];
-      v.u2 = P[7];
-      v.ctr1 = P[8];
-      v.ctr2 = P[9];
-      v.cu1 = P[10];
-      v.cu2 = P[11];
-      v.L2 = P[12];
-      v.k0 = P[13];
-      v.tnum = P[14];
-      v.ov1 = P[15];
-      v.ov2 = P[16];
-      const int64_t s0 = fptr[i], s1 = fptr[i + 1];
-      for (int32_t h0 = 0; h0 < H; h0 += 64) {
-        const int32_t h = h0 + lane;
-        bool sel = false, match = false;
-        double amin = 0.0, e0 = 0.0, e1 = 0.0, e2 = 0.0;
-        if (h < H) {
-          double gw[3], Gt[3], Glen;
+    uint32_t head = 0, tail = 0;
+
+    /* the family whose |G| the reflection fits (with a margin), or -1 */
+    auto family = [&](int32_t h, double gn) -> int32_t {
+      const int32_t f = famidx[h];
+      return f >= 0 && __builtin_fabs(gn - glen_poss[f]) < 0.1 + 1e-6 ? f : -1;
+    };
+
+    /* n queued events: the exact event for the expected count, the spot search for a match */
+    auto events = [&](uint32_t n) {
+      bool sel = false, match = false;
+      double amin = 0.0, e0 = 0.0, e1 = 0.0, e2 = 0.0;
+      if ((uint32_t)lane < n) {
+        const uint32_t ev = ring[(head + lane) & (GT_RING - 1)];
+        const int32_t i = (int32_t)((ev >> 2) / (uint32_t)H), h = (int32_t)((ev >> 2) - (uint32_t)i * (uint32_t)H);
+        const double *P = proj + GT_PROJ_DOUBLES * i;
+        double gw[3], Gt[3];
+        if (TAB) {
+          gw[0] = tab[4 * h];
+          gw[1] = tab[4 * h + 1];
+          gw[2] = tab[4 * h + 2];
+        } else {
           grs_Gw(sub, hkl + 3 * h, gw);
-          grs_Gt(v.c, v.s, gw[0], gw[1], gw[2], Gt);
-          const double beta = grs_event_beta(&v, Gt, &Glen);
-          int32_t dy, dz;
-          sel = grs_event_finish(g, &v, Gt, Glen, beta, &dy, &dz) != 0;
+        }
+        grs_Gt(P[0], P[1], gw[0], gw[1], gw[2], Gt);
+        if (ev & 1u) {
+          /* the projection's terms as k_fast's omega_terms names them; the
+           * centre is taken at the effective detector distance, along u */
+          const double bt[10] = {P[5], P[6], P[7], P[13], P[8] - P[3], P[9] - P[4], P[12], P[14], P[15], P[16]};
+          const double gn2 = (gw[0] * gw[0] + gw[1] * gw[1]) + gw[2] * gw[2];
+          const double t5[5] = {gw[0], gw[1], gw[2], fast_rsq(gn2), gn2};
+          b1_out bo;
+          int st = b1_classify(g, P[0], P[1], nullptr, bt, t5, thr, &bo);
+          if (st == 2) {
+            grs_vw v;
+            gt_vw(P, &v);
+            double Glen;
+            const double beta = grs_event_beta(&v, Gt, &Glen);
+            int32_t dy, dz;
+            st = grs_event_finish(g, &v, Gt, Glen, beta, &dy, &dz) != 0;
+          }
+          sel = st != 0;
+        }
+        if (ev & 2u) {
           const int32_t f = famidx[h];
-          if (f >= 0 && s1 > s0) {
-            const double n0 = Gt[0] / Glen, n1 = Gt[1] / Glen, n2 = Gt[2] / Glen;
-            /* spots to visit: the z window of the family's sorted list
-             * (packed unit vectors su, entries lo .. e - 1, found from the
-             * bucket start below zlo), or every spot of the projection */
-            const double *W;
-            int64_t k0, k1;
-            double best = 0.0;
-            bool any = false;
-            if (skey) {
-              const int64_t base = (int64_t)f * nsp + s0;
-              const int32_t mlen = slen[4 * i + f];
-              const double zlo = n2 - GT_WIN, zhi = n2 + GT_WIN;
-              int32_t b = 0;
-              if (zlo == zlo) {
-                const double q = __builtin_floor((zlo + 1.0) * (0.5 * (double)GRS_GT_NB)) - 1.0;
-                b = q < 0.0 ? 0 : (q > (double)GRS_GT_NB ? GRS_GT_NB : (int32_t)q);
-              }
-              int32_t lo = bst[(int64_t)(4 * i + f) * (GRS_GT_NB + 1) + b];
-              W = su + 3 * base;
-              /* the key of a finite entry is its packed z (W[3k + 2]) */
-              while (lo < mlen && W[3 * lo + 2] < zlo) lo++;
-              int32_t k = lo;
-              for (; k < mlen && W[3 * k + 2] <= zhi; k++) {
-                const double *w = W + 3 * k;
-                const double d = (n0 * w[0] + n1 * w[1]) + n2 * w[2];
-                if (d == d && (!any || d > best)) {
-                  best = d;
-                  any = true;
-                }
-              }
-              k0 = lo;
-              k1 = k;
-            } else {
-              W = nullptr;
-              k0 = s0;
-              k1 = s1;
-              for (int64_t k = k0; k < k1; k++) {
-                const double *w = units + 12 * k + 3 * f;
-                const double d = (n0 * w[0] + n1 * w[1]) + n2 * w[2];
-                if (d == d && (!any || d > best)) {
-                  best = d;
-                  any = true;
-                }
-              }
+          const int64_t s0 = fptr[i], s1 = fptr[i + 1];
+          /* |Gt| as grs_event_beta forms it */
+          const double Glen = grs_sqrt((Gt[0] * Gt[0] + Gt[1] * Gt[1]) + Gt[2] * Gt[2]);
+          const double n0 = Gt[0] / Glen, n1 = Gt[1] / Glen, n2 = Gt[2] / Glen;
+          /* spots to visit: the z window of the family's sorted list
+           * (packed unit vectors su, entries lo .. e - 1, found from the
+           * bucket start below zlo), or every spot of the projection */
+          const double *W = nullptr;
+          int64_t k0 = s0, k1 = s1, kb = -1;
+          double best = -__builtin_inf(), second = -__builtin_inf();
+          auto visit = [&](double d, int64_t k) {
+            if (d > best) {
+              second = best;
+              best = d;
+              kb = k;
+            } else if (d > second) {
+              second = d;
             }
-            if (any) {
-              /* the smallest angle and, as MATLAB's min, the first spot (in
-               * the projection's order) that has it: the full scan visits
-               * spots in that order, the window carries their indices */
+          };
+          if (skey) {
+            const int64_t base = (int64_t)f * nsp + s0;
+            const int32_t mlen = slen[4 * i + f];
+            const double zlo = n2 - GT_WIN, zhi = n2 + GT_WIN;
+            /* zlo can round up to the next bucket start only within 1e-15 of
+             * it, and a spot there is more than 1.01 degrees away */
+            int32_t b = 0;
+            if (zlo == zlo) {
+              const double q = __builtin_floor((zlo + 1.0) * (0.5 * (double)GRS_GT_NB));
+              b = q < 0.0 ? 0 : (q > (double)GRS_GT_NB ? GRS_GT_NB : (int32_t)q);
+            }
+            k0 = bst[(int64_t)(4 * i + f) * (GRS_GT_NB + 1) + b];
+            W = su + 3 * base;
+            /* four entries a step, so that their loads are in flight together;
+             * the key of a finite entry is its packed z */
+            int32_t k = (int32_t)k0;
+            while (k < mlen) {
+              double w[4][3];
+#pragma unroll
+              for (int j = 0; j < 4; j++) {
+                const double *e = W + 3 * (k + j < mlen ? k + j : mlen - 1);
+                w[j][0] = e[0];
+                w[j][1] = e[1];
+                w[j][2] = e[2];
+              }
+#pragma unroll
+              for (int j = 0; j < 4; j++)
+                if (k + j < mlen && w[j][2] <= zhi) visit((n0 * w[j][0] + n1 * w[j][1]) + n2 * w[j][2], k + j);
+              k += 4;
+              if (w[3][2] > zhi) break;
+            }
+            k1 = k < mlen ? k : mlen;
+          } else {
+            for (int64_t k = k0; k < k1; k++) {
+              const double *w = units + 12 * k + 3 * f;
+              visit((n0 * w[0] + n1 * w[1]) + n2 * w[2], k);
+            }
+          }
+          if (kb >= 0) {
+            /* the smallest angle and, as MATLAB's min, the first spot (in
+             * the projection's order) that has it: the full scan visits
+             * spots in that order, the window carries their indices */
+            const double lim = best - 1e-12;
+            const double *wbest = W ? W + 3 * kb : units + 12 * kb + 3 * f;
+            amin = best > 1.0 ? 0.0 : (grs_acos(best) * 180.0) / GRS_PI;
+            if (second >= lim) {
               amin = 1e300;
               int64_t aidx = INT64_MAX;
-              const double *wbest = nullptr;
-              const double lim = best - 1e-12;
               for (int64_t k = k0; k < k1; k++) {
                 const double *w = W ? W + 3 * k : units + 12 * k + 3 * f;
                 const double d = (n0 * w[0] + n1 * w[1]) + n2 * w[2];
@@ -355,35 +465,95 @@ __global__ __launch_bounds__(256, 4) void k_gt_score(const grs_dgeo *g, const do
                   }
                 }
               }
-              match = amin < 1.0 && grs_fabs(Glen - glen_poss[f]) < 0.1;
-              if (match && cost_mode) {
-                const double x0 = n0 - wbest[0], x1 = n1 - wbest[1], x2 = n2 - wbest[2];
-                e0 = x0 * x0;
-                e1 = x1 * x1;
-                e2 = x2 * x2;
-              }
+            }
+            match = amin < 1.0 && grs_fabs(Glen - glen_poss[f]) < 0.1;
+            if (match && cost_mode) {
+              const double x0 = n0 - wbest[0], x1 = n1 - wbest[1], x2 = n2 - wbest[2];
+              e0 = x0 * x0;
+              e1 = x1 * x1;
+              e2 = x2 * x2;
             }
           }
         }
-        expect += __popcll(__ballot(sel));
-        const uint64_t mm = __ballot(match);
-        if (match) list[nm + __popcll(gt_lanes_below(mm, lane))] = amin;
-        nm += __popcll(mm);
-        if (cost_mode) {
-          /* the matches of this batch in lane order: every lane adds them
-           * in sequence (the wave-uniform loop keeps the shuffles whole) */
-          for (uint64_t m = mm; m; m &= m - 1) {
-            const int l = __ffsll((long long)m) - 1;
-            c0 = c0 + __shfl(e0, l);
-            c1 = c1 + __shfl(e1, l);
-            c2 = c2 + __shfl(e2, l);
+      }
+      head += n;
+      expect += __popcll(__ballot(sel));
+      const uint64_t mm = __ballot(match);
+      if (match) list[nm + __popcll(gt_lanes_below(mm, lane))] = amin;
+      nm += __popcll(mm);
+      if (cost_mode) {
+        /* the matches of this batch in lane order: every lane adds them
+         * in sequence (the wave-uniform loop keeps the shuffles whole) */
+        for (uint64_t m = mm; m; m &= m - 1) {
+          const int l = __ffsll((long long)m) - 1;
+          c0 = c0 + gt_lane(e0, l);
+          c1 = c1 + gt_lane(e1, l);
+          c2 = c2 + gt_lane(e2, l);
+        }
+      }
+    };
+
+    if (TAB) {
+      for (int32_t h = lane; h < H; h += 64) {
+        double gw[3];
+        grs_Gw(sub, hkl + 3 * h, gw);
+        const double gn = __builtin_sqrt((gw[0] * gw[0] + gw[1] * gw[1]) + gw[2] * gw[2]);
+        tab[4 * h] = gw[0];
+        tab[4 * h + 1] = gw[1];
+        tab[4 * h + 2] = gw[2];
+        tab[4 * h + 3] = 1.0 / gn;
+        tfam[h] = family(h, gn);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    for (int32_t i = 0; i < nrot; i++) {
+      const double *P = proj + GT_PROJ_DOUBLES * i;
+      const double c = P[0], s = P[1], u0 = P[5], u1 = P[6], u2 = P[7];
+      const double blo = band[2 * i] - (GT_WIN + 1e-6), bhi = band[2 * i + 1] + (GT_WIN + 1e-6);
+      for (int32_t h0 = 0; h0 < H; h0 += 64) {
+        const int32_t h = h0 + lane;
+        uint32_t want = 0;
+        if (h < H) {
+          double gw[3], rg;
+          int32_t f;
+          if (TAB) {
+            gw[0] = tab[4 * h];
+            gw[1] = tab[4 * h + 1];
+            gw[2] = tab[4 * h + 2];
+            rg = tab[4 * h + 3];
+            f = tfam[h];
+          } else {
+            grs_Gw(sub, hkl + 3 * h, gw);
+            const double gn = __builtin_sqrt((gw[0] * gw[0] + gw[1] * gw[1]) + gw[2] * gw[2]);
+            rg = 1.0 / gn;
+            f = family(h, gn);
           }
+          const double G0 = c * gw[0] - s * gw[1], G1 = s * gw[0] + c * gw[1];
+          const double cb = __builtin_fma(u0, G0, __builtin_fma(u1, G1, u2 * gw[2])) * rg;
+          const double lam = (-4.0 * GRS_PI) * cb * rg;
+          if (cb < 1e-12 && cb > cb_lo && lam > lam_lo && lam < lam_hi) want = 1u;
+          if (f >= 0 && cb >= blo && cb <= bhi) want |= 2u;
+        }
+        const uint64_t m = __ballot(want != 0u);
+        if (want) ring[(tail + __popcll(gt_lanes_below(m, lane))) & (GT_RING - 1)] = (((uint32_t)i * (uint32_t)H + (uint32_t)h) << 2) | want;
+        tail += (uint32_t)__popcll(m);
+        if (tail - head >= 64u) {
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          events(64u);
         }
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (tail != head) events(tail - head);
     __threadfence_block();
     double med = __builtin_nan(""), mean = __builtin_nan("");
-    if (nm > 0) {
+    if (nm > 0 && !cost_mode) {
       /* ranks with ties broken by position: the elements of rank k1 and k2 */
       const int32_t k1 = (nm & 1) ? (nm >> 1) : (nm >> 1) - 1, k2 = nm >> 1;
       double v1 = 0.0, v2 = 0.0;
@@ -409,11 +579,16 @@ __global__ __launch_bounds__(256, 4) void k_gt_score(const grs_dgeo *g, const do
       v1 = __shfl(v1, l1);
       v2 = __shfl(v2, l2);
       med = (nm & 1) ? v1 : v1 + (v2 - v1) / 2.0;
-      if (lane == 0) {
-        double acc = 0.0;
-        for (int32_t t = 0; t < nm; t++) acc = acc + list[t];
-        mean = acc / (double)nm;
+    }
+    if (nm > 0) {
+      /* the mean adds in list order: 64 angles a load, the lanes' values in turn */
+      double acc = 0.0;
+      for (int32_t b = 0; b < nm; b += 64) {
+        const double x = b + lane < nm ? list[b + lane] : 0.0;
+        const int32_t cnt = nm - b < 64 ? nm - b : 64;
+        for (int32_t t = 0; t < cnt; t++) acc = acc + gt_lane(x, t);
       }
+      mean = acc / (double)nm;
     }
     if (lane == 0) {
       o[0] = (double)nm;
@@ -469,17 +644,30 @@ hipError_t grs_launch_gt_sort(const int64_t *d_fptr, int32_t nrot, const double 
 
 int64_t grs_gt_sort_max() { return GT_SORT_MAX; }
 
-hipError_t grs_launch_gt_score(const grs_dgeo *d_g, const double *d_hkl, const int32_t *d_famidx,
+hipError_t grs_launch_gt_band(const double *d_proj, const int64_t *d_fptr, int32_t nrot, const double *d_units,
+                              int32_t nfam, double *d_band, hipStream_t st) {
+  if (nrot <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_gt_band, dim3((unsigned)nrot), dim3(64), 0, st, d_proj, d_fptr, d_units, nfam, d_band);
+  return hipGetLastError();
+}
+
+hipError_t grs_launch_gt_score(const grs_dgeo *d_g, const double *d_hkl, int32_t H, const int32_t *d_famidx,
                                const double *d_glen_poss, const double *d_SUB, const int32_t *d_valid, int64_t N,
-                               const double *d_proj, const int64_t *d_fptr, const double *d_units,
+                               const double *d_proj, const double *d_band, const int64_t *d_fptr, const double *d_units,
                                const double *d_skey, const double *d_su, const int32_t *d_sorig,
                                const int32_t *d_bst, const int32_t *d_slen, int64_t nsp, int32_t cost_mode,
                                double *d_scratch, int64_t cap, int64_t waves, double *d_out, hipStream_t st) {
   if (N <= 0) return hipSuccess;
   int64_t w = waves < N ? waves : N;
   const int64_t blocks = (w + 3) / 4;
-  hipLaunchKernelGGL(k_gt_score, dim3((unsigned)blocks), dim3(256), 0, st, d_g, d_hkl, d_famidx, d_glen_poss, d_SUB,
-                     d_valid, N, d_proj, d_fptr, d_units, d_skey, d_su, d_sorig, d_bst, d_slen, nsp, cost_mode, d_scratch,
-                     cap, d_out);
+  const bool tab = H <= GT_TAB_MAX;
+  const size_t lds = 4 * sizeof(double) * (size_t)(tab ? 4 * H + GT_RING / 2 + (H + 1) / 2 : GT_RING / 2);
+  const auto kernel = tab ? &k_gt_score<true> : &k_gt_score<false>;
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), lds, st, d_g, d_hkl, d_famidx, d_glen_poss, d_SUB,
+                     d_valid, N, d_proj, d_band, d_fptr, d_units, d_skey, d_su, d_sorig, d_bst, d_slen, nsp, cost_mode,
+                     d_scratch, cap, d_out);
   return hipGetLastError();
 }

@@ -239,12 +239,15 @@ hipError_t grs_launch_gt_sort(const int64_t *d_fptr, int32_t nrot, const double 
                               int64_t max_frame, double *d_skey, double *d_su, int32_t *d_sorig, int32_t *d_bst,
                               int32_t *d_slen, hipStream_t st);
 int64_t grs_gt_sort_max();
+/* d_band: 2*nrot, the range of beam . spot unit vector per projection */
+hipError_t grs_launch_gt_band(const double *d_proj, const int64_t *d_fptr, int32_t nrot, const double *d_units,
+                              int32_t nfam, double *d_band, hipStream_t st);
 /* d_skey == nullptr: every spot of a projection is visited.  cost_mode != 0:
  * rows [Nr_match, matched cost, ratio, mean] (calc_Gt_match), else
  * [Nr_match, median angle, ratio, mean] (calc_Gt_match_fun) */
-hipError_t grs_launch_gt_score(const grs_dgeo *d_g, const double *d_hkl, const int32_t *d_famidx,
+hipError_t grs_launch_gt_score(const grs_dgeo *d_g, const double *d_hkl, int32_t H, const int32_t *d_famidx,
                                const double *d_glen_poss, const double *d_SUB, const int32_t *d_valid, int64_t N,
-                               const double *d_proj, const int64_t *d_fptr, const double *d_units,
+                               const double *d_proj, const double *d_band, const int64_t *d_fptr, const double *d_units,
                                const double *d_skey, const double *d_su, const int32_t *d_sorig,
                                const int32_t *d_bst, const int32_t *d_slen, int64_t nsp, int32_t cost_mode,
                                double *d_scratch, int64_t cap, int64_t waves, double *d_out, hipStream_t st);

@@ -193,3 +193,24 @@ def test_forward_gt_dense_spots_and_full_scan(engine, scene):
             same = (got == ref) | (np.isnan(got) & np.isnan(ref))
             assert same.all(), (name, sname, np.argwhere(~same)[:5])
             assert got[:3, 0].min() > 10
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [1, 63, 65, 128, 1024, 1025])
+def test_forward_gt_reflection_counts(engine, scene, H):
+    """One and several passes of 64 reflections, queues that never fill and
+    that fill at every pass, and the counts around the reflection table's
+    limit (reflections repeated: each is scored by itself)."""
+    s = scene
+    hkl = np.concatenate([s.hkl] * (H // s.hkl.shape[0] + 1))[:H]
+    engine.set_geometry(s.geo, hkl, s.rot)
+    engine.set_distance_stack(s.proj)
+    rng = np.random.default_rng(47)
+    frames = _frames(s, rng)
+    engine.set_frame_spots(frames)
+    fam_sq, dposs = _families(s)
+    q = np.concatenate([s.q[:1], s.q[:1] + rng.normal(scale=0.003, size=(1, 4)) * [0, 1, 1, 1], scenes.random_quats(rng, 3)])
+    for sem, name in ((_lib.GT_MATCH, "match"), (_lib.GT_MATCH_FUN, "fun")):
+        got = engine.forward_gt(s.centers[0], q, fam_sq, dposs, sem)
+        ref = GM.gt_score(s.geo, s.centers[0], q, s.rot, hkl, frames, fam_sq, dposs, semantics=name)
+        assert np.array_equal(got, ref, equal_nan=True), name
