@@ -808,67 +808,52 @@ grs_status grs_grow_indexed_region(grs_ctx *c, const double *vox, int64_t M, con
   grs_status s = check_ready(c);
   if (s != GRS_OK) return s;
   if (M == 0) return GRS_OK;
-  /* only voxels inside the mask are scored */
-  std::vector<int64_t> idx;
-  idx.reserve(M);
-  for (int64_t i = 0; i < M; i++) {
-    double *o = out + 7 * i;
-    o[0] = vox[6 * i];
-    o[1] = vox[6 * i + 1];
-    o[2] = vox[6 * i + 2];
-    o[3] = o[4] = o[5] = o[6] = 0.0;
-    if (vox[6 * i + 4] > 0.0) idx.push_back(i);
-  }
-  ENSURE(c, c->d_U, sizeof(double) * 9);
   ENSURE(c, c->d_sub, sizeof(double) * 9);
   ENSURE(c, c->d_valid, sizeof(int32_t));
-  ENSURE(c, c->d_p1, sizeof(double) * 14);
-  HIPCHK(c, hipMemcpyAsync(c->d_U.p, U, sizeof(double) * 9, hipMemcpyHostToDevice, c->st));
-  HIPCHK(c, hipMemcpyAsync(c->d_p1.p, p1, sizeof(double) * 14, hipMemcpyHostToDevice, c->st));
-  HIPCHK(c, grs_launch_sub_from_U(P<grs_dgeo>(c->d_geo), P<double>(c->d_U), 1, P<double>(c->d_sub),
+  ENSURE(c, c->d_p1, sizeof(double) * (14 + 9)); /* param1, then U */
+  double p1U[14 + 9];
+  std::memcpy(p1U, p1, sizeof(double) * 14);
+  std::memcpy(p1U + 14, U, sizeof(double) * 9);
+  HIPCHK(c, hipMemcpyAsync(c->d_p1.p, p1U, sizeof(p1U), hipMemcpyHostToDevice, c->st));
+  HIPCHK(c, grs_launch_sub_from_U(P<grs_dgeo>(c->d_geo), P<double>(c->d_p1) + 14, 1, P<double>(c->d_sub),
                                   P<int32_t>(c->d_valid), c->st));
   const int64_t chunk = voxel_chunk(c);
-  std::vector<double> rows;
-  std::vector<int32_t> hns, hni;
-  std::vector<double> hC;
-  std::vector<float> hmed;
-  for (int64_t b = 0; b < (int64_t)idx.size(); b += chunk) {
-    int64_t m = (int64_t)idx.size() - b;
-    if (m > chunk) m = chunk;
-    rows.resize(3 * m);
-    for (int64_t k = 0; k < m; k++)
-      for (int j = 0; j < 3; j++) rows[3 * k + j] = vox[6 * idx[b + k] + j];
-    ENSURE(c, c->d_rows, sizeof(double) * 3 * m);
+  for (int64_t b = 0; b < M; b += chunk) {
+    const int64_t m = M - b < chunk ? M - b : chunk;
+    /* only voxels inside the mask are scored: counted here while that is
+     * quicker than a round trip (a pass over the rows' mask column) */
+    int64_t E = -1;
+    if (m <= 16384) {
+      E = 0;
+      for (int64_t i = b; i < b + m; i++) E += vox[6 * i + 4] > 0.0 ? 1 : 0;
+    }
+    const int64_t nb = grs_grow_blocks(m);
+    ENSURE(c, c->d_rows, sizeof(double) * 6 * m);
     ENSURE(c, c->d_pos, sizeof(double) * 3 * m);
-    ENSURE(c, c->d_ns, sizeof(int32_t) * m);
-    ENSURE(c, c->d_ni, sizeof(int32_t) * m);
-    ENSURE(c, c->d_C, sizeof(double) * m);
-    ENSURE(c, c->d_med, sizeof(float) * m);
-    HIPCHK(c, hipMemcpyAsync(c->d_rows.p, rows.data(), sizeof(double) * 3 * m, hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, grs_launch_voxel_pos(P<double>(c->d_rows), m, 3, P<double>(c->d_p1), P<double>(c->d_pos), c->st));
-    s = run_eval(c, GRS_MAP_ONE_U, m, m, nullptr, nullptr, method, P<int32_t>(c->d_ns), P<int32_t>(c->d_ni),
+    ENSURE(c, c->d_evox, sizeof(int32_t) * m); /* a row's place among the scored ones */
+    ENSURE(c, c->d_rowstart, sizeof(int64_t) + sizeof(int32_t) * nb);
+    ENSURE(c, c->d_eu, sizeof(double) * 7 * m); /* output rows */
+    HIPCHK(c, hipMemcpyAsync(c->d_rows.p, vox + 6 * b, sizeof(double) * 6 * m, hipMemcpyHostToDevice, c->st));
+    int64_t *d_total = P<int64_t>(c->d_rowstart);
+    int32_t *d_count = E == m ? nullptr : reinterpret_cast<int32_t *>(d_total + 1);
+    HIPCHK(c, grs_launch_grow_list(P<double>(c->d_rows), m, P<double>(c->d_p1), d_count, P<double>(c->d_pos),
+                                   P<int32_t>(c->d_evox), d_total, c->st));
+    if (E < 0) {
+      HIPCHK(c, hipMemcpyAsync(&E, d_total, sizeof(E), hipMemcpyDeviceToHost, c->st));
+      HIPCHK(c, hipStreamSynchronize(c->st));
+    }
+    ENSURE(c, c->d_ns, sizeof(int32_t) * E);
+    ENSURE(c, c->d_ni, sizeof(int32_t) * E);
+    ENSURE(c, c->d_C, sizeof(double) * E);
+    ENSURE(c, c->d_med, sizeof(float) * E);
+    s = run_eval(c, GRS_MAP_ONE_U, E, E, nullptr, nullptr, method, P<int32_t>(c->d_ns), P<int32_t>(c->d_ni),
                  P<double>(c->d_C), P<float>(c->d_med));
     if (s != GRS_OK) return s;
-    hns.resize(m);
-    hni.resize(m);
-    hC.resize(m);
-    hmed.resize(m);
-    HIPCHK(c, hipMemcpyAsync(hns.data(), c->d_ns.p, sizeof(int32_t) * m, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipMemcpyAsync(hni.data(), c->d_ni.p, sizeof(int32_t) * m, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipMemcpyAsync(hC.data(), c->d_C.p, sizeof(double) * m, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipMemcpyAsync(hmed.data(), c->d_med.p, sizeof(float) * m, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(c, grs_launch_grow_out(P<double>(c->d_rows), m, P<double>(c->d_p1), P<int32_t>(c->d_evox),
+                                  P<int32_t>(c->d_ns), P<int32_t>(c->d_ni), P<double>(c->d_C), P<float>(c->d_med),
+                                  P<double>(c->d_eu), c->st));
+    HIPCHK(c, hipMemcpyAsync(out + 7 * b, c->d_eu.p, sizeof(double) * 7 * m, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
-    for (int64_t k = 0; k < m; k++) {
-      const double *v = vox + 6 * idx[b + k];
-      double *o = out + 7 * idx[b + k];
-      double Cn = hC[k], dm = (double)hmed[k];
-      double lim = nanmin2(v[5], p1[13]);
-      bool flag = (Cn > v[3] && dm <= lim) && (Cn >= p1[11] * (1.0 - p1[12]));
-      o[3] = (double)hns[k];
-      o[4] = (double)hni[k];
-      o[5] = dm;
-      o[6] = flag ? 1.0 : 0.0;
-    }
   }
   return GRS_OK;
 }

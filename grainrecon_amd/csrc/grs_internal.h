@@ -207,6 +207,14 @@ hipError_t grs_launch_pair_rows(const grs_dgeo *d_g, const double *d_hkl, const 
                                 const int32_t *d_off, const int64_t *d_row_ptr, double *d_rows, hipStream_t st);
 
 /* region growth (grs_region.hip) */
+/* rows of cuda_grow_indexed_region: d_count (grs_grow_blocks(M) ints) and
+ * d_total, or nullptr when every row is inside the mask */
+int64_t grs_grow_blocks(int64_t M);
+hipError_t grs_launch_grow_list(const double *d_rows, int64_t M, const double *d_p1, int32_t *d_count, double *d_pos,
+                                int32_t *d_slot, int64_t *d_total, hipStream_t st);
+hipError_t grs_launch_grow_out(const double *d_rows, int64_t M, const double *d_p1, const int32_t *d_slot,
+                               const int32_t *d_ns, const int32_t *d_ni, const double *d_C, const float *d_med,
+                               double *d_out, hipStream_t st);
 hipError_t grs_launch_region_list(const double *d_I, const double *d_mask, const double *d_dm, int64_t nx, int64_t ny,
                                   const int64_t *lo, const int64_t *bdim, const double *cp, double boxL,
                                   int64_t seed_lin, double seed_comp, double *d_rows, uint32_t *d_counts,

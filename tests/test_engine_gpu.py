@@ -174,6 +174,28 @@ def test_grow_parity(engine, method):
         assert got[:, 6].sum() > 0
 
 
+@pytest.mark.parametrize("M", [1, 255, 257, 1023, 1024, 16384, 16385, 32768, 262145])
+def test_grow_row_counts(engine, M):
+    """Row counts around the blocks of the row listing and around the rules
+    that choose the voxel-bounds kernel and where the mask is counted; every
+    row inside the mask, some, none."""
+    s = scenes.make_scene(seed=41, ngrains=2, spread_mm=0.02)
+    engine.set_geometry(s.geo, s.hkl, s.rot)
+    engine.set_distance_stack(s.proj)
+    rng = np.random.default_rng(M)
+    vox = np.column_stack([rng.integers(14, 27, (M, 2)), rng.integers(16, 25, M), rng.uniform(0, 0.6, M), np.ones(M),
+                           rng.uniform(0, 30, M)]).astype(float)
+    p1 = _p1()
+    pick = np.unique(np.concatenate([[0, M - 1], rng.integers(0, M, 40)]))
+    for mask in (np.ones(M), (rng.random(M) < 0.7) * 1.0, np.zeros(M)):
+        vox[:, 4] = mask
+        got = engine.grow_indexed_region(vox, s.U[0], p1)
+        ref = oracle.grow(s.geo, s.stack, vox[pick], s.U[0], s.rot, s.hkl, p1)
+        assert np.array_equal(_bits(got[pick]), _bits(ref))
+        assert np.array_equal(got[:, :3], vox[:, :3]) and not got[mask == 0, 3:].any()
+        assert (got[mask == 1, 3] > 0).all()
+
+
 @pytest.mark.parametrize("method", METHODS, ids=["fast", "plain"])
 def test_compete_parity(engine, method):
     s = scenes.make_scene(seed=43, ngrains=3, spread_mm=0.03)
