@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 #include "../../include/grscore.h"
@@ -104,6 +105,7 @@ struct grs_ctx {
   DevBuf f_in, f_cnt; /* fit_batch: packed per-step inputs and counts */
   void *h_pin = nullptr; /* pinned staging of fit_batch (hipHostMalloc) */
   size_t h_pin_cap = 0;
+  unsigned char *h_stage = nullptr; /* pinned staging of large transfers (staged_copy) */
   /* device address of this GPU's allocation-free scratch (nullptr if the
    * lookup failed; noalloc_err then holds the reason) */
   unsigned char *noalloc = nullptr;
@@ -201,6 +203,96 @@ static void free_buf(DevBuf &b) {
   if (b.p) hipFree(b.p);
   b.p = nullptr;
   b.cap = 0;
+}
+
+/* Large transfers between the caller's (pageable) memory and the device.  The
+ * runtime copies through its own staging with one thread (30 GB/s up, 18 GB/s
+ * down); here kStageThreads threads each move every kStageThreads-th chunk
+ * through two pinned buffers of their own, so that the DMA of one chunk runs
+ * beside the host copies of the others and first touches of fresh pages are
+ * shared.  A copy on the stream costs about 18 us beside its bytes, hence the
+ * large chunks: 759 MB move at 31, 40, 46 and 50 GB/s in chunks of 1, 2, 4
+ * and 8 MB (57 for one copy from pinned memory), the same with 4 threads as
+ * with 16.  The call of the single-precision operator that brings them:
+ * 26.4 -> 15.8 ms; a growth call of 3.2M voxels (154 MB up, 180 MB down into
+ * fresh pages): 61 -> 48 ms.  Below kStageMin there are too few chunks to
+ * overlap.  The copies go to the context's stream in any order among
+ * themselves before the function returns; an upload returns with its buffers
+ * free again, a download with the data in place. */
+static const int kStageThreads = 4;
+static const size_t kStageChunk = (size_t)8 << 20;
+static const size_t kStageMin = (size_t)48 << 20;
+
+static hipError_t stage_worker(grs_ctx *c, bool up, char *dev, char *host, size_t bytes, int w, int T) {
+  hipError_t e = hipSetDevice(c->device);
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  for (int j = 0; j < 2 && e == hipSuccess; j++) e = hipEventCreateWithFlags(&ev[j], hipEventDisableTiming);
+  unsigned char *buf[2] = {c->h_stage + (size_t)(2 * w) * kStageChunk, c->h_stage + (size_t)(2 * w + 1) * kStageChunk};
+  const size_t n = (bytes + kStageChunk - 1) / kStageChunk;
+  auto len = [&](size_t k) { return k + 1 < n ? kStageChunk : bytes - k * kStageChunk; };
+  size_t held[2] = {n, n}; /* the chunk in each buffer, n: none */
+  int j = 0;
+  for (size_t k = (size_t)w; e == hipSuccess && k < n; k += (size_t)T, j ^= 1) {
+    if (held[j] < n) {
+      e = hipEventSynchronize(ev[j]);
+      if (e == hipSuccess && !up) std::memcpy(host + held[j] * kStageChunk, buf[j], len(held[j]));
+      if (e != hipSuccess) break;
+    }
+    if (up) std::memcpy(buf[j], host + k * kStageChunk, len(k));
+    e = up ? hipMemcpyAsync(dev + k * kStageChunk, buf[j], len(k), hipMemcpyHostToDevice, c->st)
+           : hipMemcpyAsync(buf[j], dev + k * kStageChunk, len(k), hipMemcpyDeviceToHost, c->st);
+    if (e == hipSuccess) e = hipEventRecord(ev[j], c->st);
+    held[j] = k;
+  }
+  for (int i = 0; i < 2; i++, j ^= 1)
+    if (held[j] < n && ev[j]) {
+      const hipError_t s = hipEventSynchronize(ev[j]);
+      if (s == hipSuccess && e == hipSuccess && !up) std::memcpy(host + held[j] * kStageChunk, buf[j], len(held[j]));
+      if (e == hipSuccess) e = s;
+    }
+  for (int i = 0; i < 2; i++)
+    if (ev[i]) (void)hipEventDestroy(ev[i]);
+  return e;
+}
+
+static hipError_t staged_copy(grs_ctx *c, bool up, void *dev, void *host, size_t bytes) {
+  const hipMemcpyKind kind = up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
+  if (bytes >= kStageMin && !c->h_stage) {
+    void *p = nullptr;
+    if (hipHostMalloc(&p, 2 * kStageThreads * kStageChunk, hipHostMallocDefault) == hipSuccess)
+      c->h_stage = static_cast<unsigned char *>(p);
+    else
+      (void)hipGetLastError();
+  }
+  if (bytes < kStageMin || !c->h_stage)
+    return hipMemcpyAsync(up ? dev : host, up ? host : dev, bytes, kind, c->st);
+  char *d = static_cast<char *>(dev), *h = static_cast<char *>(host);
+  hipError_t err[kStageThreads];
+  std::thread th[kStageThreads];
+  for (int w = 1; w < kStageThreads; w++) {
+    err[w] = hipSuccess;
+    try {
+      th[w] = std::thread([=, &err]() { err[w] = stage_worker(c, up, d, h, bytes, w, kStageThreads); });
+    } catch (...) {
+      /* no thread: its chunks are moved below */
+    }
+  }
+  err[0] = stage_worker(c, up, d, h, bytes, 0, kStageThreads);
+  for (int w = 1; w < kStageThreads; w++) {
+    if (th[w].joinable()) th[w].join();
+    else err[w] = stage_worker(c, up, d, h, bytes, w, kStageThreads);
+  }
+  for (int w = 0; w < kStageThreads; w++)
+    if (err[w] != hipSuccess) return err[w];
+  return hipSuccess;
+}
+
+static hipError_t copy_up(grs_ctx *c, void *dev, const void *host, size_t bytes) {
+  return staged_copy(c, true, dev, const_cast<void *>(host), bytes);
+}
+
+static hipError_t copy_down(grs_ctx *c, void *host, const void *dev, size_t bytes) {
+  return staged_copy(c, false, const_cast<void *>(dev), host, bytes);
 }
 
 /* largest non-negative float key k with (double)as_float(k) <= thr */
@@ -323,6 +415,7 @@ void grs_destroy(grs_ctx *c) {
   for (hipEvent_t e : c->tev) hipEventDestroy(e);
   for (DevBuf *b : bufs) free_buf(*b);
   if (c->h_pin) hipHostFree(c->h_pin);
+  if (c->h_stage) hipHostFree(c->h_stage);
   for (hipEvent_t e : c->tpairs) hipEventDestroy(e);
   if (c->st) hipStreamDestroy(c->st);
   delete c;
@@ -438,8 +531,10 @@ grs_status grs_set_distance_stack(grs_ctx *c, const float *proj, int64_t nz, int
   HIPCHK(c, hipSetDevice(c->device));
   int64_t n = nz * ny * nrot;
   ENSURE(c, c->d_keys, sizeof(uint32_t) * n);
-  HIPCHK(c, hipMemcpyAsync(c->d_keys.p, proj, sizeof(float) * n,
-                           on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, c->st));
+  if (on_device)
+    HIPCHK(c, hipMemcpyAsync(c->d_keys.p, proj, sizeof(float) * n, hipMemcpyDeviceToDevice, c->st));
+  else
+    HIPCHK(c, copy_up(c, c->d_keys.p, proj, sizeof(float) * n));
   ENSURE(c, c->d_bad, sizeof(uint32_t));
   HIPCHK(c, hipMemsetAsync(c->d_bad.p, 0, sizeof(uint32_t), c->st));
   HIPCHK(c, grs_launch_check_keys(P<uint32_t>(c->d_keys), n, P<uint32_t>(c->d_bad), c->st));
@@ -833,7 +928,7 @@ grs_status grs_grow_indexed_region(grs_ctx *c, const double *vox, int64_t M, con
     ENSURE(c, c->d_evox, sizeof(int32_t) * m); /* a row's place among the scored ones */
     ENSURE(c, c->d_rowstart, sizeof(int64_t) + sizeof(int32_t) * nb);
     ENSURE(c, c->d_eu, sizeof(double) * 7 * m); /* output rows */
-    HIPCHK(c, hipMemcpyAsync(c->d_rows.p, vox + 6 * b, sizeof(double) * 6 * m, hipMemcpyHostToDevice, c->st));
+    HIPCHK(c, copy_up(c, c->d_rows.p, vox + 6 * b, sizeof(double) * 6 * m));
     int64_t *d_total = P<int64_t>(c->d_rowstart);
     int32_t *d_count = E == m ? nullptr : reinterpret_cast<int32_t *>(d_total + 1);
     HIPCHK(c, grs_launch_grow_list(P<double>(c->d_rows), m, P<double>(c->d_p1), d_count, P<double>(c->d_pos),
@@ -852,7 +947,7 @@ grs_status grs_grow_indexed_region(grs_ctx *c, const double *vox, int64_t M, con
     HIPCHK(c, grs_launch_grow_out(P<double>(c->d_rows), m, P<double>(c->d_p1), P<int32_t>(c->d_evox),
                                   P<int32_t>(c->d_ns), P<int32_t>(c->d_ni), P<double>(c->d_C), P<float>(c->d_med),
                                   P<double>(c->d_eu), c->st));
-    HIPCHK(c, hipMemcpyAsync(out + 7 * b, c->d_eu.p, sizeof(double) * 7 * m, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(c, copy_down(c, out + 7 * b, c->d_eu.p, sizeof(double) * 7 * m));
     HIPCHK(c, hipStreamSynchronize(c->st));
   }
   return GRS_OK;
@@ -2101,7 +2196,7 @@ grs_status grs_set_volume(grs_ctx *c, int32_t which, const double *v, int64_t nx
   }
   const size_t n = (size_t)(nx * ny * nz);
   ENSURE(c, c->v_vol[which], sizeof(double) * n);
-  HIPCHK(c, hipMemcpyAsync(c->v_vol[which].p, v, sizeof(double) * n, hipMemcpyHostToDevice, c->st));
+  HIPCHK(c, copy_up(c, c->v_vol[which].p, v, sizeof(double) * n));
   HIPCHK(c, hipStreamSynchronize(c->st));
   c->v_set[which] = true;
   return GRS_OK;
@@ -2113,7 +2208,7 @@ grs_status grs_get_volume(grs_ctx *c, int32_t which, double *v, int64_t n) {
   if (!c->v_set[which]) return fail(c, GRS_ERR_STATE, "volume %d not set", which);
   if (n != c->v_dim[0] * c->v_dim[1] * c->v_dim[2]) return fail(c, GRS_ERR_ARG, "size mismatch");
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, hipMemcpyAsync(v, c->v_vol[which].p, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, c->st));
+  HIPCHK(c, copy_down(c, v, c->v_vol[which].p, sizeof(double) * (size_t)n));
   HIPCHK(c, hipStreamSynchronize(c->st));
   return GRS_OK;
 }
@@ -2718,8 +2813,10 @@ grs_status grs_set_binary_stack(grs_ctx *c, const uint8_t *mask, int64_t nz, int
   HIPCHK(c, hipSetDevice(c->device));
   const int64_t n = nz * ny * nrot;
   ENSURE(c, c->d_mask, (size_t)n);
-  HIPCHK(c, hipMemcpyAsync(c->d_mask.p, mask, (size_t)n, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
-                           c->st));
+  if (on_device)
+    HIPCHK(c, hipMemcpyAsync(c->d_mask.p, mask, (size_t)n, hipMemcpyDeviceToDevice, c->st));
+  else
+    HIPCHK(c, copy_up(c, c->d_mask.p, mask, (size_t)n));
   HIPCHK(c, hipStreamSynchronize(c->st));
   c->mnz = nz;
   c->mny = ny;
@@ -2765,7 +2862,7 @@ grs_status grs_get_mask(grs_ctx *c, uint8_t *out, int64_t n) {
   if (!c) return GRS_ERR_ARG;
   if (!out || n != c->mnz * c->mny * c->mnrot) return fail(c, GRS_ERR_ARG, "output size does not match the mask");
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, hipMemcpyAsync(out, c->d_mask.p, (size_t)n, hipMemcpyDeviceToHost, c->st));
+  HIPCHK(c, copy_down(c, out, c->d_mask.p, (size_t)n));
   HIPCHK(c, hipStreamSynchronize(c->st));
   return GRS_OK;
 }
@@ -2775,7 +2872,7 @@ grs_status grs_get_distance_stack(grs_ctx *c, float *out, int64_t n) {
   if (!c->stack_set) return fail(c, GRS_ERR_STATE, "distance stack not set");
   if (!out || n != c->snz * c->sny * c->snrot) return fail(c, GRS_ERR_ARG, "output size does not match the stack");
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, hipMemcpyAsync(out, c->d_keys.p, sizeof(float) * (size_t)n, hipMemcpyDeviceToHost, c->st));
+  HIPCHK(c, copy_down(c, out, c->d_keys.p, sizeof(float) * (size_t)n));
   HIPCHK(c, hipStreamSynchronize(c->st));
   return GRS_OK;
 }

@@ -60,6 +60,23 @@ def test_edt_at_tile_edges(engine, nz, ny):
         assert np.array_equal(d[:, :, i].view(np.uint32), ref.view(np.uint32)), i
 
 
+@pytest.mark.parametrize("extra", [0, 1, 5])
+def test_large_transfers_keep_every_byte(engine, extra):
+    """Stacks and volumes above the size that goes through the staging
+    threads, with a last chunk that is whole, nearly whole or short."""
+    rng = np.random.default_rng(extra)
+    nz, ny, nrot = 1024, 1024, 14 + extra
+    d = rng.random((nrot, ny, nz + extra), dtype=np.float32).transpose(2, 1, 0)
+    engine.set_distance_stack(d)
+    assert np.array_equal(engine.get_distance_stack(d.shape), d)
+    v = rng.random((256 + extra, 256, 160 + extra))
+    engine.set_volume("Mask", v)
+    assert np.array_equal(engine.get_volume("Mask"), v)
+    m = rng.random((48 + extra, ny, nz)) < 0.5
+    engine.set_binary_stack(m.transpose(2, 1, 0))
+    assert np.array_equal(engine.get_mask((nz, ny, 48 + extra)), m.transpose(2, 1, 0))
+
+
 def test_rendered_scene_scores_one_at_truth(engine):
     s = scenes.make_scene(seed=73, ngrains=3, dilate=1)
     engine.set_geometry(s.geo, s.hkl, s.rot)
