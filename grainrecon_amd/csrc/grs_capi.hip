@@ -630,8 +630,9 @@ static grs_status launch_tuned(grs_ctx *c, grs_eval_args a, int kind, int64_t wa
     tune_cfg k = t.done ? t.cfg : tune_cfg{8, GRS_MASK_BITS, 0};
     if (k.mask == GRS_MASK_TILED && !c->tbits_ok) k.mask = GRS_MASK_BITS;
     apply_cfg(&a, k);
-    /* fewer waves than CUs (the steps of the orientation fits): one wave
-     * per block, so that every evaluation has a CU to itself */
+    /* fewer waves than CUs: one wave per block, so that every evaluation has
+     * a CU to itself (the kernel with the median shares each evaluation among
+     * a block's waves there, grs_launch_fast) */
     const int32_t wpb = waves < grs_fast_wave_slots(c->device) / 64 ? 1 : k.wpb;
     HIPCHK(c, launch(a, wpb));
     return GRS_OK;
@@ -1590,139 +1591,82 @@ grs_status grs_cuda_forward_comp_compete(const float *vox, int64_t n_vox, const 
 
 /* ---- orientation fit --------------------------------------------------------- */
 
+/* c->h_pin holds at least bytes (its contents are lost when it grows) */
+static grs_status ensure_pin(grs_ctx *c, size_t bytes) {
+  if (c->h_pin_cap >= bytes) return GRS_OK;
+  if (c->h_pin) HIPCHK(c, hipHostFree(c->h_pin));
+  c->h_pin = nullptr;
+  c->h_pin_cap = 0;
+  const hipError_t e = hipHostMalloc(&c->h_pin, 2 * bytes, hipHostMallocDefault);
+  if (e != hipSuccess) {
+    c->h_pin = nullptr;
+    (void)hipGetLastError();
+    return fail(c, GRS_ERR_NOMEM, "hipHostMalloc(%zu bytes) failed: %s", 2 * bytes, hipGetErrorString(e));
+  }
+  c->h_pin_cap = 2 * bytes;
+  return GRS_OK;
+}
+
 /* M fits, fit m at pos[3m..] from x0[3m..] (the body of grs_fit_or_local) */
 static grs_status fit_batch(grs_ctx *c, const double *pos, const double *x0, int64_t M, double half_width,
                             int32_t max_fun_evals, int32_t max_iter, double tol_fun, double tol_x, double *x_out,
                             double *fval, int32_t *n_fun_evals, int32_t *n_iter) {
-  grs_status s = GRS_OK;
   if (M > INT32_MAX / 4) return fail(c, GRS_ERR_ARG, "too many fits");
-  std::vector<grs_nm> nm((size_t)M);
-  for (int64_t m = 0; m < M; m++) {
-    double lo[3], hi[3];
-    for (int k = 0; k < 3; k++) {
-      /* fit_OR_constrain_with_local_comp_cuda.m:124-125 */
-      const double a = x0[3 * m + k] - half_width, b = x0[3 * m + k] + half_width;
-      lo[k] = grs_nm_max(a, -1.0);
-      hi[k] = (b != b) ? 1.0 : (b < 1.0 ? b : 1.0);
+  if (c->H > 240) return fail(c, GRS_ERR_ARG, "the fast method supports at most 240 reflections (got %d)", c->H);
+  const int64_t most = 65536; /* fits per launch (a block each) */
+  if (M > most) {
+    for (int64_t b = 0; b < M; b += most) {
+      const grs_status s = fit_batch(c, pos + 3 * b, x0 + 3 * b, M - b < most ? M - b : most, half_width, max_fun_evals,
+                                     max_iter, tol_fun, tol_x, x_out + 3 * b, fval + b, n_fun_evals + b, n_iter + b);
+      if (s != GRS_OK) return s;
     }
-    nm[m].max_fe = max_fun_evals;
-    nm[m].max_it = max_iter;
-    nm[m].tol_f = tol_fun;
-    nm[m].tol_x = tol_x;
-    nm[m].start(3, x0 + 3 * m, lo, hi);
+    return GRS_OK;
   }
-  ENSURE(c, c->d_pos, sizeof(double) * 3 * M);
-  HIPCHK(c, hipMemcpyAsync(c->d_pos.p, pos, sizeof(double) * 3 * M, hipMemcpyHostToDevice, c->st));
-  /* the positions stay fixed during the fits: their omega-solve bounds once */
+  /* positions, starts and the count of unfinished fits up in one copy from
+   * pinned memory; results and that count back in one */
+  const size_t in_bytes = sizeof(double) * 6 * (size_t)M, out_bytes = sizeof(double) * (6 * (size_t)M + 1);
+  grs_status s = ensure_pin(c, in_bytes + out_bytes);
+  if (s != GRS_OK) return s;
+  double *h_in = static_cast<double *>(c->h_pin), *h_out = h_in + 6 * M;
+  std::memcpy(h_in, pos, sizeof(double) * 3 * (size_t)M);
+  std::memcpy(h_in + 3 * M, x0, sizeof(double) * 3 * (size_t)M);
+  ENSURE(c, c->f_in, in_bytes);
+  ENSURE(c, c->f_cnt, out_bytes);
+  ENSURE(c, c->m_nm, grs_fit_nm_bytes() * (size_t)M);
   ENSURE(c, c->d_vb, sizeof(double) * GRS_VB * (size_t)M);
-  HIPCHK(c, grs_launch_voxel_bounds(P<grs_dgeo>(c->d_geo), P<double>(c->d_pos), M, P<double>(c->d_cs), c->nrot,
-                                    P<double>(c->d_vb), c->st));
-  /* each step: [q (4E doubles) | eval voxel (E) | eval orientation (E)]
-   * uploaded in one copy from pinned memory, [ns (E) | ni (E)] back in one.
-   * A launch of E evaluations takes about the time of one while every
-   * evaluation has a SIMD to itself; within that many, a fit's requested
-   * reflection goes out with the three points its value can lead to
-   * (grs_nm::follow_ups), and the one the method then requests is fed from
-   * that launch's value instead of a launch of its own.  The method's
-   * sequence of points, values and counts is unchanged. */
-  const int64_t spec_max = grs_fast_wave_slots(c->device) / 16;
-  std::vector<int64_t> first;
-  std::vector<int32_t> npv, nspec;
-  std::vector<double> fvals;
-  std::vector<double> su((size_t)M * 3 * GRS_NM_NMAX);
-  for (;;) {
-    first.assign((size_t)M + 1, 0);
-    npv.assign((size_t)M, 0);
-    nspec.assign((size_t)M, 0);
-    int64_t E = 0, nrefl = 0;
-    for (int64_t m = 0; m < M; m++) {
-      if (nm[m].done()) continue;
-      E += nm[m].npend;
-      nrefl += nm[m].st == grs_nm::REFLECT ? 1 : 0;
-    }
-    if (E == 0) break;
-    const bool spec = E + 3 * nrefl <= spec_max;
-    E = 0;
-    for (int64_t m = 0; m < M; m++) {
-      first[m] = E;
-      if (nm[m].done()) continue;
-      npv[m] = nm[m].npend;
-      if (spec) nspec[m] = nm[m].follow_ups(reinterpret_cast<double (*)[GRS_NM_NMAX]>(&su[(size_t)m * 3 * GRS_NM_NMAX]));
-      E += npv[m] + nspec[m];
-    }
-    first[M] = E;
-    const size_t in_bytes = (sizeof(double) * 4 + sizeof(int32_t) * 2) * (size_t)E;
-    const size_t cnt_bytes = sizeof(int32_t) * 2 * (size_t)E;
-    if (c->h_pin_cap < in_bytes + cnt_bytes) {
-      if (c->h_pin) HIPCHK(c, hipHostFree(c->h_pin));
-      c->h_pin = nullptr;
-      c->h_pin_cap = 0;
-      const size_t want = 2 * (in_bytes + cnt_bytes);
-      const hipError_t e = hipHostMalloc(&c->h_pin, want, hipHostMallocDefault);
-      if (e != hipSuccess) {
-        c->h_pin = nullptr;
-        (void)hipGetLastError();
-        return fail(c, GRS_ERR_NOMEM, "hipHostMalloc(%zu bytes) failed: %s", want, hipGetErrorString(e));
-      }
-      c->h_pin_cap = want;
-    }
-    double *hq = static_cast<double *>(c->h_pin);
-    int32_t *hvox = reinterpret_cast<int32_t *>(hq + 4 * E), *heu = hvox + E;
-    int32_t *hcnt = reinterpret_cast<int32_t *>(static_cast<char *>(c->h_pin) + in_bytes);
-    for (int64_t m = 0; m < M; m++) {
-      if (nm[m].done()) continue;
-      for (int p = 0; p < npv[m] + nspec[m]; p++) {
-        const int64_t e = first[m] + p;
-        double x[3];
-        nm[m].xform(p < npv[m] ? nm[m].pend[p] : &su[((size_t)m * 3 + (size_t)(p - npv[m])) * GRS_NM_NMAX], x);
-        hq[4 * e] = 0.0; /* q0 is recomputed from the vector part (fit_OR_fun_local.m:9) */
-        hq[4 * e + 1] = x[0];
-        hq[4 * e + 2] = x[1];
-        hq[4 * e + 3] = x[2];
-        hvox[e] = (int32_t)m;
-        heu[e] = (int32_t)e;
-      }
-    }
-    ENSURE(c, c->f_in, in_bytes);
-    ENSURE(c, c->f_cnt, cnt_bytes);
-    ENSURE(c, c->d_sub, sizeof(double) * 9 * E);
-    ENSURE(c, c->d_valid, sizeof(int32_t) * E);
-    ENSURE(c, c->d_C, sizeof(double) * E);
-    ENSURE(c, c->d_med, sizeof(float) * E);
-    HIPCHK(c, hipMemcpyAsync(c->f_in.p, hq, in_bytes, hipMemcpyHostToDevice, c->st));
-    double *dq = P<double>(c->f_in);
-    int32_t *dvox = reinterpret_cast<int32_t *>(dq + 4 * E), *deu = dvox + E;
-    int32_t *dns = P<int32_t>(c->f_cnt), *dni = dns + E;
-    HIPCHK(c, grs_launch_sub_from_q(P<grs_dgeo>(c->d_geo), dq, E, P<double>(c->d_sub), P<int32_t>(c->d_valid),
+  double *d_pos = P<double>(c->f_in), *d_x0 = d_pos + 3 * M, *d_res = P<double>(c->f_cnt) + 1;
+  HIPCHK(c, hipMemcpyAsync(d_pos, h_in, in_bytes, hipMemcpyHostToDevice, c->st));
+  HIPCHK(c, grs_launch_voxel_bounds(P<grs_dgeo>(c->d_geo), d_pos, M, P<double>(c->d_cs), c->nrot, P<double>(c->d_vb),
                                     c->st));
-    s = run_eval(c, GRS_MAP_PAIRS, E, M, dvox, deu, GRS_METHOD_FAST, dns, dni, P<double>(c->d_C),
-                 P<float>(c->d_med), true);
-    if (s != GRS_OK) return s;
-    HIPCHK(c, hipMemcpyAsync(hcnt, dns, cnt_bytes, hipMemcpyDeviceToHost, c->st));
+  grs_eval_args a;
+  std::memset(&a, 0, sizeof(a));
+  a.g = P<grs_dgeo>(c->d_geo);
+  a.hkl = P<double>(c->d_hkl);
+  a.cs = P<double>(c->d_cs);
+  a.vb = P<double>(c->d_vb);
+  a.pos = d_pos;
+  a.keys = P<uint32_t>(c->d_keys);
+  a.nrot = c->nrot;
+  /* hits on the bit mask where a counts-only launch has built it */
+  a.count_keys = c->bits_valid ? 0 : 1;
+  a.hit_bits = P<uint32_t>(c->d_bits);
+  int64_t left = 0;
+  for (int32_t first = 1; first || left > 0; first = 0) {
+    HIPCHK(c, grs_launch_fill_u64(P<unsigned long long>(c->f_cnt), 1, 0, c->st));
+    if (c->timing) HIPCHK(c, timing_begin(c));
+    HIPCHK(c, grs_launch_fit_nm(&a, c->H, M, d_x0, half_width, max_fun_evals, max_iter, tol_fun, tol_x, first,
+                                c->m_nm.p, d_res, P<int32_t>(c->f_cnt), c->st));
+    if (c->timing) HIPCHK(c, timing_end(c));
+    HIPCHK(c, hipMemcpyAsync(h_out, c->f_cnt.p, out_bytes, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
-    fvals.resize((size_t)E);
-    for (int64_t e = 0; e < E; e++) /* fit_OR_fun_local.m:98; 0/0 (no event, or a skipped row) is NaN */
-      fvals[e] = 1.0 - (double)hcnt[E + e] / (double)hcnt[e];
-    for (int64_t m = 0; m < M; m++) {
-      if (first[m + 1] == first[m]) continue;
-      nm[m].feed(&fvals[first[m]]);
-      /* an expansion or contraction found among the follow-ups (bit for bit) */
-      while (nspec[m] > 0 && !nm[m].done() && nm[m].npend == 1 &&
-             (nm[m].st == grs_nm::EXPAND || nm[m].st == grs_nm::CONTRACT_OUT || nm[m].st == grs_nm::CONTRACT_IN)) {
-        int hit = -1;
-        for (int s2 = 0; s2 < nspec[m] && hit < 0; s2++)
-          if (std::memcmp(nm[m].pend[0], &su[((size_t)m * 3 + (size_t)s2) * GRS_NM_NMAX],
-                          sizeof(double) * (size_t)nm[m].n) == 0)
-            hit = s2;
-        if (hit < 0) break;
-        nm[m].feed(&fvals[first[m] + npv[m] + hit]);
-      }
-    }
+    std::memcpy(&left, h_out, sizeof(left));
   }
   for (int64_t m = 0; m < M; m++) {
-    nm[m].result(x_out + 3 * m, fval + m);
-    n_fun_evals[m] = nm[m].nf;
-    n_iter[m] = nm[m].it;
+    const double *r = h_out + 1 + 6 * m;
+    for (int k = 0; k < 3; k++) x_out[3 * m + k] = r[k];
+    fval[m] = r[3];
+    n_fun_evals[m] = (int32_t)r[4];
+    n_iter[m] = (int32_t)r[5];
   }
   return GRS_OK;
 }

@@ -318,7 +318,7 @@ __global__ __launch_bounds__(256, 4) void k_gt_score(const grs_dgeo *g, const do
   if (threadIdx.x == 0) b1_thresholds(g, thr);
   __syncthreads();
   const int32_t H = g->H, nrot = g->nrot;
-  const int lane = threadIdx.x & 63, wib = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   /* per wave: G and 1/|G| of each reflection (4 doubles), the ring, the families */
   const int32_t Ht = TAB ? H : 0;
   double *tab = gts + (int64_t)wib * (4 * Ht + GT_RING / 2 + (Ht + 1) / 2);

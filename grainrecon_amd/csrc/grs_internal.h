@@ -114,6 +114,15 @@ hipError_t grs_launch_omega_cs(const double *d_rot, int32_t nrot, double *d_cs, 
 /* wpb: waves per block, 1, 2 or 4; n_waves: a multiple of 4 (wave slots of the scratch) */
 hipError_t grs_launch_fast(const grs_eval_args *a, int32_t H, int64_t n_waves, int32_t wpb, hipStream_t st);
 hipError_t grs_launch_fast_counts(const grs_eval_args *a, int32_t H, int64_t n_waves, int32_t wpb, hipStream_t st);
+/* M orientation fits, a block each (k_fit_nm): a describes the voxels (pos,
+ * vb of fit m's voxel at m) and the hit test (count_keys or hit_bits); d_nm
+ * holds M * grs_fit_nm_bytes() of state between launches (first != 0 starts
+ * the fits), d_res 6 doubles per fit (x, f, evaluations, iterations), d_left
+ * the number of unfinished fits is added to */
+size_t grs_fit_nm_bytes(void);
+hipError_t grs_launch_fit_nm(const grs_eval_args *a, int32_t H, int64_t M, const double *d_x0, double half_width,
+                             int32_t max_fe, int32_t max_it, double tol_f, double tol_x, int32_t first, void *d_nm,
+                             double *d_res, int32_t *d_left, hipStream_t st);
 hipError_t grs_launch_fast_audit(const grs_eval_args *a, int32_t H, int64_t n_waves, hipStream_t st);
 hipError_t grs_launch_fill_u64(unsigned long long *d_p, int64_t n, unsigned long long v, hipStream_t st);
 hipError_t grs_launch_winner_list(const unsigned long long *d_row_best, const int64_t *d_row_eoff, int64_t m,

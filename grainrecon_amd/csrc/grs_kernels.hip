@@ -35,6 +35,7 @@
 #include <hip/hip_runtime.h>
 
 #include "grs_internal.h"
+#include "grs_nm_lanes.h"
 #include "grs_resolve.h"
 
 #define GRS_WPB 8      /* largest number of waves per block of k_fast (the launch chooses 1, 2, 4 or 8) */
@@ -863,27 +864,422 @@ __device__ __forceinline__ int om_ranges(const grs_dgeo *g, double g0, double g1
   return (int)mask;
 }
 
-template <bool MEDIAN, int MAP, bool AUDIT>
+/* LDS regions of one wave of k_fast / k_fit_nm */
+struct fast_lds_regions {
+  double *gwt;      /* per reflection: G, 1/|G|, |G|^2 (indexed by the reflection) */
+  uint32_t *ring1;  /* phase-A survivors (omega << 8 | hkl) */
+  uint32_t *ring2;  /* events for the exact pipeline */
+  uint32_t *ring3;  /* selected events: stack index */
+  uint32_t *rstart; /* omega-solve ranges: (i0 << 8 | hkl) */
+  uint32_t *rcum;   /* exclusive prefix of range lengths */
+  double *Pw;       /* S*pos of the voxel */
+  /* S*U*B of the evaluation: the omega solve reads it from LDS, which keeps
+   * its 18 registers free for the candidate loop */
+  double *sbuf;
+};
+
+/* the regions of wave wib when every wave holds reflections hlo .. hlo + Hn - 1 at most */
+__device__ __forceinline__ fast_lds_regions fast_regions(double *smem, int wib, int32_t hlo, int32_t Hn) {
+  fast_lds_regions L;
+  double *w = smem + wib * fast_wave_doubles(Hn);
+  L.gwt = w - (int64_t)hlo * GRS_GWT;
+  L.ring1 = (uint32_t *)(w + (int64_t)Hn * GRS_GWT);
+  L.ring2 = L.ring1 + GRS_QCAP;
+  L.ring3 = L.ring2 + GRS_QCAP;
+  L.rstart = L.ring3 + GRS_QCAP;
+  L.rcum = L.rstart + 4 * Hn;
+  L.Pw = w + (int64_t)Hn * GRS_GWT + GRS_RING_DOUBLES + GRS_RANGE_DOUBLES(Hn);
+  L.sbuf = L.Pw + 4;
+  return L;
+}
+
+/* One wave scores the events of reflections hlo .. hend - 1 of the evaluation
+ * (voxel vi, orientation sub): the counts and, with MEDIAN, the keys of the
+ * selected events in wlist.  TEAM: the waves of a block share the
+ * evaluation, each with its own reflections, and append their keys to one
+ * list through the block's counter tcount. */
+template <bool MEDIAN, bool AUDIT, bool TEAM>
+__device__ __forceinline__ void score_events(const grs_eval_args &a, const grs_dgeo *g, const double *b1thr,
+                                             const double *btab, const fast_lds_regions &L, const double *sub,
+                                             int64_t vi, int32_t hlo, int32_t hend, uint32_t *wlist, int32_t *tcount,
+                                             int32_t *ns_out, int32_t *ni_out) {
+  const int lane = threadIdx.x & 63;
+  double *gwt = L.gwt;
+  uint32_t *ring1 = L.ring1, *ring2 = L.ring2, *ring3 = L.ring3, *rstart = L.rstart, *rcum = L.rcum;
+  double *Pw = L.Pw, *sbuf = L.sbuf;
+  const int32_t nrot = g->nrot;
+  const int64_t nz = g->nz, nzny = g->nz * g->ny;
+  const uint32_t nz32 = (uint32_t)nz, nzny32 = (uint32_t)nzny; /* the stack holds fewer than 2^32 entries */
+  /* counts-only on the tiled mask: the selected events carry tiled bit numbers */
+  const bool tiled = !MEDIAN && a.bits_tiled && !a.count_keys;
+  const uint32_t ntz = (uint32_t)((nz + 31) >> 5), nty = (uint32_t)((g->ny + 31) >> 5);
+  const uint32_t *hbits = tiled ? a.hit_tbits : a.hit_bits;
+  const double m4pi = -4.0 * GRS_PI;
+  /* phase A margins: see the header comment */
+  const double dcb = 1e-12;
+  const double cbm = g->cos_beta_max - dcb;
+  const double lmin = g->lambda_min, lmax = g->lambda_max;
+  const double lrel = 1e-9 * lmax;
+  const double inv4pi = 1.0 / (4.0 * GRS_PI);
+  const double idom = g->om_solve ? 1.0 / g->dom : 0.0;
+  /* per-reflection terms; with the omega solve also the candidate ranges */
+  const bool solve = g->om_solve != 0;
+  if (lane == 0) {
+    voxel_P(g, a.pos + 3 * vi, Pw);
+#pragma unroll
+    for (int k = 0; k < 9; k++) sbuf[k] = sub[k];
+  }
+  wave_sync();
+  double vW = 0.0, vu2lo = 0.0, vu2hi = 0.0, sK = 1.0, val = 0.0, vbe = 0.0, vga = 0.0;
+  double vzt = 1e300, vzb = -1e300, vsn = 1.0, vcn = 0.0, vte = 0.0, vya = 1e300, vdl = 0.0;
+  if (solve) {
+    const double *b = a.vb + GRS_VB * vi;
+    vW = b[0];
+    vu2lo = b[1];
+    vu2hi = b[2];
+    sK = __builtin_sqrt(b[3]);
+    val = b[4];
+    vbe = b[5];
+    vga = b[6];
+    vzt = b[7];
+    vzb = b[8];
+    vsn = b[9];
+    vcn = b[10];
+    vte = b[11];
+    vya = b[12];
+    vdl = b[13];
+  }
+  uint32_t R = 0;
+  bool overflow = false;
+  for (int hb = hlo; hb < hend; hb += 64) {
+    const int h = hb + lane;
+    int nr_h = 0; /* bit mask of the valid slots of ri0/ri1, or -1 */
+    int32_t ri0[6], ri1[6];
+    if (h < hend) {
+      double gw[3];
+      grs_Gw(sbuf, a.hkl + 3 * h, gw);
+      double n2 = (gw[0] * gw[0] + gw[1] * gw[1]) + gw[2] * gw[2];
+      const double ign = fast_rsq(n2);
+      const double gn = n2 * ign;
+      double *t = gwt + h * GRS_GWT;
+      t[0] = gw[0];
+      t[1] = gw[1];
+      t[2] = gw[2];
+      t[3] = ign;
+      t[4] = n2;
+      double ml = lrel + (1e-12 * (4.0 * GRS_PI)) * ign; /* absolute lambda margin */
+      if (solve) {
+        /* cos(beta) window: beta and lambda bounds with the phase-A margins,
+         * the detector cone and the detector rows and columns.  cos(beta) = u . G/gn lies within rg W
+         * of r' cos(omega + phi') / gn + c0 + u2 g2 / gn, where
+         * (g0', g1') = (g0 + ga g1, g1 - ga g0) has modulus r' and angle
+         * phi' and u2 spans [vb[1], vb[2]] (the voxel bounds), so the
+         * window moves onto the first term. */
+        double lo_cb = cbm;
+        double lw = -(lmax + ml) * gn * inv4pi;
+        lo_cb = lw > lo_cb ? lw : lo_cb;
+        lo_cb = -sK > lo_cb ? -sK : lo_cb;
+        const double z = gw[2] * ign;
+        const double st = det_sin_theta(z, -lo_cb, vzt, vzb, vya, vdl, vsn, vcn, vte);
+        lo_cb = -st > lo_cb ? -st : lo_cb;
+        double hi_cb = dcb;
+        double hw = -(lmin - ml) * gn * inv4pi;
+        hi_cb = hw < hi_cb ? hw : hi_cb;
+        const double q2 = gw[0] * gw[0] + gw[1] * gw[1];
+        const double rg = q2 > 0.0 ? q2 * fast_rsq(q2) * ign : 0.0;
+        const double c0 = (val * gw[0] + vbe * gw[1]) * (0.5 * ign);
+        const double sa = z * vu2lo, sb = z * vu2hi;
+        const double slo = sa < sb ? sa : sb, shi = sa < sb ? sb : sa;
+        const double w = rg * vW;
+        nr_h = om_ranges(g, gw[0] + vga * gw[1], gw[1] - vga * gw[0], gn, ((lo_cb - c0) - shi) - w - 1e-12,
+                         ((hi_cb - c0) - slo) + w + 1e-12, nrot, idom, ri0, ri1);
+      }
+    }
+    if (solve) {
+      overflow = overflow || (__ballot(nr_h < 0) != 0);
+      const uint32_t msk = nr_h > 0 ? (uint32_t)nr_h : 0u;
+      const int cnt = __popc(msk);
+      int incl = cnt;
+      for (int off = 1; off < 64; off <<= 1) {
+        int v = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += v;
+      }
+      uint32_t pos = R + (uint32_t)(incl - cnt);
+#pragma unroll
+      for (int k = 0; k < 6; k++) {
+        if ((msk >> k) & 1u) {
+          rstart[pos] = ((uint32_t)ri0[k] << 8) | (uint32_t)h;
+          rcum[pos] = (uint32_t)(ri1[k] - ri0[k] + 1);
+          pos++;
+        }
+      }
+      R += (uint32_t)__shfl(incl, 63, 64);
+    }
+  }
+  wave_sync();
+  uint32_t total = 0;
+  if (solve && !overflow) {
+    /* lengths -> exclusive prefix sums */
+    for (uint32_t cb = 0; cb < R; cb += 64) {
+      const uint32_t r = cb + lane;
+      const uint32_t len = r < R ? rcum[r] : 0u;
+      uint32_t incl = len;
+      for (int off = 1; off < 64; off <<= 1) {
+        uint32_t v = (uint32_t)__shfl_up((int)incl, off, 64);
+        if (lane >= off) incl += v;
+      }
+      wave_sync();
+      if (r < R) rcum[r] = total + incl - len;
+      total += (uint32_t)__shfl((int)incl, 63, 64);
+      wave_sync();
+    }
+    if (lane == 0) rcum[R] = total;
+    wave_sync();
+  }
+
+  const double *vpos = a.pos + 3 * vi;
+  uint32_t head1 = 0, tail1 = 0, head2 = 0, tail2 = 0, head3 = 0, tail3 = 0;
+  int32_t ns = 0, ni = 0;
+  /* the gather of the previous batch is consumed one batch later */
+  bool p_sel = false, p_hit = false;
+  uint32_t p_key = 0;
+
+  auto consume = [&]() {
+    uint64_t ms = __ballot(p_sel);
+    if (MEDIAN) {
+      int32_t at = ns;
+      if (TEAM && ms) {
+        /* the team's waves append to one list */
+        if (lane == 0) at = atomicAdd(tcount, (int32_t)__popcll(ms));
+        at = __builtin_amdgcn_readfirstlane(at);
+      }
+      if (p_sel) wlist[at + (int32_t)lane_prefix(ms)] = p_key;
+    }
+    ns += (int32_t)__popcll(ms);
+    bool hit;
+    if (MEDIAN) hit = p_sel && g->has_hit && p_key <= g->hit_key;
+    else hit = p_hit;
+    ni += (int32_t)__popcll(__ballot(hit));
+    p_sel = false;
+    p_hit = false;
+  };
+
+  /* gather: distance key (or hit bit) of n selected events of ring3 */
+  auto gather = [&](uint32_t n) {
+    consume();
+    if ((uint32_t)lane < n) {
+      uint32_t idx = ring3[(head3 + lane) & (GRS_QCAP - 1)];
+      p_sel = true;
+      if (MEDIAN) p_key = a.keys[idx];
+      else if (a.count_keys) p_hit = g->has_hit && a.keys[idx] <= g->hit_key;
+      else p_hit = (hbits[idx >> 5] >> (idx & 31u)) & 1u;
+    }
+    head3 += n;
+  };
+
+  auto push3 = [&](bool sel, uint32_t idx) {
+    uint64_t m = __ballot(sel);
+    if (sel) ring3[(tail3 + lane_prefix(m)) & (GRS_QCAP - 1)] = idx;
+    tail3 += (uint32_t)__popcll(m);
+    if (tail3 - head3 >= 64) {
+      wave_sync();
+      gather(64);
+      wave_sync();
+    }
+  };
+
+  /* phase B2: exact pipeline on n events of ring2 */
+  auto b2 = [&](uint32_t n) {
+    bool sel = false;
+    uint32_t idx = 0;
+    if ((uint32_t)lane < n) {
+      double yz[2];
+      sel = exact_event(a.g, vpos, a.cs, gwt, ring2[(head2 + lane) & (GRS_QCAP - 1)], &idx, yz) != 0;
+      if (sel && tiled) {
+        const uint32_t omx = idx / nzny32, rem = idx - omx * nzny32, y0 = rem / nz32;
+        idx = grs_tiled_bit(omx, y0 + 1u, rem - y0 * nz32 + 1u, ntz, nty);
+      }
+    }
+    head2 += n;
+    push3(sel, idx);
+  };
+
+  /* phase B1: resolve n events of ring1 or queue them for the exact pipeline */
+  auto b1_core = [&](bool valid, uint32_t ev, uint32_t n) {
+    int st = 0;
+    uint32_t idx = 0;
+    bool bad = false, inwin = false;
+    double dev = 0.0;
+    if (valid) {
+      int32_t om = (int32_t)(ev >> 8), h = (int32_t)(ev & 255u);
+      const double *t = gwt + h * GRS_GWT;
+      b1_out o;
+      o.ry = o.rz = 0.0;
+      o.dy = o.dz = 0;
+      o.win = 0;
+      const double *brow = btab ? btab + GRS_BT * om : nullptr;
+      const double cc = brow ? brow[10] : a.cs[2 * om], ss = brow ? brow[11] : a.cs[2 * om + 1];
+      st = b1_classify(g, cc, ss, Pw, brow, t, b1thr, &o);
+      if (st == 1)
+        idx = tiled ? grs_tiled_bit((uint32_t)om, (uint32_t)o.dy, (uint32_t)o.dz, ntz, nty)
+                    : (uint32_t)(o.dz - 1) + (uint32_t)(o.dy - 1) * nz32 + (uint32_t)om * nzny32;
+      inwin = o.win != 0;
+      if (AUDIT) {
+        double yz[2] = {0.0, 0.0};
+        uint32_t eidx = 0;
+        const int es = exact_event(a.g, vpos, a.cs, gwt, ev, &eidx, yz);
+        bad = (st == 0 && es) || (st == 1 && (!es || eidx != idx));
+        if (st == 1 && es) dev = __builtin_fmax(__builtin_fabs(o.ry - yz[0]), __builtin_fabs(o.rz - yz[1]));
+      }
+    }
+    if (AUDIT) {
+      /* whole-wave reductions, outside the divergent block */
+      uint64_t mb = __ballot(bad), m1 = __ballot(st == 1), m0 = __ballot(valid && st == 0);
+      uint64_t m2 = __ballot(st == 2), mw = __ballot(inwin);
+      for (int off = 32; off >= 1; off >>= 1) dev = __builtin_fmax(dev, __shfl_xor(dev, off, 64));
+      if (lane == 0) {
+        atomicAdd(a.audit + 0, (unsigned long long)n);
+        atomicAdd(a.audit + 1, (unsigned long long)__popcll(m1));
+        atomicAdd(a.audit + 2, (unsigned long long)__popcll(m0));
+        atomicAdd(a.audit + 3, (unsigned long long)__popcll(m2));
+        atomicAdd(a.audit + 4, (unsigned long long)__popcll(mb));
+        atomicMax(a.audit + 5, (unsigned long long)__double_as_longlong(dev));
+        atomicAdd(a.audit + 6, (unsigned long long)__popcll(mw));
+      }
+    }
+    uint64_t m2 = __ballot(st == 2);
+    if (st == 2) ring2[(tail2 + lane_prefix(m2)) & (GRS_QCAP - 1)] = ev;
+    tail2 += (uint32_t)__popcll(m2);
+    push3(st == 1, idx);
+    if (tail2 - head2 >= 64) {
+      wave_sync();
+      b2(64);
+      wave_sync();
+    }
+  };
+
+  auto b1 = [&](uint32_t n) {
+    const bool valid = (uint32_t)lane < n;
+    const uint32_t ev = valid ? ring1[(head1 + lane) & (GRS_QCAP - 1)] : 0u;
+    head1 += n;
+    b1_core(valid, ev, n);
+  };
+
+  if (solve && !overflow) {
+    /* candidates of the omega solve, 64 per step, straight to phase B1.
+     * Ranges are non-empty and rcum is their exclusive prefix, so the range
+     * of candidate base + l is rb plus the number of later ranges that
+     * start at or before base + l, where rb is the last range starting
+     * before base (0 at base 0).  Those starts lie in the next 64 ranges;
+     * each marks its position in ring1 (unused on this path) and a ballot
+     * turns the marks into a bit mask. */
+    uint32_t rb = 0;
+    for (uint32_t base = 0; base < total; base += 64) {
+      const uint32_t idx = base + (uint32_t)lane;
+      const bool valid = idx < total;
+      ring1[lane] = 0u;
+      wave_sync();
+      const uint32_t rn = rb + 1u + (uint32_t)lane;
+      if (rn < R) {
+        const uint32_t p = rcum[rn] - base;
+        if (p < 64u) ring1[p] = 1u;
+      }
+      wave_sync();
+      const uint64_t starts = __ballot(ring1[lane] != 0u);
+      const uint64_t upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
+      const uint32_t r = rb + (uint32_t)__popcll(starts & upto);
+      rb += (uint32_t)__popcll(starts);
+      uint32_t ev = 0;
+      if (valid) {
+        const uint32_t st0 = rstart[r];
+        ev = (((st0 >> 8) + (idx - rcum[r])) << 8) | (st0 & 255u);
+      }
+      b1_core(valid, ev, total - base < 64u ? total - base : 64u);
+    }
+  }
+  /* phase A (no omega solve): wave-uniform steps of 64 consecutive events;
+   * lane l owns event l + 64*k, tracked as (omega, hkl) without divisions */
+  const int32_t Hn = hend - hlo;
+  int32_t om = 0, h = hlo;
+  int32_t nsteps = 0;
+  if (!(solve && !overflow) && Hn > 0) {
+    nsteps = (nrot * Hn + 63) / 64;
+    om = lane / Hn;
+    h = hlo + (lane - om * Hn);
+  }
+  for (int32_t k = 0; k < nsteps; ++k) {
+    bool pass = false;
+    if (om < nrot) {
+      const double c = a.cs[2 * om], s = a.cs[2 * om + 1];
+      double swv[3], uv[3];
+      beam_terms(g, Pw, c, s, swv, uv);
+      const double u0 = uv[0], u1 = uv[1], u2 = uv[2];
+      const double *t = gwt + h * GRS_GWT;
+      double Gt0 = c * t[0] - s * t[1];
+      double Gt1 = s * t[0] + c * t[1];
+      double dot = __builtin_fma(u2, t[2], __builtin_fma(u1, Gt1, u0 * Gt0));
+      double l4 = m4pi * dot;
+      /* the phase-A thresholds of the reflection (margins: see the header comment) */
+      const double gn = __builtin_sqrt(t[4]);
+      const double ml = lrel + (1e-12 * (4.0 * GRS_PI)) * t[3];
+      pass = (dot < dcb * gn) && (dot > cbm * gn) && (l4 > (lmin - ml) * t[4]) && (l4 < (lmax + ml) * t[4]);
+    }
+    uint64_t m = __ballot(pass);
+    if (pass) ring1[(tail1 + lane_prefix(m)) & (GRS_QCAP - 1)] = ((uint32_t)om << 8) | (uint32_t)h;
+    tail1 += (uint32_t)__popcll(m);
+    if (tail1 - head1 >= 64) {
+      wave_sync();
+      b1(64);
+      wave_sync();
+    }
+    h += 64;
+    while (h >= hend) {
+      h -= Hn;
+      om++;
+    }
+  }
+  while (tail1 != head1) {
+    uint32_t n = tail1 - head1;
+    if (n > 64) n = 64;
+    wave_sync();
+    b1(n);
+    wave_sync();
+  }
+  while (tail2 != head2) {
+    uint32_t n = tail2 - head2;
+    if (n > 64) n = 64;
+    wave_sync();
+    b2(n);
+    wave_sync();
+  }
+  while (tail3 != head3) {
+    uint32_t n = tail3 - head3;
+    if (n > 64) n = 64;
+    wave_sync();
+    gather(n);
+    wave_sync();
+  }
+  consume();
+  *ns_out = ns;
+  *ni_out = ni;
+}
+
+template <bool MEDIAN, int MAP, bool AUDIT, bool TEAM>
 __global__ __launch_bounds__(64 * GRS_WPB, GRS_FAST_MIN_WAVES) void k_fast(grs_eval_args a, int32_t H) {
   extern __shared__ double smem[];
   const int lane = threadIdx.x & 63;
-  const int wib = threadIdx.x >> 6;
-  const int64_t per_wave = fast_wave_doubles(H);
-  double *gwt = smem + wib * per_wave;
-  uint32_t *ring1 = (uint32_t *)(gwt + (int64_t)H * GRS_GWT); /* phase-A survivors (omega << 8 | hkl) */
-  uint32_t *ring2 = ring1 + GRS_QCAP;                          /* events for the exact pipeline */
-  uint32_t *ring3 = ring2 + GRS_QCAP;                          /* selected events: stack index */
-  uint32_t *rstart = ring3 + GRS_QCAP;                         /* omega-solve ranges: (i0 << 8 | hkl) */
-  uint32_t *rcum = rstart + 4 * H;                             /* exclusive prefix of range lengths */
-  double *Pw = gwt + (int64_t)H * GRS_GWT + GRS_RING_DOUBLES + GRS_RANGE_DOUBLES(H); /* S*pos of the voxel */
-  /* S*U*B of the evaluation: the omega solve reads it from LDS, which keeps
-   * its 18 registers free for the candidate loop */
-  double *sbuf = Pw + 4;
+  const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); /* uniform: a wave's addresses and bounds stay scalar */
+  /* a team's waves split the reflections evenly */
+  const int32_t Hn = TEAM ? (H + (int)(blockDim.x >> 6) - 1) / (int)(blockDim.x >> 6) : H;
+  const int32_t hlo = TEAM ? (wib * Hn < H ? wib * Hn : H) : 0, hend = hlo + Hn < H ? hlo + Hn : H;
+  const int64_t per_wave = fast_wave_doubles(Hn);
+  const fast_lds_regions L = fast_regions(smem, wib, hlo, Hn);
   /* the geometry constants live in LDS: the loop bodies read ~30 of them per
    * batch, and neither scalar registers (spilled) nor vector loads (the
    * compiler cannot prove them unchanged across the loop's stores) serve */
   __shared__ grs_dgeo sg;
   __shared__ double b1thr[12]; /* b1_thresholds */
+  __shared__ int32_t team[3];  /* TEAM: ns, ni and the keys listed so far */
   if (threadIdx.x == 0) {
     sg = *a.g;
     b1_thresholds(&sg, b1thr);
@@ -895,7 +1291,7 @@ __global__ __launch_bounds__(64 * GRS_WPB, GRS_FAST_MIN_WAVES) void k_fast(grs_e
    * once per block into LDS behind the per-wave regions (the launch sizes
    * the allocation with the same rule) */
   const double *btab = nullptr;
-  if (MAP == GRS_MAP_ONE_VOXEL && a.nrot == g->nrot && fast_tab_doubles(MAP, a.nrot, H, wpb) > 0 &&
+  if (!TEAM && MAP == GRS_MAP_ONE_VOXEL && a.nrot == g->nrot && fast_tab_doubles(MAP, a.nrot, H, wpb) > 0 &&
       a.e0 < a.n_eval) {
     double *bt = smem + (int64_t)wpb * per_wave;
     double P[3];
@@ -926,27 +1322,10 @@ __global__ __launch_bounds__(64 * GRS_WPB, GRS_FAST_MIN_WAVES) void k_fast(grs_e
    * evaluations (neighbouring samples of a CSR row share detector tiles) */
   int64_t vblock = blockIdx.x;
   if (a.xcd_map && (gridDim.x & 7u) == 0u) vblock = (int64_t)(blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  const int64_t gwave = vblock * wpb + wib;
-  const int64_t nwaves = (int64_t)gridDim.x * wpb;
+  /* an evaluation per wave, or per block of a team */
+  const int64_t gwave = TEAM ? vblock : vblock * wpb + wib;
+  const int64_t nwaves = TEAM ? gridDim.x : (int64_t)gridDim.x * wpb;
   uint32_t *wlist = MEDIAN ? a.scratch + gwave * a.scratch_stride : nullptr;
-  const int32_t nrot = g->nrot;
-  const int64_t nz = g->nz, nzny = g->nz * g->ny;
-  const uint32_t nz32 = (uint32_t)nz, nzny32 = (uint32_t)nzny; /* the stack holds fewer than 2^32 entries */
-  /* counts-only on the tiled mask: the selected events carry tiled bit numbers */
-  const bool tiled = !MEDIAN && a.bits_tiled && !a.count_keys;
-  const uint32_t ntz = (uint32_t)((nz + 31) >> 5), nty = (uint32_t)((g->ny + 31) >> 5);
-  const uint32_t *hbits = tiled ? a.hit_tbits : a.hit_bits;
-  const double m4pi = -4.0 * GRS_PI;
-  /* phase A margins: see the header comment */
-  const double dcb = 1e-12;
-  const double cbm = g->cos_beta_max - dcb;
-  const double lmin = g->lambda_min, lmax = g->lambda_max;
-  const double lrel = 1e-9 * lmax;
-  const double inv4pi = 1.0 / (4.0 * GRS_PI);
-  const double idom = g->om_solve ? 1.0 / g->dom : 0.0;
-  /* starting (omega, hkl) of each lane in the flattened event space */
-  const int32_t om0 = lane / H, h0 = lane - (lane / H) * H;
-
   int64_t row_hint = -1;
   for (int64_t e = a.e0 + gwave; e < a.n_eval; e += nwaves) {
     int64_t vi, row, jloc;
@@ -961,7 +1340,7 @@ __global__ __launch_bounds__(64 * GRS_WPB, GRS_FAST_MIN_WAVES) void k_fast(grs_e
         } else if (lane == 0 && ok == 0) {
           atomicMax(a.csr.row_best + row, (unsigned long long)(((1ull << GRS_KEY_JBITS) - 1) - (uint64_t)jloc));
         }
-      } else if (lane == 0) {
+      } else if (lane == 0 && (!TEAM || wib == 0)) {
         a.out_ns[e] = 0;
         a.out_ni[e] = 0;
         a.out_C[e] = 0.0;
@@ -969,330 +1348,25 @@ __global__ __launch_bounds__(64 * GRS_WPB, GRS_FAST_MIN_WAVES) void k_fast(grs_e
       }
       continue;
     }
-    /* per-reflection terms; with the omega solve also the candidate ranges */
-    const bool solve = g->om_solve != 0;
-    if (lane == 0) {
-      voxel_P(g, a.pos + 3 * vi, Pw);
-#pragma unroll
-      for (int k = 0; k < 9; k++) sbuf[k] = sub[k];
+    int32_t ns, ni;
+    if (TEAM) {
+      if (threadIdx.x == 0) team[0] = team[1] = team[2] = 0;
+      __syncthreads();
     }
-    wave_sync();
-    double vW = 0.0, vu2lo = 0.0, vu2hi = 0.0, sK = 1.0, val = 0.0, vbe = 0.0, vga = 0.0;
-    double vzt = 1e300, vzb = -1e300, vsn = 1.0, vcn = 0.0, vte = 0.0, vya = 1e300, vdl = 0.0;
-    if (solve) {
-      const double *b = a.vb + GRS_VB * vi;
-      vW = b[0];
-      vu2lo = b[1];
-      vu2hi = b[2];
-      sK = __builtin_sqrt(b[3]);
-      val = b[4];
-      vbe = b[5];
-      vga = b[6];
-      vzt = b[7];
-      vzb = b[8];
-      vsn = b[9];
-      vcn = b[10];
-      vte = b[11];
-      vya = b[12];
-      vdl = b[13];
+    score_events<MEDIAN, AUDIT, TEAM>(a, g, b1thr, btab, L, sub, vi, hlo, hend, wlist, &team[2], &ns, &ni);
+    if (TEAM) {
+      if (lane == 0) {
+        atomicAdd(&team[0], ns);
+        atomicAdd(&team[1], ni);
+      }
+      __threadfence_block();
+      __syncthreads();
+      /* the first wave closes the evaluation; the others wait for it where
+       * the counters are cleared */
+      if (wib != 0) continue;
+      ns = team[0];
+      ni = team[1];
     }
-    uint32_t R = 0;
-    bool overflow = false;
-    for (int hb = 0; hb < H; hb += 64) {
-      const int h = hb + lane;
-      int nr_h = 0; /* bit mask of the valid slots of ri0/ri1, or -1 */
-      int32_t ri0[6], ri1[6];
-      if (h < H) {
-        double gw[3];
-        grs_Gw(sbuf, a.hkl + 3 * h, gw);
-        double n2 = (gw[0] * gw[0] + gw[1] * gw[1]) + gw[2] * gw[2];
-        const double ign = fast_rsq(n2);
-        const double gn = n2 * ign;
-        double *t = gwt + h * GRS_GWT;
-        t[0] = gw[0];
-        t[1] = gw[1];
-        t[2] = gw[2];
-        t[3] = ign;
-        t[4] = n2;
-        double ml = lrel + (1e-12 * (4.0 * GRS_PI)) * ign; /* absolute lambda margin */
-        if (solve) {
-          /* cos(beta) window: beta and lambda bounds with the phase-A margins,
-           * the detector cone and the detector rows and columns.  cos(beta) = u . G/gn lies within rg W
-           * of r' cos(omega + phi') / gn + c0 + u2 g2 / gn, where
-           * (g0', g1') = (g0 + ga g1, g1 - ga g0) has modulus r' and angle
-           * phi' and u2 spans [vb[1], vb[2]] (the voxel bounds), so the
-           * window moves onto the first term. */
-          double lo_cb = cbm;
-          double lw = -(lmax + ml) * gn * inv4pi;
-          lo_cb = lw > lo_cb ? lw : lo_cb;
-          lo_cb = -sK > lo_cb ? -sK : lo_cb;
-          const double z = gw[2] * ign;
-          const double st = det_sin_theta(z, -lo_cb, vzt, vzb, vya, vdl, vsn, vcn, vte);
-          lo_cb = -st > lo_cb ? -st : lo_cb;
-          double hi_cb = dcb;
-          double hw = -(lmin - ml) * gn * inv4pi;
-          hi_cb = hw < hi_cb ? hw : hi_cb;
-          const double q2 = gw[0] * gw[0] + gw[1] * gw[1];
-          const double rg = q2 > 0.0 ? q2 * fast_rsq(q2) * ign : 0.0;
-          const double c0 = (val * gw[0] + vbe * gw[1]) * (0.5 * ign);
-          const double sa = z * vu2lo, sb = z * vu2hi;
-          const double slo = sa < sb ? sa : sb, shi = sa < sb ? sb : sa;
-          const double w = rg * vW;
-          nr_h = om_ranges(g, gw[0] + vga * gw[1], gw[1] - vga * gw[0], gn, ((lo_cb - c0) - shi) - w - 1e-12,
-                           ((hi_cb - c0) - slo) + w + 1e-12, nrot, idom, ri0, ri1);
-        }
-      }
-      if (solve) {
-        overflow = overflow || (__ballot(nr_h < 0) != 0);
-        const uint32_t msk = nr_h > 0 ? (uint32_t)nr_h : 0u;
-        const int cnt = __popc(msk);
-        int incl = cnt;
-        for (int off = 1; off < 64; off <<= 1) {
-          int v = __shfl_up(incl, off, 64);
-          if (lane >= off) incl += v;
-        }
-        uint32_t pos = R + (uint32_t)(incl - cnt);
-#pragma unroll
-        for (int k = 0; k < 6; k++) {
-          if ((msk >> k) & 1u) {
-            rstart[pos] = ((uint32_t)ri0[k] << 8) | (uint32_t)h;
-            rcum[pos] = (uint32_t)(ri1[k] - ri0[k] + 1);
-            pos++;
-          }
-        }
-        R += (uint32_t)__shfl(incl, 63, 64);
-      }
-    }
-    wave_sync();
-    uint32_t total = 0;
-    if (solve && !overflow) {
-      /* lengths -> exclusive prefix sums */
-      for (uint32_t cb = 0; cb < R; cb += 64) {
-        const uint32_t r = cb + lane;
-        const uint32_t len = r < R ? rcum[r] : 0u;
-        uint32_t incl = len;
-        for (int off = 1; off < 64; off <<= 1) {
-          uint32_t v = (uint32_t)__shfl_up((int)incl, off, 64);
-          if (lane >= off) incl += v;
-        }
-        wave_sync();
-        if (r < R) rcum[r] = total + incl - len;
-        total += (uint32_t)__shfl((int)incl, 63, 64);
-        wave_sync();
-      }
-      if (lane == 0) rcum[R] = total;
-      wave_sync();
-    }
-
-    const double *vpos = a.pos + 3 * vi;
-    uint32_t head1 = 0, tail1 = 0, head2 = 0, tail2 = 0, head3 = 0, tail3 = 0;
-    int32_t ns = 0, ni = 0;
-    /* the gather of the previous batch is consumed one batch later */
-    bool p_sel = false, p_hit = false;
-    uint32_t p_key = 0;
-
-    auto consume = [&]() {
-      uint64_t ms = __ballot(p_sel);
-      if (MEDIAN && p_sel) wlist[ns + (int32_t)lane_prefix(ms)] = p_key;
-      ns += (int32_t)__popcll(ms);
-      bool hit;
-      if (MEDIAN) hit = p_sel && g->has_hit && p_key <= g->hit_key;
-      else hit = p_hit;
-      ni += (int32_t)__popcll(__ballot(hit));
-      p_sel = false;
-      p_hit = false;
-    };
-
-    /* gather: distance key (or hit bit) of n selected events of ring3 */
-    auto gather = [&](uint32_t n) {
-      consume();
-      if ((uint32_t)lane < n) {
-        uint32_t idx = ring3[(head3 + lane) & (GRS_QCAP - 1)];
-        p_sel = true;
-        if (MEDIAN) p_key = a.keys[idx];
-        else if (a.count_keys) p_hit = g->has_hit && a.keys[idx] <= g->hit_key;
-        else p_hit = (hbits[idx >> 5] >> (idx & 31u)) & 1u;
-      }
-      head3 += n;
-    };
-
-    auto push3 = [&](bool sel, uint32_t idx) {
-      uint64_t m = __ballot(sel);
-      if (sel) ring3[(tail3 + lane_prefix(m)) & (GRS_QCAP - 1)] = idx;
-      tail3 += (uint32_t)__popcll(m);
-      if (tail3 - head3 >= 64) {
-        wave_sync();
-        gather(64);
-        wave_sync();
-      }
-    };
-
-    /* phase B2: exact pipeline on n events of ring2 */
-    auto b2 = [&](uint32_t n) {
-      bool sel = false;
-      uint32_t idx = 0;
-      if ((uint32_t)lane < n) {
-        double yz[2];
-        sel = exact_event(a.g, vpos, a.cs, gwt, ring2[(head2 + lane) & (GRS_QCAP - 1)], &idx, yz) != 0;
-        if (sel && tiled) {
-          const uint32_t omx = idx / nzny32, rem = idx - omx * nzny32, y0 = rem / nz32;
-          idx = grs_tiled_bit(omx, y0 + 1u, rem - y0 * nz32 + 1u, ntz, nty);
-        }
-      }
-      head2 += n;
-      push3(sel, idx);
-    };
-
-    /* phase B1: resolve n events of ring1 or queue them for the exact pipeline */
-    auto b1_core = [&](bool valid, uint32_t ev, uint32_t n) {
-      int st = 0;
-      uint32_t idx = 0;
-      bool bad = false, inwin = false;
-      double dev = 0.0;
-      if (valid) {
-        int32_t om = (int32_t)(ev >> 8), h = (int32_t)(ev & 255u);
-        const double *t = gwt + h * GRS_GWT;
-        b1_out o;
-        o.ry = o.rz = 0.0;
-        o.dy = o.dz = 0;
-        o.win = 0;
-        const double *brow = btab ? btab + GRS_BT * om : nullptr;
-        const double cc = brow ? brow[10] : a.cs[2 * om], ss = brow ? brow[11] : a.cs[2 * om + 1];
-        st = b1_classify(g, cc, ss, Pw, brow, t, b1thr, &o);
-        if (st == 1)
-          idx = tiled ? grs_tiled_bit((uint32_t)om, (uint32_t)o.dy, (uint32_t)o.dz, ntz, nty)
-                      : (uint32_t)(o.dz - 1) + (uint32_t)(o.dy - 1) * nz32 + (uint32_t)om * nzny32;
-        inwin = o.win != 0;
-        if (AUDIT) {
-          double yz[2] = {0.0, 0.0};
-          uint32_t eidx = 0;
-          const int es = exact_event(a.g, vpos, a.cs, gwt, ev, &eidx, yz);
-          bad = (st == 0 && es) || (st == 1 && (!es || eidx != idx));
-          if (st == 1 && es) dev = __builtin_fmax(__builtin_fabs(o.ry - yz[0]), __builtin_fabs(o.rz - yz[1]));
-        }
-      }
-      if (AUDIT) {
-        /* whole-wave reductions, outside the divergent block */
-        uint64_t mb = __ballot(bad), m1 = __ballot(st == 1), m0 = __ballot(valid && st == 0);
-        uint64_t m2 = __ballot(st == 2), mw = __ballot(inwin);
-        for (int off = 32; off >= 1; off >>= 1) dev = __builtin_fmax(dev, __shfl_xor(dev, off, 64));
-        if (lane == 0) {
-          atomicAdd(a.audit + 0, (unsigned long long)n);
-          atomicAdd(a.audit + 1, (unsigned long long)__popcll(m1));
-          atomicAdd(a.audit + 2, (unsigned long long)__popcll(m0));
-          atomicAdd(a.audit + 3, (unsigned long long)__popcll(m2));
-          atomicAdd(a.audit + 4, (unsigned long long)__popcll(mb));
-          atomicMax(a.audit + 5, (unsigned long long)__double_as_longlong(dev));
-          atomicAdd(a.audit + 6, (unsigned long long)__popcll(mw));
-        }
-      }
-      uint64_t m2 = __ballot(st == 2);
-      if (st == 2) ring2[(tail2 + lane_prefix(m2)) & (GRS_QCAP - 1)] = ev;
-      tail2 += (uint32_t)__popcll(m2);
-      push3(st == 1, idx);
-      if (tail2 - head2 >= 64) {
-        wave_sync();
-        b2(64);
-        wave_sync();
-      }
-    };
-
-    auto b1 = [&](uint32_t n) {
-      const bool valid = (uint32_t)lane < n;
-      const uint32_t ev = valid ? ring1[(head1 + lane) & (GRS_QCAP - 1)] : 0u;
-      head1 += n;
-      b1_core(valid, ev, n);
-    };
-
-    if (solve && !overflow) {
-      /* candidates of the omega solve, 64 per step, straight to phase B1.
-       * Ranges are non-empty and rcum is their exclusive prefix, so the range
-       * of candidate base + l is rb plus the number of later ranges that
-       * start at or before base + l, where rb is the last range starting
-       * before base (0 at base 0).  Those starts lie in the next 64 ranges;
-       * each marks its position in ring1 (unused on this path) and a ballot
-       * turns the marks into a bit mask. */
-      uint32_t rb = 0;
-      for (uint32_t base = 0; base < total; base += 64) {
-        const uint32_t idx = base + (uint32_t)lane;
-        const bool valid = idx < total;
-        ring1[lane] = 0u;
-        wave_sync();
-        const uint32_t rn = rb + 1u + (uint32_t)lane;
-        if (rn < R) {
-          const uint32_t p = rcum[rn] - base;
-          if (p < 64u) ring1[p] = 1u;
-        }
-        wave_sync();
-        const uint64_t starts = __ballot(ring1[lane] != 0u);
-        const uint64_t upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
-        const uint32_t r = rb + (uint32_t)__popcll(starts & upto);
-        rb += (uint32_t)__popcll(starts);
-        uint32_t ev = 0;
-        if (valid) {
-          const uint32_t st0 = rstart[r];
-          ev = (((st0 >> 8) + (idx - rcum[r])) << 8) | (st0 & 255u);
-        }
-        b1_core(valid, ev, total - base < 64u ? total - base : 64u);
-      }
-    }
-    /* phase A (no omega solve): wave-uniform steps of 64 consecutive events;
-     * lane l owns event l + 64*k, tracked as (omega, hkl) without divisions */
-    int32_t om = om0, h = h0;
-    const int32_t nsteps = (solve && !overflow) ? 0 : (nrot * H + 63) / 64;
-    for (int32_t k = 0; k < nsteps; ++k) {
-      bool pass = false;
-      if (om < nrot) {
-        const double c = a.cs[2 * om], s = a.cs[2 * om + 1];
-        double swv[3], uv[3];
-        beam_terms(g, Pw, c, s, swv, uv);
-        const double u0 = uv[0], u1 = uv[1], u2 = uv[2];
-        const double *t = gwt + h * GRS_GWT;
-        double Gt0 = c * t[0] - s * t[1];
-        double Gt1 = s * t[0] + c * t[1];
-        double dot = __builtin_fma(u2, t[2], __builtin_fma(u1, Gt1, u0 * Gt0));
-        double l4 = m4pi * dot;
-        /* the phase-A thresholds of the reflection (margins: see the header comment) */
-        const double gn = __builtin_sqrt(t[4]);
-        const double ml = lrel + (1e-12 * (4.0 * GRS_PI)) * t[3];
-        pass = (dot < dcb * gn) && (dot > cbm * gn) && (l4 > (lmin - ml) * t[4]) && (l4 < (lmax + ml) * t[4]);
-      }
-      uint64_t m = __ballot(pass);
-      if (pass) ring1[(tail1 + lane_prefix(m)) & (GRS_QCAP - 1)] = ((uint32_t)om << 8) | (uint32_t)h;
-      tail1 += (uint32_t)__popcll(m);
-      if (tail1 - head1 >= 64) {
-        wave_sync();
-        b1(64);
-        wave_sync();
-      }
-      h += 64;
-      while (h >= H) {
-        h -= H;
-        om++;
-      }
-    }
-    while (tail1 != head1) {
-      uint32_t n = tail1 - head1;
-      if (n > 64) n = 64;
-      wave_sync();
-      b1(n);
-      wave_sync();
-    }
-    while (tail2 != head2) {
-      uint32_t n = tail2 - head2;
-      if (n > 64) n = 64;
-      wave_sync();
-      b2(n);
-      wave_sync();
-    }
-    while (tail3 != head3) {
-      uint32_t n = tail3 - head3;
-      if (n > 64) n = 64;
-      wave_sync();
-      gather(n);
-      wave_sync();
-    }
-    consume();
     if (MEDIAN) {
       __threadfence_block();
       float med = 2000.0f;
@@ -1315,6 +1389,125 @@ __global__ __launch_bounds__(64 * GRS_WPB, GRS_FAST_MIN_WAVES) void k_fast(grs_e
       atomicMax(a.csr.row_best + row, (unsigned long long)((cpart << GRS_KEY_JBITS) | jpart));
     }
     wave_sync();
+  }
+}
+
+/* ---------------------------------------------------------------------- */
+/* orientation fits                                                        */
+
+/* One block per fit of 1 - Nr_intersect/Nr_simu over (q1, q2, q3)
+ * (fit_OR_constrain_with_local_comp_cuda.m:116-126): the whole
+ * fminsearchbnd on the device.  The block's 16 waves are four teams of four
+ * (score_events with the reflections split four ways), one team per point: a
+ * requested reflection is scored together with the three points that its
+ * value can lead to (grs_nm::follow_ups), the initial simplex and a shrink
+ * have at most four points.  The first wave steps the method
+ * (nm_lanes).  The points, values and counts are the sequential method's.
+ * Bound: one iteration's chain (a wave's events of 22 of 86 reflections, the step
+ * of the simplex and the barriers between).  A launch, two copies and a
+ * synchronisation per iteration took 3.3 ms for 24 fits of 64 iterations
+ * (52 us each, 36 of them one wave's walk through all events); this takes
+ * 1.5 ms.  GRS_FIT_SLICE requests end a launch, so that it ends whatever max_iter
+ * is; the host launches again while fits are left. */
+#define GRS_FIT_TEAM 4
+#define GRS_FIT_PTS 4
+#define GRS_FIT_SLICE 4096
+
+__global__ __launch_bounds__(64 * GRS_FIT_TEAM * GRS_FIT_PTS, GRS_FAST_MIN_WAVES) void k_fit_nm(
+    grs_eval_args a, int32_t H, const double *x0, double half_width, int32_t max_fe, int32_t max_it, double tol_f,
+    double tol_x, int32_t first, grs_nm *nms, double *res, int32_t *left) {
+  GRS_NO_CONTRACT
+  extern __shared__ double smem[];
+  __shared__ __align__(16) unsigned char nm_buf[sizeof(grs_nm)];
+  __shared__ double xs[GRS_FIT_PTS][3];
+  __shared__ grs_dgeo sg;
+  __shared__ double b1thr[12];
+  __shared__ int32_t cnt[GRS_FIT_PTS][2];
+  __shared__ int npts;
+  grs_nm *nm = reinterpret_cast<grs_nm *>(nm_buf);
+  const int t = threadIdx.x, lane = t & 63, wib = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int64_t m = blockIdx.x;
+  const int p = wib / GRS_FIT_TEAM, w = wib % GRS_FIT_TEAM;
+  const int32_t Hn = (H + GRS_FIT_TEAM - 1) / GRS_FIT_TEAM;
+  const int32_t hlo = w * Hn < H ? w * Hn : H, hend = hlo + Hn < H ? hlo + Hn : H;
+  const fast_lds_regions L = fast_regions(smem, wib, hlo, Hn);
+  if (t == 0) {
+    sg = *a.g;
+    b1_thresholds(&sg, b1thr);
+    if (first) {
+      double lo[3], hi[3], xm[3];
+      for (int k = 0; k < 3; k++) {
+        /* fit_OR_constrain_with_local_comp_cuda.m:124-125 */
+        xm[k] = x0[3 * m + k];
+        const double u = xm[k] - half_width, v = xm[k] + half_width;
+        lo[k] = grs_nm_max(u, -1.0);
+        hi[k] = (v != v) ? 1.0 : (v < 1.0 ? v : 1.0);
+      }
+      nm->max_fe = max_fe;
+      nm->max_it = max_it;
+      nm->tol_f = tol_f;
+      nm->tol_x = tol_x;
+      nm->nf = 0;
+      nm->it = 0;
+      nm->start(3, xm, lo, hi);
+    } else {
+      *nm = nms[m];
+    }
+  }
+  __syncthreads();
+  int32_t step = 0;
+  for (; step < GRS_FIT_SLICE; step++) {
+    if (t == 0) npts = nm->done() ? 0 : (nm->st == grs_nm::REFLECT ? 4 : nm->npend);
+    if (t < 2 * GRS_FIT_PTS) cnt[t >> 1][t & 1] = 0;
+    __syncthreads();
+    const int np = npts;
+    if (np == 0) break;
+    if (t < 3 * np) {
+      const int q = t / 3, k = t - 3 * q;
+      /* a reflection's follow-ups: grs_nm::follow_ups, coordinate k */
+      double u = nm->pend[q][k];
+      if (nm->st == grs_nm::REFLECT && q > 0) {
+        const double xb = nm->xbar[k], vn = nm->v[nm->n][k];
+        u = q == 1 ? (1.0 + 2.0) * xb - 2.0 * vn : q == 2 ? (1.0 + 0.5) * xb - 0.5 * vn : (1.0 - 0.5) * xb + 0.5 * vn;
+      }
+      double u3[3];
+      u3[k] = u;
+      nm->xform1(u3, k, &xs[q][k]);
+    }
+    __syncthreads();
+    double U[9], sub[9];
+    if (p < np && grs_U_from_q(xs[p][0], xs[p][1], xs[p][2], U)) {
+      grs_SUB(a.g, U, sub);
+      int32_t ns, ni;
+      score_events<false, false, true>(a, &sg, b1thr, nullptr, L, sub, m, hlo, hend, nullptr, nullptr, &ns, &ni);
+      if (lane == 0) {
+        atomicAdd(&cnt[p][0], ns);
+        atomicAdd(&cnt[p][1], ni);
+      }
+    }
+    __syncthreads();
+    if (wib == 0) {
+      /* fit_OR_fun_local.m:98; 0/0 (no event, or |q_vec| > 1) is NaN */
+      double f[GRS_FIT_PTS];
+#pragma unroll
+      for (int q = 0; q < GRS_FIT_PTS; q++) f[q] = 1.0 - (double)cnt[q][1] / (double)cnt[q][0];
+      nm_lanes S{nm, t, t < nm->n};
+      const bool refl = nm->st == grs_nm::REFLECT;
+      S.feed(f);
+      if (refl) {
+        const int q = nm->st == grs_nm::EXPAND ? 1 : nm->st == grs_nm::CONTRACT_OUT ? 2 : nm->st == grs_nm::CONTRACT_IN ? 3 : 0;
+        if (q > 0) S.feed(&f[q]);
+      }
+    }
+    __syncthreads();
+  }
+  if (t == 0) {
+    nms[m] = *nm;
+    if (!nm->done()) atomicAdd(left, 1);
+    double *r = res + 6 * m;
+    nm->result(r, r + 3);
+    r[4] = (double)nm->nf;
+    r[5] = (double)nm->it;
   }
 }
 
@@ -1579,13 +1772,13 @@ static size_t fast_lds(int32_t H, int wpb, const grs_eval_args *a) {
 
 /* Resident blocks per CU of one k_fast instantiation at wpb waves per block
  * (cached per wpb). */
-template <bool MEDIAN, int MAP, bool AUDIT>
+template <bool MEDIAN, int MAP, bool AUDIT, bool TEAM>
 static int fast_blocks_per_cu(size_t lds, int wpb) {
   static int cached[GRS_WPB + 1] = {0};
   static size_t cached_lds[GRS_WPB + 1] = {0};
   if (cached[wpb] == 0 || cached_lds[wpb] != lds) {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_fast<MEDIAN, MAP, AUDIT>, 64 * wpb, lds) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_fast<MEDIAN, MAP, AUDIT, TEAM>, 64 * wpb, lds) != hipSuccess ||
         nb <= 0)
       nb = 1;
     cached[wpb] = nb;
@@ -1602,35 +1795,69 @@ static int device_cus() {
   return cus;
 }
 
-/* Persistent launch: at most as many waves as can be resident at once. */
-template <bool MEDIAN, int MAP, bool AUDIT = false>
+/* Persistent launch: at most as many waves as can be resident at once.
+ * TEAM: the block's waves share each evaluation. */
+template <bool MEDIAN, int MAP, bool AUDIT = false, bool TEAM = false>
 static hipError_t launch_fast_impl(const grs_eval_args *a, int32_t H, int64_t n_waves, int wpb, hipStream_t st) {
   if (wpb != 1 && wpb != 2 && wpb != 4 && wpb != 8) return hipErrorInvalidValue;
-  /* every wave of the launch needs a scratch slot: fewer slots than a block
-   * has waves take smaller blocks */
-  while (wpb > 1 && n_waves < wpb) wpb >>= 1;
-  size_t lds = fast_lds(H, wpb, a);
+  /* every wave (team) of the launch needs a scratch slot: fewer slots than a
+   * block has waves take smaller blocks */
+  while (!TEAM && wpb > 1 && n_waves < wpb) wpb >>= 1;
+  size_t lds = TEAM ? (size_t)wpb * (size_t)fast_wave_doubles((H + wpb - 1) / wpb) * sizeof(double) : fast_lds(H, wpb, a);
   if (lds > 65536) {
     /* above the default dynamic LDS limit of a launch */
-    hipError_t e = hipFuncSetAttribute((const void *)k_fast<MEDIAN, MAP, AUDIT>,
+    hipError_t e = hipFuncSetAttribute((const void *)k_fast<MEDIAN, MAP, AUDIT, TEAM>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
   }
-  int64_t resident = (int64_t)device_cus() * fast_blocks_per_cu<MEDIAN, MAP, AUDIT>(lds, wpb);
-  int64_t blocks = n_waves / wpb; /* n_waves is a multiple of 4: no wave beyond the scratch slots */
+  int64_t resident = (int64_t)device_cus() * fast_blocks_per_cu<MEDIAN, MAP, AUDIT, TEAM>(lds, wpb);
+  int64_t blocks = TEAM ? a->n_eval - a->e0 : n_waves / wpb; /* n_waves is a multiple of 4: no wave beyond the scratch slots */
+  if (TEAM && blocks > n_waves) blocks = n_waves;
   if (blocks > resident) blocks = resident;
   if (blocks < 1) blocks = 1;
-  hipLaunchKernelGGL((k_fast<MEDIAN, MAP, AUDIT>), dim3((unsigned)blocks), dim3(64 * wpb), lds, st, *a, H);
+  hipLaunchKernelGGL((k_fast<MEDIAN, MAP, AUDIT, TEAM>), dim3((unsigned)blocks), dim3(64 * wpb), lds, st, *a, H);
+  return hipGetLastError();
+}
+
+/* Waves that share an evaluation in a launch of n evaluations (1: none).
+ * While the chip has more SIMDs than evaluations the call takes as long as
+ * one wave's walk through an evaluation's events, and splitting the
+ * reflections shortens it; the set-up is repeated by every wave, so larger launches
+ * lose.  A one-voxel call of 100, 300, 729, 1500, 2187, 4000 orientations (86
+ * reflections, 181 angles; whole call on resident buffers, us): a wave each
+ * 44, 73, 69, 78, 75, 71; two 37, 40, 44, 54, 70, 86; four 35, 38, 44, 66, 81,
+ * 118; eight 34, 41, 58, 86, 112, 179.  The order is the same with 64 x 361. */
+static int fast_team(int64_t n) { return n <= 512 ? 4 : n <= 2560 ? 2 : 1; }
+
+template <int MAP>
+static hipError_t launch_fast_median(const grs_eval_args *a, int32_t H, int64_t n_waves, int wpb, hipStream_t st) {
+  const int team = fast_team(a->n_eval - a->e0);
+  if (team > 1) return launch_fast_impl<true, MAP, false, true>(a, H, n_waves, team, st);
+  return launch_fast_impl<true, MAP>(a, H, n_waves, wpb, st);
+}
+
+size_t grs_fit_nm_bytes(void) { return sizeof(grs_nm); }
+
+hipError_t grs_launch_fit_nm(const grs_eval_args *a, int32_t H, int64_t M, const double *d_x0, double half_width,
+                             int32_t max_fe, int32_t max_it, double tol_f, double tol_x, int32_t first, void *d_nm,
+                             double *d_res, int32_t *d_left, hipStream_t st) {
+  if (M <= 0) return hipSuccess;
+  const int waves = GRS_FIT_TEAM * GRS_FIT_PTS;
+  const size_t lds = (size_t)waves * (size_t)fast_wave_doubles((H + GRS_FIT_TEAM - 1) / GRS_FIT_TEAM) * sizeof(double);
+  hipError_t e = hipFuncSetAttribute((const void *)k_fit_nm, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_fit_nm, dim3((unsigned)M), dim3(64 * waves), lds, st, *a, H, d_x0, half_width, max_fe, max_it,
+                     tol_f, tol_x, first, static_cast<grs_nm *>(d_nm), d_res, d_left);
   return hipGetLastError();
 }
 
 hipError_t grs_launch_fast(const grs_eval_args *a, int32_t H, int64_t n_waves, int32_t wpb, hipStream_t st) {
   if (a->n_eval <= a->e0) return hipSuccess;
   switch (a->map) {
-    case GRS_MAP_ONE_VOXEL: return launch_fast_impl<true, GRS_MAP_ONE_VOXEL>(a, H, n_waves, wpb, st);
-    case GRS_MAP_ONE_U: return launch_fast_impl<true, GRS_MAP_ONE_U>(a, H, n_waves, wpb, st);
-    case GRS_MAP_PAIRS: return launch_fast_impl<true, GRS_MAP_PAIRS>(a, H, n_waves, wpb, st);
-    case GRS_MAP_CSR_LIST: return launch_fast_impl<true, GRS_MAP_CSR_LIST>(a, H, n_waves, wpb, st);
+    case GRS_MAP_ONE_VOXEL: return launch_fast_median<GRS_MAP_ONE_VOXEL>(a, H, n_waves, wpb, st);
+    case GRS_MAP_ONE_U: return launch_fast_median<GRS_MAP_ONE_U>(a, H, n_waves, wpb, st);
+    case GRS_MAP_PAIRS: return launch_fast_median<GRS_MAP_PAIRS>(a, H, n_waves, wpb, st);
+    case GRS_MAP_CSR_LIST: return launch_fast_median<GRS_MAP_CSR_LIST>(a, H, n_waves, wpb, st);
     default: return hipErrorInvalidValue;
   }
 }

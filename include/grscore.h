@@ -294,11 +294,9 @@ grs_status grs_device_copy(grs_ctx *ctx, void *d_dst, const void *d_src, int64_t
  * max(x0 - half_width, -1) .. min(x0 + half_width, 1) (the reference uses
  * 0.02), by fminsearchbnd with MaxFunEvals, MaxIter, TolFun, TolX (the
  * reference passes 2000, 2000, 1e-10 and the default 1e-4).  Each fit follows
- * the sequential method exactly; the evaluations of all active fits are
- * scored together in one device launch per step (while the batch is small,
- * with each requested reflection's three possible follow-ups, so that an
- * expansion or contraction needs no launch of its own; the counts returned
- * are the method's own).  A point with no selected
+ * the sequential method exactly and runs to its end on the device, one block
+ * per fit (a requested reflection is scored together with its three possible
+ * follow-ups; the counts returned are the method's own).  A point with no selected
  * event or |q_vec| > 1 has the value NaN.  Outputs: x_out (3 per fit), fval,
  * the number of evaluations and of iterations. */
 grs_status grs_fit_or_local(grs_ctx *ctx, const double *pos, const double *x0, int64_t M, double half_width,
@@ -547,8 +545,9 @@ grs_status grs_get_tuning(grs_ctx *ctx, int32_t kind, int32_t *waves_per_block, 
  * waves per block 1, 2, 4 or 8, a GRS_MASK_* source (GRS_MASK_BITS for kind 0),
  * XCD mapping 0 or 1.  waves_per_block = 0 forgets the kind's configuration,
  * so that the next large call tunes again.  Whatever the configuration, a
- * launch of fewer waves than the device has CUs (the orientation fits'
- * steps) runs one wave per block.  No reference counterpart. */
+ * counts-only launch of fewer waves than the device has CUs runs one wave per
+ * block, and a launch of kind 0 with up to 2560 evaluations shares each of
+ * them among the waves of a block.  No reference counterpart. */
 grs_status grs_set_launch_config(grs_ctx *ctx, int32_t kind, int32_t waves_per_block, int32_t mask_layout,
                                  int32_t xcd_map);
 

@@ -174,6 +174,26 @@ def test_grow_parity(engine, method):
         assert got[:, 6].sum() > 0
 
 
+@pytest.mark.parametrize("H", [1, 3, 65, 86, 240])
+def test_small_launches_share_evaluations(engine, H):
+    """Launch sizes around the rules that share an evaluation among four or
+    two waves, with reflection counts that leave waves without work, uneven
+    or whole shares, on uniform rotation angles and on others (where a wave
+    scans its own events): counts, C and median equal the plain kernel's."""
+    s = scenes.make_scene(seed=47, ngrains=2, spread_mm=0.02, nrot=13)
+    hkl = np.concatenate([s.hkl, 2 * s.hkl, 3 * s.hkl])[:H]
+    rng = np.random.default_rng(H)
+    uneven = np.sort(rng.uniform(0, 360, s.rot.size))
+    for rot in (s.rot, uneven):
+        engine.set_geometry(s.geo, hkl, rot)
+        engine.set_distance_stack(s.proj)
+        q = np.concatenate([s.q, [[0.1, 0.9, 0.5, 0.3]], scenes.random_quats(rng, 2600)])
+        ref = engine.forward_comp(s.centers[0], q, _lib.METHOD_PLAIN)
+        for n in (1, 2, 511, 512, 513, 2560, 2561):
+            for x, y in zip(engine.forward_comp(s.centers[0], q[:n]), ref):
+                assert np.array_equal(_bits(x), _bits(y[:n])), n
+
+
 @pytest.mark.parametrize("M", [1, 255, 257, 1023, 1024, 16384, 16385, 32768, 262145])
 def test_grow_row_counts(engine, M):
     """Row counts around the blocks of the row listing and around the rules

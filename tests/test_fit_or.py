@@ -55,3 +55,40 @@ def test_batched_fit_equals_sequential_oracle(engine, scene):
         assert (fv[m] == rf) or (np.isnan(fv[m]) and np.isnan(rf))
         assert nf[m] == rnf and it[m] == rit
     assert np.sum(fv[:5] < 0.5) >= 3 and np.isnan(fv[5]) and nf[5] >= 2000
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [1, 3, 85, 86])
+def test_fits_with_uneven_reflection_shares(engine, scene, H):
+    """Reflection counts that split unevenly over a team's waves (some left
+    without any), with the hits read from the keys and from the bit mask
+    (which a counts-only call builds): each fit equals the sequential one."""
+    s = scene
+    hkl = s.hkl[:H]
+    engine.set_geometry(s.geo, hkl, s.rot)
+    engine.set_distance_stack(s.proj)
+    pos, x0 = _starts(s, np.random.default_rng(H), 3)
+    ref = [fit_or_local(s.geo, s.stack, pos[m], x0[m], s.rot, hkl, max_fun_evals=60) for m in range(3)]
+    for _ in range(2):
+        x, fv, nf, it = engine.fit_or_local(pos, x0, max_fun_evals=60)
+        for m, (rx, rf, rnf, rit) in enumerate(ref):
+            np.testing.assert_array_equal(x[m], rx)
+            assert (fv[m] == rf or (np.isnan(fv[m]) and np.isnan(rf))) and nf[m] == rnf and it[m] == rit
+        engine.compete_csr(pos[:1], [0, 1], s.q[:1], 2, 0.004)
+
+
+@pytest.mark.gpu
+def test_fit_longer_than_one_launch(engine, scene):
+    """A fit whose every value is NaN shrinks at each iteration: 4 + 5 k
+    evaluations after k iterations, so 20,000 end it at 20,004 in iteration
+    4,001, more requests than one launch serves."""
+    s = scene
+    engine.set_geometry(s.geo, s.hkl, s.rot)
+    engine.set_distance_stack(s.proj)
+    pos, x0 = _starts(s, np.random.default_rng(5), 2)
+    x0[1] = [0.9, 0.5, 0.3]
+    x, fv, nf, it = engine.fit_or_local(pos, x0, max_fun_evals=20000, max_iter=1000000)
+    assert np.isnan(fv[1]) and nf[1] == 20004 and it[1] == 4001
+    rx, rf, rnf, rit = fit_or_local(s.geo, s.stack, pos[0], x0[0], s.rot, s.hkl, max_fun_evals=20000, max_iter=1000000)
+    np.testing.assert_array_equal(x[0], rx)
+    assert fv[0] == rf and nf[0] == rnf and it[0] == rit
