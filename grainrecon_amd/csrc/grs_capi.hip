@@ -103,7 +103,7 @@ struct grs_ctx {
   /* grain centre-of-mass fit buffers */
   DevBuf m_rows, m_rptr, m_nm, m_cs, m_dis;
   DevBuf f_in, f_cnt; /* fit_batch: packed per-step inputs and counts */
-  void *h_pin = nullptr; /* pinned staging of fit_batch (hipHostMalloc) */
+  void *h_pin = nullptr; /* pinned memory of small calls (ensure_pin) */
   size_t h_pin_cap = 0;
   unsigned char *h_stage = nullptr; /* pinned staging of large transfers (staged_copy) */
   /* device address of this GPU's allocation-free scratch (nullptr if the
@@ -123,6 +123,9 @@ struct grs_ctx {
 /* event pairs created with the context (no call creates events later, the
  * allocation-free entry included) */
 static const int64_t kTimingPairs = 64;
+
+/* evaluations up to which a host call goes through pinned memory (forward_comp_impl) */
+static const int64_t kPinnedEvals = 8192;
 
 /* adds the elapsed times of the recorded pairs to the totals */
 static hipError_t timing_harvest(grs_ctx *c) {
@@ -383,6 +386,13 @@ grs_status grs_create(int32_t device, grs_ctx **out) {
   /* the allocation-free entry's scratch on this device (a failed lookup
    * only disables that entry, which then reports the reason) */
   c->noalloc = noalloc_lookup(device, c->noalloc_err, sizeof(c->noalloc_err));
+  /* the pinned memory of small calls (allocated by the first one otherwise) */
+  if (hipHostMalloc(&c->h_pin, 52 * kPinnedEvals, hipHostMallocDefault) == hipSuccess) {
+    c->h_pin_cap = 52 * kPinnedEvals;
+  } else {
+    c->h_pin = nullptr;
+    (void)hipGetLastError();
+  }
   *out = c;
   return GRS_OK;
 }
@@ -750,6 +760,22 @@ static grs_status run_eval(grs_ctx *c, int32_t map, int64_t n_eval, int64_t V, c
   return GRS_OK;
 }
 
+/* c->h_pin holds at least bytes (its contents are lost when it grows) */
+static grs_status ensure_pin(grs_ctx *c, size_t bytes) {
+  if (c->h_pin_cap >= bytes) return GRS_OK;
+  if (c->h_pin) HIPCHK(c, hipHostFree(c->h_pin));
+  c->h_pin = nullptr;
+  c->h_pin_cap = 0;
+  const hipError_t e = hipHostMalloc(&c->h_pin, 2 * bytes, hipHostMallocDefault);
+  if (e != hipSuccess) {
+    c->h_pin = nullptr;
+    (void)hipGetLastError();
+    return fail(c, GRS_ERR_NOMEM, "hipHostMalloc(%zu bytes) failed: %s", 2 * bytes, hipGetErrorString(e));
+  }
+  c->h_pin_cap = 2 * bytes;
+  return GRS_OK;
+}
+
 static grs_status forward_comp_impl(grs_ctx *c, const double *pos, const double *q, int64_t N, bool q_dev,
                                     int32_t *ns, int32_t *ni, double *C, float *med, bool out_dev,
                                     int32_t method) {
@@ -760,7 +786,26 @@ static grs_status forward_comp_impl(grs_ctx *c, const double *pos, const double 
   if (s != GRS_OK) return s;
   if (N == 0) return GRS_OK;
   const double *d_q = q;
-  if (!q_dev) {
+  int32_t *d_ns = ns, *d_ni = ni;
+  double *d_C = C;
+  float *d_med = med;
+  /* small calls on host buffers (q and the outputs together): the kernels read
+   * the orientations from pinned host memory and write the results there,
+   * without copy commands (five of them and their gaps were 60 of 145 us for 729
+   * orientations); a call of kPinnedEvals moves 0.4 MB, 8 us on the bus */
+  const bool pinned = !q_dev && !out_dev && N <= kPinnedEvals;
+  unsigned char *pin = nullptr;
+  if (pinned) {
+    s = ensure_pin(c, (size_t)N * 52);
+    if (s != GRS_OK) return s;
+    pin = static_cast<unsigned char *>(c->h_pin);
+    std::memcpy(pin, q, sizeof(double) * 4 * (size_t)N);
+    d_q = reinterpret_cast<const double *>(pin);
+    d_C = reinterpret_cast<double *>(pin + 32 * N);
+    d_ns = reinterpret_cast<int32_t *>(pin + 40 * N);
+    d_ni = reinterpret_cast<int32_t *>(pin + 44 * N);
+    d_med = reinterpret_cast<float *>(pin + 48 * N);
+  } else if (!q_dev) {
     ENSURE(c, c->d_q, sizeof(double) * 4 * N);
     HIPCHK(c, hipMemcpyAsync(c->d_q.p, q, sizeof(double) * 4 * N, hipMemcpyHostToDevice, c->st));
     d_q = P<double>(c->d_q);
@@ -768,13 +813,10 @@ static grs_status forward_comp_impl(grs_ctx *c, const double *pos, const double 
   ENSURE(c, c->d_sub, sizeof(double) * 9 * N);
   ENSURE(c, c->d_valid, sizeof(int32_t) * N);
   ENSURE(c, c->d_pos, sizeof(double) * 3);
-  HIPCHK(c, hipMemcpyAsync(c->d_pos.p, pos, sizeof(double) * 3, hipMemcpyHostToDevice, c->st));
-  HIPCHK(c, grs_launch_sub_from_q(P<grs_dgeo>(c->d_geo), d_q, N, P<double>(c->d_sub), P<int32_t>(c->d_valid),
-                                  c->st));
-  int32_t *d_ns = ns, *d_ni = ni;
-  double *d_C = C;
-  float *d_med = med;
-  if (!out_dev) {
+  ENSURE(c, c->d_vb, sizeof(double) * GRS_VB);
+  HIPCHK(c, grs_launch_one_voxel(P<grs_dgeo>(c->d_geo), pos, P<double>(c->d_cs), c->nrot, d_q, N, P<double>(c->d_pos),
+                                 P<double>(c->d_vb), P<double>(c->d_sub), P<int32_t>(c->d_valid), c->st));
+  if (!out_dev && !pinned) {
     ENSURE(c, c->d_ns, sizeof(int32_t) * N);
     ENSURE(c, c->d_ni, sizeof(int32_t) * N);
     ENSURE(c, c->d_C, sizeof(double) * N);
@@ -784,9 +826,18 @@ static grs_status forward_comp_impl(grs_ctx *c, const double *pos, const double 
     d_C = P<double>(c->d_C);
     d_med = P<float>(c->d_med);
   }
-  s = run_eval(c, GRS_MAP_ONE_VOXEL, N, 1, nullptr, nullptr, method, d_ns, d_ni, d_C, d_med);
-  if (s != GRS_OK) return s;
-  if (!out_dev) {
+  s = run_eval(c, GRS_MAP_ONE_VOXEL, N, 1, nullptr, nullptr, method, d_ns, d_ni, d_C, d_med, true);
+  if (s != GRS_OK) {
+    if (pinned) (void)hipStreamSynchronize(c->st); /* nothing reads the pinned memory any more */
+    return s;
+  }
+  if (pinned) {
+    HIPCHK(c, hipStreamSynchronize(c->st));
+    std::memcpy(C, d_C, sizeof(double) * (size_t)N);
+    std::memcpy(ns, d_ns, sizeof(int32_t) * (size_t)N);
+    std::memcpy(ni, d_ni, sizeof(int32_t) * (size_t)N);
+    std::memcpy(med, d_med, sizeof(float) * (size_t)N);
+  } else if (!out_dev) {
     HIPCHK(c, hipMemcpyAsync(ns, d_ns, sizeof(int32_t) * N, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipMemcpyAsync(ni, d_ni, sizeof(int32_t) * N, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipMemcpyAsync(C, d_C, sizeof(double) * N, hipMemcpyDeviceToHost, c->st));
@@ -1590,22 +1641,6 @@ grs_status grs_cuda_forward_comp_compete(const float *vox, int64_t n_vox, const 
 }
 
 /* ---- orientation fit --------------------------------------------------------- */
-
-/* c->h_pin holds at least bytes (its contents are lost when it grows) */
-static grs_status ensure_pin(grs_ctx *c, size_t bytes) {
-  if (c->h_pin_cap >= bytes) return GRS_OK;
-  if (c->h_pin) HIPCHK(c, hipHostFree(c->h_pin));
-  c->h_pin = nullptr;
-  c->h_pin_cap = 0;
-  const hipError_t e = hipHostMalloc(&c->h_pin, 2 * bytes, hipHostMallocDefault);
-  if (e != hipSuccess) {
-    c->h_pin = nullptr;
-    (void)hipGetLastError();
-    return fail(c, GRS_ERR_NOMEM, "hipHostMalloc(%zu bytes) failed: %s", 2 * bytes, hipGetErrorString(e));
-  }
-  c->h_pin_cap = 2 * bytes;
-  return GRS_OK;
-}
 
 /* M fits, fit m at pos[3m..] from x0[3m..] (the body of grs_fit_or_local) */
 static grs_status fit_batch(grs_ctx *c, const double *pos, const double *x0, int64_t M, double half_width,

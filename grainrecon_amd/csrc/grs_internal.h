@@ -104,6 +104,11 @@ hipError_t grs_launch_voxel_bounds(const grs_dgeo *d_g, const double *d_pos, int
                                    int32_t nrot, double *d_vb, hipStream_t st);
 hipError_t grs_launch_voxel_pos(const double *d_rows, int64_t M, int32_t row_stride, const double *d_p1,
                                 double *d_pos, hipStream_t st);
+/* the position pos (host) of a one-voxel launch and its bounds, and S*U*B of
+ * N orientations; d_q may be pinned host memory */
+hipError_t grs_launch_one_voxel(const grs_dgeo *d_g, const double *pos, const double *d_cs, int32_t nrot,
+                                const double *d_q, int64_t N, double *d_pos, double *d_vb, double *d_SUB,
+                                int32_t *d_valid, hipStream_t st);
 hipError_t grs_launch_sub_from_q(const grs_dgeo *d_g, const double *d_q, int64_t N, double *d_SUB, int32_t *d_valid,
                                  hipStream_t st);
 hipError_t grs_launch_sub_from_U(const grs_dgeo *d_g, const double *d_U, int64_t N, double *d_SUB, int32_t *d_valid,

@@ -277,12 +277,11 @@ __device__ __forceinline__ void vb_write(const grs_dgeo *g, double al, double be
  * one-voxel call short), and the extremes are reduced across each wave and
  * then across the four waves; maxima, minima and flags are exact, so the
  * result does not depend on the partition. */
-__global__ __launch_bounds__(256) void k_voxel_bounds(const grs_dgeo *g, const double *pos, int64_t V,
-                                                      const double *cs, int32_t nrot, double *vb) {
+__device__ __forceinline__ void voxel_bounds_block(const grs_dgeo *g, const double *pos, const double *cs,
+                                                   int32_t nrot, double *vb) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int64_t v = blockIdx.x; /* one block per voxel, one omega per thread */
   double P[3];
-  voxel_P(g, pos + 3 * v, P);
+  voxel_P(g, pos, P);
   const double al = P[0] / g->Lss, be = P[1] / g->Lss, ga = (g->RAO - g->P0y) / g->Lss;
   const double oy = g->RAO - g->P0y, oz = -g->P0z;
   const double on = __builtin_sqrt(oy * oy + oz * oz);
@@ -331,7 +330,13 @@ __global__ __launch_bounds__(256) void k_voxel_bounds(const grs_dgeo *g, const d
     A.rows = A.rows && r[10] != 0.0;
     nan_any = nan_any || r[11] != 0.0;
   }
-  vb_write(g, al, be, ga, A, nan_any, vb + GRS_VB * v);
+  vb_write(g, al, be, ga, A, nan_any, vb);
+}
+
+__global__ __launch_bounds__(256) void k_voxel_bounds(const grs_dgeo *g, const double *pos, const double *cs,
+                                                      int32_t nrot, double *vb) {
+  const int64_t v = blockIdx.x;
+  voxel_bounds_block(g, pos + 3 * v, cs, nrot, vb + GRS_VB * v);
 }
 
 /* The same bounds with L lanes per voxel (a power of two), lane l taking the
@@ -491,6 +496,30 @@ __global__ void k_sub_from_q(const grs_dgeo *g, const double *q, int64_t N, doub
   if (i >= N) return;
   double U[9];
   int ok = grs_U_from_q(q[4 * i + 1], q[4 * i + 2], q[4 * i + 3], U);
+  valid[i] = ok;
+  if (ok) grs_SUB(g, U, SUB + 9 * i);
+  else
+    for (int k = 0; k < 9; k++) SUB[9 * i + k] = 0.0;
+}
+
+/* What a one-voxel launch needs beside the stack, in one kernel: block 0
+ * writes the position (which comes with the launch) and its bounds, the
+ * others S*U*B of 256 orientations each. */
+struct one_pos {
+  double x[3];
+};
+__global__ __launch_bounds__(256) void k_one_voxel(const grs_dgeo *g, one_pos at, const double *cs, int32_t nrot,
+                                                   const double *q, int64_t N, double *pos, double *vb, double *SUB,
+                                                   int32_t *valid) {
+  if (blockIdx.x == 0) {
+    if (threadIdx.x < 3) pos[threadIdx.x] = at.x[threadIdx.x];
+    voxel_bounds_block(g, at.x, cs, nrot, vb);
+    return;
+  }
+  const int64_t i = (int64_t)(blockIdx.x - 1) * 256 + threadIdx.x;
+  if (i >= N) return;
+  double U[9];
+  const int ok = grs_U_from_q(q[4 * i + 1], q[4 * i + 2], q[4 * i + 3], U);
   valid[i] = ok;
   if (ok) grs_SUB(g, U, SUB + 9 * i);
   else
@@ -1732,7 +1761,7 @@ hipError_t grs_launch_voxel_bounds(const grs_dgeo *d_g, const double *d_pos, int
    * counts: 6 us for one voxel), else enough lanes per voxel for about eight
    * waves per SIMD of 256 CUs */
   if (V < 1024)
-    hipLaunchKernelGGL(k_voxel_bounds, dim3((unsigned)V), dim3(256), 0, st, d_g, d_pos, V, d_cs, nrot, d_vb);
+    hipLaunchKernelGGL(k_voxel_bounds, dim3((unsigned)V), dim3(256), 0, st, d_g, d_pos, d_cs, nrot, d_vb);
   else if (V < 32768)
     hipLaunchKernelGGL(k_voxel_bounds_lanes<16>, dim3((unsigned)((V * 16 + 255) / 256)), dim3(256), 0, st, d_g, d_pos,
                        V, d_cs, nrot, d_vb);
@@ -1742,6 +1771,15 @@ hipError_t grs_launch_voxel_bounds(const grs_dgeo *d_g, const double *d_pos, int
   else
     hipLaunchKernelGGL(k_voxel_bounds_lanes<1>, dim3((unsigned)((V + 255) / 256)), dim3(256), 0, st, d_g, d_pos, V,
                        d_cs, nrot, d_vb);
+  return hipGetLastError();
+}
+
+hipError_t grs_launch_one_voxel(const grs_dgeo *d_g, const double *pos, const double *d_cs, int32_t nrot,
+                                const double *d_q, int64_t N, double *d_pos, double *d_vb, double *d_SUB,
+                                int32_t *d_valid, hipStream_t st) {
+  one_pos at = {{pos[0], pos[1], pos[2]}};
+  hipLaunchKernelGGL(k_one_voxel, dim3((unsigned)(1 + (N + 255) / 256)), dim3(256), 0, st, d_g, at, d_cs, nrot, d_q, N,
+                     d_pos, d_vb, d_SUB, d_valid);
   return hipGetLastError();
 }
 

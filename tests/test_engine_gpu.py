@@ -174,6 +174,21 @@ def test_grow_parity(engine, method):
         assert got[:, 6].sum() > 0
 
 
+@pytest.mark.parametrize("method", METHODS, ids=["fast", "plain"])
+def test_host_buffers_around_the_pinned_limit(engine, method):
+    """Host calls that go through pinned memory, and the next larger ones."""
+    s = scenes.make_scene(seed=49, ngrains=2, spread_mm=0.02, nrot=7)
+    engine.set_geometry(s.geo, s.hkl, s.rot)
+    engine.set_distance_stack(s.proj)
+    q = np.concatenate([s.q, [[0.1, 0.9, 0.5, 0.3]], scenes.random_quats(np.random.default_rng(49), 8191)])
+    whole = engine.forward_comp(s.centers[0], q, method)
+    ref = oracle.or_space_comp(s.geo, s.stack, s.centers[0], q[:64], s.rot, s.hkl)
+    assert np.array_equal(whole[0][:64], ref[:, 0]) and np.array_equal(_bits(whole[2][:64]), _bits(ref[:, 2].copy()))
+    for n in (1, 8191, 8192, 8193):
+        for x, y in zip(engine.forward_comp(s.centers[0], q[:n], method), whole):
+            assert np.array_equal(_bits(x), _bits(y[:n])), n
+
+
 @pytest.mark.parametrize("H", [1, 3, 65, 86, 240])
 def test_small_launches_share_evaluations(engine, H):
     """Launch sizes around the rules that share an evaluation among four or
