@@ -102,6 +102,50 @@ __device__ __forceinline__ void omega_terms(const grs_dgeo *g, const double *P, 
   w->ov2 = swv[2] - g->detz00;
 }
 
+/* The unrounded spot coordinates of an event from cos(beta) = cb, its rotated
+ * G (G1, G2; g2 = |G|^2) and the terms w; false where a guard sends it to
+ * the exact pipeline. */
+__device__ __forceinline__ bool b1_spot(const grs_dgeo *g, const om_terms &w, double G1, double G2, double cb,
+                                        double g2, const double *thr, double *ry, double *rz) {
+  const double omc = __builtin_fma(-cb, cb, 1.0);
+  const double cth = omc * fast_rsq(omc);
+  const double s2t = -2.0 * cb * cth;
+  const double c2t = __builtin_fma(-2.0 * cb, cb, 1.0);
+  const double nv2 = __builtin_fma(G1, G1, G2 * G2);
+  if (!(nv2 >= 1e-12 * g2)) return false;
+  /* the remaining per (voxel, omega) terms from u and SamposW: center is
+   * grainpos * L / grainpos(1), so center/|center| = u, center(2:3) =
+   * L u(2:3) / u0, L2 = (Lsd - SW1) / u0 (cos(alpha) = u0); K_out(2:3) =
+   * (dety22, detz22) - SamposW(2:3) = d + diffvec e; and the t numerator
+   * and offsets of forward_comp.m:51-54 */
+  const double k0 = w.k0, d1 = w.d1, d2 = w.d2, L2 = w.L2;
+  const double *R = g->R;
+  const double tnum = w.tnum;
+  const double ov1 = w.ov1, ov2 = w.ov2;
+  const double inv = fast_rsq(nv2);
+  const double ap = __builtin_fma(G1, w.u1, G2 * w.u2) * inv;
+  if (!(__builtin_fabs(ap) <= 0.99)) return false;
+  const double oma = __builtin_fma(-ap, ap, 1.0);
+  const double sph = oma * fast_rsq(oma);
+  const double sphy = __builtin_fma(sph, c2t, -ap * s2t);
+  if (!(__builtin_fabs(sphy) >= 1e-3)) return false;
+  const double diffvec = L2 * s2t * fast_rcp(sphy);
+  /* K_out = (Lsd, y22, z22) - SamposW unnormalised: t K_out is the same
+   * vector for K_out and K_out / |K_out|, and the guard |R(:,1) . K_out| >=
+   * 1e-3 |K_out| is taken squared */
+  const double k1 = __builtin_fma(diffvec * G1, inv, d1);
+  const double k2 = __builtin_fma(diffvec * G2, inv, d2);
+  const double kk = __builtin_fma(k0, k0, __builtin_fma(k1, k1, k2 * k2));
+  const double tden = __builtin_fma(R[0], k0, __builtin_fma(R[3], k1, R[6] * k2));
+  if (!(tden * tden >= 1e-6 * kk)) return false;
+  const double t = tnum * fast_rcp(tden);
+  const double w0 = __builtin_fma(t, k0, -k0), w1 = __builtin_fma(t, k1, ov1), w2 = __builtin_fma(t, k2, ov2);
+  /* thr[6..11]: -R(:,2) / pixelysize and -R(:,3) / pixelzsize */
+  *ry = __builtin_fma(thr[6], w0, __builtin_fma(thr[7], w1, __builtin_fma(thr[8], w2, g->dety0)));
+  *rz = __builtin_fma(thr[9], w0, __builtin_fma(thr[10], w1, __builtin_fma(thr[11], w2, g->detz0)));
+  return true;
+}
+
 __device__ __forceinline__ int b1_classify(const grs_dgeo *g, double c, double s, const double *P, const double *bt,
                                            const double *gt, const double *thr, b1_out *o) {
   om_terms w;
@@ -132,42 +176,8 @@ __device__ __forceinline__ int b1_classify(const grs_dgeo *g, double c, double s
   /* inside by less than the margins: the exact pipeline decides */
   if (!(cb < -1e-12 && cb > thr[3] && lam > thr[4] && lam < thr[5])) return 2;
   o->win = 1;
-  const double omc = __builtin_fma(-cb, cb, 1.0);
-  const double cth = omc * fast_rsq(omc);
-  const double s2t = -2.0 * cb * cth;
-  const double c2t = __builtin_fma(-2.0 * cb, cb, 1.0);
-  const double nv2 = __builtin_fma(G1, G1, G2 * G2);
-  if (!(nv2 >= 1e-12 * g2)) return 2;
-  /* the remaining per (voxel, omega) terms from u and SamposW: center is
-   * grainpos * L / grainpos(1), so center/|center| = u, center(2:3) =
-   * L u(2:3) / u0, L2 = (Lsd - SW1) / u0 (cos(alpha) = u0); K_out(2:3) =
-   * (dety22, detz22) - SamposW(2:3) = d + diffvec e; and the t numerator
-   * and offsets of forward_comp.m:51-54 */
-  const double k0 = w.k0, d1 = w.d1, d2 = w.d2, L2 = w.L2;
-  const double *R = g->R;
-  const double tnum = w.tnum;
-  const double ov1 = w.ov1, ov2 = w.ov2;
-  const double inv = fast_rsq(nv2);
-  const double ap = __builtin_fma(G1, u1, G2 * u2) * inv;
-  if (!(__builtin_fabs(ap) <= 0.99)) return 2;
-  const double oma = __builtin_fma(-ap, ap, 1.0);
-  const double sph = oma * fast_rsq(oma);
-  const double sphy = __builtin_fma(sph, c2t, -ap * s2t);
-  if (!(__builtin_fabs(sphy) >= 1e-3)) return 2;
-  const double diffvec = L2 * s2t * fast_rcp(sphy);
-  /* K_out = (Lsd, y22, z22) - SamposW unnormalised: t K_out is the same
-   * vector for K_out and K_out / |K_out|, and the guard |R(:,1) . K_out| >=
-   * 1e-3 |K_out| is taken squared */
-  const double k1 = __builtin_fma(diffvec * G1, inv, d1);
-  const double k2 = __builtin_fma(diffvec * G2, inv, d2);
-  const double kk = __builtin_fma(k0, k0, __builtin_fma(k1, k1, k2 * k2));
-  const double tden = __builtin_fma(R[0], k0, __builtin_fma(R[3], k1, R[6] * k2));
-  if (!(tden * tden >= 1e-6 * kk)) return 2;
-  const double t = tnum * fast_rcp(tden);
-  const double w0 = __builtin_fma(t, k0, -k0), w1 = __builtin_fma(t, k1, ov1), w2 = __builtin_fma(t, k2, ov2);
-  /* thr[6..11]: -R(:,2) / pixelysize and -R(:,3) / pixelzsize */
-  const double ry = __builtin_fma(thr[6], w0, __builtin_fma(thr[7], w1, __builtin_fma(thr[8], w2, g->dety0)));
-  const double rz = __builtin_fma(thr[9], w0, __builtin_fma(thr[10], w1, __builtin_fma(thr[11], w2, g->detz0)));
+  double ry, rz;
+  if (!b1_spot(g, w, G1, G2, cb, g2, thr, &ry, &rz)) return 2;
   o->ry = ry;
   o->rz = rz;
   double ky, kz;
