@@ -12,7 +12,11 @@
  *                    its search box and sets one bit per positive grain id in
  *                    an LDS bitset; an empty box is grown by 2 voxels and
  *                    scanned again; the first nr_max set bits (ascending ids,
- *                    the order of unique) are written out.
+ *                    the order of unique) are written out.  Bound: the box reads
+ *                    from L2 (41^3 ids a voxel); 30,000 voxels of 300 grains
+ *                    take 1.2 ms, with an atomic per voxel read 2.2 ms.
+ * k_count_scan, k_pack_ids  the lists one after the other with their
+ *                    [first last] positions.
  */
 #include <hip/hip_runtime.h>
 
@@ -176,14 +180,28 @@ __global__ __launch_bounds__(64) void k_find_neighbors(const int32_t *gid, int64
       const int64_t bx = hi[0] - lo[0] + 1, by = hi[1] - lo[1] + 1;
       const int64_t plane = bx * by;
       bool any = false;
+      int32_t last = 0; /* the id this lane saw last */
       for (int64_t z = lo[2]; z <= hi[2]; z++) {
         const int32_t *gz = gid + (z - 1) * nx * ny;
+        /* a lane walks t = iy * bx + ix in steps of 64; an id that the lane
+         * has just seen or that is already set costs no atomic (the lanes of a
+         * grain would queue for one word) */
+        int32_t iy = lane / (int32_t)bx, ix = lane - iy * (int32_t)bx;
+        const int32_t sy = 64 / (int32_t)bx, sx = 64 - sy * (int32_t)bx;
+        const int32_t *row = gz + (lo[0] - 1) + (lo[1] - 1) * nx;
         for (int64_t t = lane; t < plane; t += 64) {
-          const int64_t iy = t / bx, ix = t - iy * bx;
-          const int32_t id = gz[(lo[0] - 1 + ix) + (lo[1] - 1 + iy) * nx];
-          if (id > 0) {
-            atomicOr(&bits[id >> 5], 1u << (id & 31));
+          const int32_t id = row[ix + (int64_t)iy * nx];
+          if (id > 0 && id != last) {
+            last = id;
             any = true;
+            const uint32_t bit = 1u << (id & 31);
+            if (!(bits[id >> 5] & bit)) atomicOr(&bits[id >> 5], bit);
+          }
+          ix += sx;
+          iy += sy;
+          if (ix >= (int32_t)bx) {
+            ix -= (int32_t)bx;
+            iy++;
           }
         }
       }
@@ -226,6 +244,44 @@ __global__ __launch_bounds__(64) void k_find_neighbors(const int32_t *gid, int64
   }
 }
 
+/* off[m] = counts before m, off[M] = their sum: one block, thread t takes a
+ * run of consecutive counts */
+__global__ __launch_bounds__(1024) void k_count_scan(const int32_t *n, int64_t M, int64_t *off) {
+  __shared__ int64_t part[1024];
+  const int tid = threadIdx.x;
+  const int64_t per = (M + 1023) / 1024, lo = tid * per, hi = lo + per < M ? lo + per : M;
+  int64_t c = 0;
+  for (int64_t m = lo; m < hi; m++) c += n[m];
+  part[tid] = c;
+  __syncthreads();
+  for (int o = 1; o < 1024; o <<= 1) {
+    const int64_t v = tid >= o ? part[tid - o] : 0;
+    __syncthreads();
+    part[tid] += v;
+    __syncthreads();
+  }
+  int64_t run = part[tid] - c;
+  for (int64_t m = lo; m < hi; m++) {
+    off[m] = run;
+    run += n[m];
+  }
+  if (tid == 1023) off[M] = part[1023];
+}
+
+/* one voxel's ids after the other and their 1-based [first last]
+ * (find_neighbor_ORs.m:26-29) */
+__global__ __launch_bounds__(256) void k_pack_ids(const int32_t *ids, const int64_t *off, int64_t M, int32_t nr_max,
+                                                  int32_t *id_all, int64_t *ind) {
+  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < M * nr_max; t += (int64_t)gridDim.x * 256) {
+    const int64_t m = t / nr_max, k = t - m * nr_max, o = off[m], n = off[m + 1] - o;
+    if (k < n) id_all[o + k] = ids[t];
+    if (k == 0) {
+      ind[2 * m] = o + 1;
+      ind[2 * m + 1] = o + n;
+    }
+  }
+}
+
 /* ---------------------------------------------------------------------- */
 /* launchers                                                               */
 
@@ -245,5 +301,15 @@ hipError_t grs_launch_find_neighbors(const int32_t *d_gid, int64_t nx, int64_t n
   int64_t blocks = M < 65536 ? M : 65536;
   hipLaunchKernelGGL(k_find_neighbors, dim3((unsigned)blocks), dim3(64), sizeof(uint32_t) * (size_t)W, st, d_gid, nx,
                      ny, nz, d_vox, M, radius, nr_max, W, d_ids, d_nout, d_bad);
+  return hipGetLastError();
+}
+
+hipError_t grs_launch_pack_ids(const int32_t *d_ids, const int32_t *d_nout, int64_t M, int32_t nr_max, int64_t *d_off,
+                               int32_t *d_id_all, int64_t *d_ind, hipStream_t st) {
+  if (M <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_count_scan, dim3(1), dim3(1024), 0, st, d_nout, M, d_off);
+  const int64_t blocks = (M * nr_max + 255) / 256 < 65536 ? (M * nr_max + 255) / 256 : 65536;
+  hipLaunchKernelGGL(k_pack_ids, dim3((unsigned)blocks), dim3(256), 0, st, d_ids, d_off, M, nr_max,
+                     d_id_all, d_ind);
   return hipGetLastError();
 }

@@ -55,10 +55,10 @@ struct grs_ctx {
   int64_t snz = 0, sny = 0, snrot = 0;
   DevBuf d_geo, d_hkl, d_rot, d_cs, d_keys;
   DevBuf d_q, d_sub, d_valid, d_pos, d_vb, d_scratch, d_ns, d_ni, d_C, d_med;
-  DevBuf d_rows, d_p1, d_U, d_eu, d_rowstart, d_best, d_evox, d_eu_idx, d_bad, d_x, d_y;
+  DevBuf d_rows, d_p1, d_U, d_eu, d_rowstart, d_evox, d_eu_idx, d_bad, d_x, d_y;
   DevBuf d_mask, d_g1, d_edt_v, d_edt_z, d_grain;
   DevBuf d_bits, d_tbits, d_rowptr, d_roweoff, d_candq, d_rowbest, d_elist;
-  DevBuf c_cen, c_grid, c_gn, c_out, c_n, c_gid, c_vox, c_ids, c_nout;
+  DevBuf c_cen, c_grid, c_gn, c_out, c_n, c_gid, c_vox, c_ids, c_nout, c_off, c_pack, c_ind;
   bool bits_valid = false; /* hit mask matches the current stack and threshold */
   bool tbits_ok = false;    /* the tiled hit mask exists (its bit numbers fit 32 bits) */
   /* resident matched-spot set of the fits */
@@ -346,12 +346,6 @@ static unsigned char *noalloc_lookup(int device, char *err, size_t errlen) {
   return g_noalloc_ptr[device];
 }
 
-static double nanmin2(double a, double b) {
-  if (a != a) return b;
-  if (b != b) return a;
-  return b < a ? b : a;
-}
-
 extern "C" {
 
 const char *grs_version(void) { return "grscore 0.1 (gfx950)"; }
@@ -403,7 +397,7 @@ void grs_destroy(grs_ctx *c) {
   hipStreamSynchronize(c->st);
   DevBuf *bufs[] = {&c->d_geo, &c->d_hkl, &c->d_rot, &c->d_cs, &c->d_keys, &c->d_q, &c->d_sub, &c->d_valid,
                     &c->d_pos, &c->d_vb, &c->d_scratch, &c->d_ns, &c->d_ni, &c->d_C, &c->d_med, &c->d_rows,
-                    &c->d_p1, &c->d_U, &c->d_eu, &c->d_rowstart, &c->d_best, &c->d_evox, &c->d_eu_idx,
+                    &c->d_p1, &c->d_U, &c->d_eu, &c->d_rowstart, &c->d_evox, &c->d_eu_idx,
                     &c->d_bad, &c->d_x, &c->d_y, &c->d_mask, &c->d_g1, &c->d_edt_v, &c->d_edt_z,
                     &c->d_grain, &c->d_bits, &c->d_tbits, &c->d_rowptr, &c->d_roweoff, &c->d_candq, &c->d_rowbest,
                     &c->d_elist, &c->f_hkl, &c->f_om, &c->f_meas, &c->f_grain, &c->f_goff, &c->f_gr6,
@@ -419,7 +413,7 @@ void grs_destroy(grs_ctx *c) {
                     &c->r_rows, &c->r_counts, &c->r_acc_lin, &c->r_acc_C, &c->t_pos, &c->t_proj, &c->t_units,
                     &c->t_fam, &c->t_dposs, &c->t_glen, &c->t_scratch, &c->t_out, &c->m_rows, &c->m_rptr,
                     &c->m_nm, &c->t_skey, &c->t_su, &c->t_bst, &c->t_slen, &c->t_sorig, &c->v_lin,
-                    &c->v_out, &c->f_in, &c->f_cnt, &c->m_cs, &c->m_dis, &c->t_band};
+                    &c->v_out, &c->f_in, &c->f_cnt, &c->m_cs, &c->m_dis, &c->t_band, &c->c_off, &c->c_pack, &c->c_ind};
   if (c->g_exec) hipGraphExecDestroy(c->g_exec);
   for (auto &kv : c->gi_cache) hipGraphExecDestroy(kv.second);
   for (hipEvent_t e : c->tev) hipEventDestroy(e);
@@ -1016,11 +1010,6 @@ grs_status grs_forward_comp_compete(grs_ctx *c, const double *vox, int64_t M, co
   grs_status s = check_ready(c);
   if (s != GRS_OK) return s;
   if (M == 0) return GRS_OK;
-  for (int64_t j = 0; j < n_id; j++) {
-    double g = id_all[j];
-    if (!(g >= 1.0 && g <= (double)G && g == std::floor(g)))
-      return fail(c, GRS_ERR_ARG, "id_all[%lld] = %g is not a grain id in 1..%lld", (long long)j, g, (long long)G);
-  }
   for (int64_t i = 0; i < M; i++) {
     double a = vox[5 * i + 3], b = vox[5 * i + 4];
     if (!(a == std::floor(a) && b == std::floor(b) && a >= 1.0 && b <= (double)n_id && b >= a - 1.0))
@@ -1031,90 +1020,58 @@ grs_status grs_forward_comp_compete(grs_ctx *c, const double *vox, int64_t M, co
   ENSURE(c, c->d_sub, sizeof(double) * 9 * (G > 0 ? G : 1));
   ENSURE(c, c->d_valid, sizeof(int32_t) * (G > 0 ? G : 1));
   ENSURE(c, c->d_p1, sizeof(double) * 11);
+  ENSURE(c, c->d_x, sizeof(double) * (n_id > 0 ? n_id : 1));
+  ENSURE(c, c->d_bad, sizeof(unsigned long long));
   if (G > 0) {
     HIPCHK(c, hipMemcpyAsync(c->d_eu.p, euler, sizeof(double) * 3 * G, hipMemcpyHostToDevice, c->st));
     HIPCHK(c, grs_launch_sub_from_euler(P<grs_dgeo>(c->d_geo), P<double>(c->d_eu), G, P<double>(c->d_sub),
                                         P<int32_t>(c->d_valid), c->st));
   }
   HIPCHK(c, hipMemcpyAsync(c->d_p1.p, p1, sizeof(double) * 11, hipMemcpyHostToDevice, c->st));
+  if (n_id > 0) HIPCHK(c, copy_up(c, c->d_x.p, id_all, sizeof(double) * n_id));
   const int64_t chunk = voxel_chunk(c);
-  std::vector<double> rows;
-  std::vector<int32_t> evox, eu;
   std::vector<int64_t> rs;
-  std::vector<int64_t> best;
-  std::vector<int32_t> hni;
-  std::vector<double> hC;
-  std::vector<float> hmed;
   for (int64_t b = 0; b < M; b += chunk) {
-    int64_t m = M - b;
-    if (m > chunk) m = chunk;
-    rows.resize(3 * m);
-    rs.assign(m + 1, 0);
-    evox.clear();
-    eu.clear();
-    for (int64_t k = 0; k < m; k++) {
-      const double *v = vox + 5 * (b + k);
-      rows[3 * k] = v[0];
-      rows[3 * k + 1] = v[1];
-      rows[3 * k + 2] = v[2];
-      int64_t lo = (int64_t)v[3], hi = (int64_t)v[4];
-      for (int64_t j = lo; j <= hi; j++) {
-        evox.push_back((int32_t)k);
-        eu.push_back((int32_t)id_all[j - 1] - 1);
-      }
-      rs[k + 1] = (int64_t)evox.size();
-    }
-    int64_t E = (int64_t)evox.size();
-    ENSURE(c, c->d_rows, sizeof(double) * 3 * m);
+    const int64_t m = M - b < chunk ? M - b : chunk;
+    /* evaluations before each row; the list itself, the winners and the
+     * output rows are formed on the device (the loops over the evaluations
+     * and the transfers of their lists and scores took 4 of the 24 ms of a call of
+     * 30,000 rows and 900,000 evaluations) */
+    rs.resize(m + 1);
+    rs[0] = 0;
+    for (int64_t k = 0; k < m; k++) rs[k + 1] = rs[k] + ((int64_t)vox[5 * (b + k) + 4] - (int64_t)vox[5 * (b + k) + 3] + 1);
+    const int64_t E = rs[m];
+    ENSURE(c, c->d_rows, sizeof(double) * 5 * m);
     ENSURE(c, c->d_pos, sizeof(double) * 3 * m);
     ENSURE(c, c->d_rowstart, sizeof(int64_t) * (m + 1));
-    ENSURE(c, c->d_best, sizeof(int64_t) * m);
+    ENSURE(c, c->d_y, sizeof(double) * 8 * m);
     ENSURE(c, c->d_evox, sizeof(int32_t) * (E > 0 ? E : 1));
     ENSURE(c, c->d_eu_idx, sizeof(int32_t) * (E > 0 ? E : 1));
     ENSURE(c, c->d_ns, sizeof(int32_t) * (E > 0 ? E : 1));
     ENSURE(c, c->d_ni, sizeof(int32_t) * (E > 0 ? E : 1));
     ENSURE(c, c->d_C, sizeof(double) * (E > 0 ? E : 1));
     ENSURE(c, c->d_med, sizeof(float) * (E > 0 ? E : 1));
-    HIPCHK(c, hipMemcpyAsync(c->d_rows.p, rows.data(), sizeof(double) * 3 * m, hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemcpyAsync(c->d_rowstart.p, rs.data(), sizeof(int64_t) * (m + 1), hipMemcpyHostToDevice, c->st));
-    if (E > 0) {
-      HIPCHK(c, hipMemcpyAsync(c->d_evox.p, evox.data(), sizeof(int32_t) * E, hipMemcpyHostToDevice, c->st));
-      HIPCHK(c, hipMemcpyAsync(c->d_eu_idx.p, eu.data(), sizeof(int32_t) * E, hipMemcpyHostToDevice, c->st));
+    HIPCHK(c, copy_up(c, c->d_rows.p, vox + 5 * b, sizeof(double) * 5 * m));
+    HIPCHK(c, copy_up(c, c->d_rowstart.p, rs.data(), sizeof(int64_t) * (m + 1)));
+    HIPCHK(c, grs_launch_compete_list(P<double>(c->d_rows), m, P<int64_t>(c->d_rowstart), P<double>(c->d_x), n_id, G,
+                                      P<double>(c->d_p1), P<double>(c->d_pos), P<int32_t>(c->d_evox),
+                                      P<int32_t>(c->d_eu_idx), P<unsigned long long>(c->d_bad), c->st));
+    if (b == 0) {
+      unsigned long long bad = 0;
+      HIPCHK(c, hipMemcpyAsync(&bad, c->d_bad.p, sizeof(bad), hipMemcpyDeviceToHost, c->st));
+      HIPCHK(c, hipStreamSynchronize(c->st));
+      if (bad != ~0ull)
+        return fail(c, GRS_ERR_ARG, "id_all[%lld] = %g is not a grain id in 1..%lld", (long long)bad, id_all[bad],
+                    (long long)G);
     }
-    HIPCHK(c, grs_launch_voxel_pos(P<double>(c->d_rows), m, 3, P<double>(c->d_p1), P<double>(c->d_pos), c->st));
     s = run_eval(c, GRS_MAP_PAIRS, E, m, P<int32_t>(c->d_evox), P<int32_t>(c->d_eu_idx), method,
                  P<int32_t>(c->d_ns), P<int32_t>(c->d_ni), P<double>(c->d_C), P<float>(c->d_med));
     if (s != GRS_OK) return s;
-    HIPCHK(c, grs_launch_compete_reduce(P<int64_t>(c->d_rowstart), m, P<int32_t>(c->d_ns), P<int32_t>(c->d_ni),
-                                        P<double>(c->d_C), P<float>(c->d_med), P<int64_t>(c->d_best), c->st));
-    best.resize(m);
-    hni.resize(E > 0 ? E : 1);
-    hC.resize(E > 0 ? E : 1);
-    hmed.resize(E > 0 ? E : 1);
-    HIPCHK(c, hipMemcpyAsync(best.data(), c->d_best.p, sizeof(int64_t) * m, hipMemcpyDeviceToHost, c->st));
-    if (E > 0) {
-      HIPCHK(c, hipMemcpyAsync(hni.data(), c->d_ni.p, sizeof(int32_t) * E, hipMemcpyDeviceToHost, c->st));
-      HIPCHK(c, hipMemcpyAsync(hC.data(), c->d_C.p, sizeof(double) * E, hipMemcpyDeviceToHost, c->st));
-      HIPCHK(c, hipMemcpyAsync(hmed.data(), c->d_med.p, sizeof(float) * E, hipMemcpyDeviceToHost, c->st));
-    }
+    HIPCHK(c, grs_launch_compete_out(P<int64_t>(c->d_rowstart), m, b, P<int32_t>(c->d_eu_idx), P<double>(c->d_eu),
+                                     P<int32_t>(c->d_ni), P<double>(c->d_C), P<float>(c->d_med), P<double>(c->d_y),
+                                     c->st));
+    HIPCHK(c, copy_down(c, out + 8 * b, c->d_y.p, sizeof(double) * 8 * m));
     HIPCHK(c, hipStreamSynchronize(c->st));
-    for (int64_t k = 0; k < m; k++) {
-      double *o = out + 8 * (b + k);
-      o[0] = (double)(b + k + 1);
-      int64_t j = best[k];
-      if (j < 0) {
-        for (int t = 1; t < 8; t++) o[t] = 0.0;
-        continue;
-      }
-      int32_t gi = eu[j];
-      o[1] = euler[3 * gi];
-      o[2] = euler[3 * gi + 1];
-      o[3] = euler[3 * gi + 2];
-      o[4] = (double)(gi + 1);
-      o[5] = hC[j];
-      o[6] = (double)hni[j];
-      o[7] = (double)hmed[j];
-    }
   }
   return GRS_OK;
 }
@@ -2653,22 +2610,21 @@ grs_status grs_find_neighbor_ors(grs_ctx *c, const int32_t *grain_id, int64_t nx
   HIPCHK(c, hipMemsetAsync(c->d_bad.p, 0, sizeof(uint32_t), c->st));
   HIPCHK(c, grs_launch_find_neighbors(P<int32_t>(c->c_gid), nx, ny, nz, P<int32_t>(c->c_vox), M, search_radius, nr_max,
                                       W, P<int32_t>(c->c_ids), P<int32_t>(c->c_nout), P<uint32_t>(c->d_bad), c->st));
-  std::vector<int32_t> nout((size_t)M), ids((size_t)M * nr_max);
+  /* packed one voxel after the other, 1-based [first last] (find_neighbor_ORs.m:26-29) */
+  ENSURE(c, c->c_off, sizeof(int64_t) * (size_t)(M + 1));
+  ENSURE(c, c->c_pack, sizeof(int32_t) * (size_t)M * nr_max);
+  ENSURE(c, c->c_ind, sizeof(int64_t) * 2 * (size_t)M);
+  HIPCHK(c, grs_launch_pack_ids(P<int32_t>(c->c_ids), P<int32_t>(c->c_nout), M, nr_max, P<int64_t>(c->c_off),
+                                P<int32_t>(c->c_pack), P<int64_t>(c->c_ind), c->st));
   uint32_t bad = 0;
+  int64_t count = 0;
   HIPCHK(c, hipMemcpyAsync(&bad, c->d_bad.p, sizeof(uint32_t), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(c, hipMemcpyAsync(nout.data(), c->c_nout.p, sizeof(int32_t) * M, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(c, hipMemcpyAsync(ids.data(), c->c_ids.p, sizeof(int32_t) * ids.size(), hipMemcpyDeviceToHost, c->st));
+  HIPCHK(c, hipMemcpyAsync(&count, P<int64_t>(c->c_off) + M, sizeof(count), hipMemcpyDeviceToHost, c->st));
   HIPCHK(c, hipStreamSynchronize(c->st));
   if (bad) return fail(c, GRS_ERR_STATE, "a search box grew to the whole volume without a positive id");
-  /* pack one voxel after the other, 1-based [first last] (find_neighbor_ORs.m:26-29) */
-  int64_t count = 0;
-  for (int64_t m = 0; m < M; m++) {
-    const int32_t n = nout[m];
-    for (int32_t k = 0; k < n; k++) id_all[count + k] = ids[(size_t)m * nr_max + k];
-    count += n;
-    ind[2 * m] = count - n + 1;
-    ind[2 * m + 1] = count;
-  }
+  HIPCHK(c, copy_down(c, id_all, c->c_pack.p, sizeof(int32_t) * (size_t)count));
+  HIPCHK(c, copy_down(c, ind, c->c_ind.p, sizeof(int64_t) * 2 * (size_t)M));
+  HIPCHK(c, hipStreamSynchronize(c->st));
   *n_total = count;
   return GRS_OK;
 }

@@ -140,8 +140,18 @@ hipError_t grs_launch_pack_hits(const uint32_t *d_keys, int64_t n, uint32_t hit_
 hipError_t grs_launch_pack_hits_tiled(const uint32_t *d_keys, int64_t nz, int64_t ny, int64_t nrot, uint32_t hit_key,
                                       int32_t has_hit, uint32_t *d_tbits, hipStream_t st);
 hipError_t grs_launch_plain(const grs_eval_args *a, int64_t n_threads, hipStream_t st);
-hipError_t grs_launch_compete_reduce(const int64_t *d_row_start, int64_t M, const int32_t *d_ns, const int32_t *d_ni,
-                                     const double *d_C, const float *d_med, int64_t *d_best, hipStream_t st);
+/* evaluation list of the compete rows: d_vox M x 5 rows [x y z start end],
+ * d_rs their M + 1 evaluation offsets, d_ids the candidate ids (1-based
+ * doubles); positions, evaluation voxels and orientations, and *d_bad the
+ * smallest index of an id outside 1..G (its evaluations use grain 1) */
+hipError_t grs_launch_compete_list(const double *d_vox, int64_t M, const int64_t *d_rs, const double *d_ids,
+                                   int64_t n_id, int64_t G, const double *d_p1, double *d_pos, int32_t *d_evox,
+                                   int32_t *d_eu, unsigned long long *d_bad, hipStream_t st);
+/* out rows [i phi1 PHI phi2 GrainId C Nr_intersect dis_median] of the first
+ * maximum of C; row0: rows before these */
+hipError_t grs_launch_compete_out(const int64_t *d_rs, int64_t M, int64_t row0, const int32_t *d_eu,
+                                  const double *d_euler, const int32_t *d_ni, const double *d_C, const float *d_med,
+                                  double *d_out, hipStream_t st);
 hipError_t grs_launch_math_eval(int fn, const double *d_x, double *d_y, int64_t n, hipStream_t st);
 hipError_t grs_launch_copy_u32(const uint32_t *d_src, uint32_t *d_dst, int64_t n, hipStream_t st);
 hipError_t grs_launch_check_keys(const uint32_t *d_keys, int64_t n, uint32_t *d_bad, hipStream_t st);
@@ -151,6 +161,9 @@ hipError_t grs_launch_check_keys(const uint32_t *d_keys, int64_t n, uint32_t *d_
 #define GRS_LS_MAX_GRID 64   /* values per (q1, q2, q3) grid */
 hipError_t grs_launch_local_sampling(const double *d_cen, const double *d_grids, const int32_t *d_gn, int64_t K,
                                      double *d_out, int64_t cap, int64_t *d_n, uint32_t *d_bad, hipStream_t st);
+/* d_off: M + 1 offsets, d_ind: M x 2 */
+hipError_t grs_launch_pack_ids(const int32_t *d_ids, const int32_t *d_nout, int64_t M, int32_t nr_max, int64_t *d_off,
+                               int32_t *d_id_all, int64_t *d_ind, hipStream_t st);
 hipError_t grs_launch_find_neighbors(const int32_t *d_gid, int64_t nx, int64_t ny, int64_t nz, const int32_t *d_vox,
                                      int64_t M, int32_t radius, int32_t nr_max, int32_t W, int32_t *d_ids,
                                      int32_t *d_nout, uint32_t *d_bad, hipStream_t st);

@@ -1717,22 +1717,60 @@ __global__ __launch_bounds__(256) void k_plain(grs_eval_args a, int64_t T) {
 /* ---------------------------------------------------------------------- */
 /* compete: first maximum of C per voxel row, NaN never wins              */
 
-__global__ void k_compete_reduce(const int64_t *row_start, int64_t M, const int32_t *ns, const int32_t *ni,
-                                 const double *C, const float *med, int64_t *best) {
-  int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_compete_ids(const double *ids, int64_t n_id, int64_t G,
+                                                     unsigned long long *bad) {
+  const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (j >= n_id) return;
+  const double g = ids[j];
+  if (!(g >= 1.0 && g <= (double)G && g == __builtin_floor(g))) atomicMin(bad, (unsigned long long)j);
+}
+
+/* one wave per row: its position and its evaluations */
+__global__ __launch_bounds__(256) void k_compete_list(const double *vox, int64_t M, const int64_t *rs,
+                                                      const double *ids, int64_t G, const double *p1, double *pos,
+                                                      int32_t *evox, int32_t *eu) {
+  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
   if (r >= M) return;
-  int64_t a = row_start[r], b = row_start[r + 1];
+  const double *v = vox + 5 * r;
+  if (lane == 0) grs_voxel_pos(v[0], v[1], v[2], p1, pos + 3 * r);
+  const int64_t e0 = rs[r], n = rs[r + 1] - e0, lo = (int64_t)v[3] - 1;
+  for (int64_t k = lane; k < n; k += 64) {
+    const double g = ids[lo + k];
+    evox[e0 + k] = (int32_t)r;
+    eu[e0 + k] = g >= 1.0 && g <= (double)G ? (int32_t)g - 1 : 0;
+  }
+}
+
+__global__ void k_compete_out(const int64_t *rs, int64_t M, int64_t row0, const int32_t *eu, const double *euler,
+                              const int32_t *ni, const double *C, const float *med, double *out) {
+  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= M) return;
+  const int64_t a = rs[r], b = rs[r + 1];
   int64_t bi = -1;
   double bc = 0.0;
   for (int64_t j = a; j < b; j++) {
-    double c = C[j];
+    const double c = C[j];
     if (c == c && (bi < 0 || c > bc)) {
       bi = j;
       bc = c;
     }
   }
   if (bi < 0 && b > a) bi = a;
-  best[r] = bi;
+  double *o = out + 8 * r;
+  o[0] = (double)(row0 + r + 1);
+  if (bi < 0) {
+    for (int t = 1; t < 8; t++) o[t] = 0.0;
+    return;
+  }
+  const int32_t g = eu[bi];
+  o[1] = euler[3 * (int64_t)g];
+  o[2] = euler[3 * (int64_t)g + 1];
+  o[3] = euler[3 * (int64_t)g + 2];
+  o[4] = (double)(g + 1);
+  o[5] = C[bi];
+  o[6] = (double)ni[bi];
+  o[7] = (double)med[bi];
 }
 
 /* ---------------------------------------------------------------------- */
@@ -1939,11 +1977,24 @@ hipError_t grs_launch_plain(const grs_eval_args *a, int64_t T, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t grs_launch_compete_reduce(const int64_t *d_row_start, int64_t M, const int32_t *d_ns, const int32_t *d_ni,
-                                     const double *d_C, const float *d_med, int64_t *d_best, hipStream_t st) {
+hipError_t grs_launch_compete_list(const double *d_vox, int64_t M, const int64_t *d_rs, const double *d_ids,
+                                   int64_t n_id, int64_t G, const double *d_p1, double *d_pos, int32_t *d_evox,
+                                   int32_t *d_eu, unsigned long long *d_bad, hipStream_t st) {
   if (M <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_compete_reduce, dim3(blocks_for(M, 256)), dim3(256), 0, st, d_row_start, M, d_ns, d_ni, d_C,
-                     d_med, d_best);
+  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, st, d_bad, (int64_t)1, ~0ull);
+  if (n_id > 0)
+    hipLaunchKernelGGL(k_compete_ids, dim3(blocks_for(n_id, 256)), dim3(256), 0, st, d_ids, n_id, G, d_bad);
+  hipLaunchKernelGGL(k_compete_list, dim3(blocks_for(M, 4)), dim3(256), 0, st, d_vox, M, d_rs, d_ids, G, d_p1, d_pos,
+                     d_evox, d_eu);
+  return hipGetLastError();
+}
+
+hipError_t grs_launch_compete_out(const int64_t *d_rs, int64_t M, int64_t row0, const int32_t *d_eu,
+                                  const double *d_euler, const int32_t *d_ni, const double *d_C, const float *d_med,
+                                  double *d_out, hipStream_t st) {
+  if (M <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_compete_out, dim3(blocks_for(M, 64)), dim3(64), 0, st, d_rs, M, row0, d_eu, d_euler, d_ni, d_C,
+                     d_med, d_out);
   return hipGetLastError();
 }
 

@@ -231,6 +231,31 @@ def test_grow_row_counts(engine, M):
         assert (got[mask == 1, 3] > 0).all()
 
 
+@pytest.mark.parametrize("counts", [[0], [1], [0, 63, 64, 65, 0, 200, 2]])
+def test_compete_row_lengths(engine, counts):
+    """Rows of no, one and more candidates than a wave lists at a time,
+    ranges that overlap and run backwards through id_all; an id that is no
+    grain is refused wherever it stands."""
+    s = scenes.make_scene(seed=43, ngrains=2, spread_mm=0.02, nrot=19)
+    engine.set_geometry(s.geo, s.hkl, s.rot)
+    engine.set_distance_stack(s.proj)
+    rng = np.random.default_rng(len(counts))
+    eu = rng.uniform([0, 0, 0], [360, 180, 360], (7, 3))
+    ids = rng.integers(1, 8, 220).astype(float)
+    rows = []
+    for k, n in enumerate(counts):
+        a = 220 - n - k
+        rows.append([14 + k, 20, 18, a, a + n - 1])
+    vox, p1 = np.array(rows, float), _p1()[:11]
+    got = engine.forward_comp_compete(vox, ids, eu, p1)
+    assert np.array_equal(_bits(got), _bits(oracle.compete(s.geo, s.stack, vox, ids, eu, s.rot, s.hkl, p1)))
+    for at, bad in ((0, 0.0), (117, 7.5), (219, 8.0), (219, np.nan)):
+        wrong = ids.copy()
+        wrong[at] = bad
+        with pytest.raises(_lib.GrsError, match=rf"id_all\[{at}\]"):
+            engine.forward_comp_compete(vox, wrong, eu, p1)
+
+
 @pytest.mark.parametrize("method", METHODS, ids=["fast", "plain"])
 def test_compete_parity(engine, method):
     s = scenes.make_scene(seed=43, ngrains=3, spread_mm=0.03)
