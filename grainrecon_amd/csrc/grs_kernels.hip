@@ -805,10 +805,9 @@ __device__ __noinline__ int exact_event(const grs_dgeo *g, const double *pos, co
  * reciprocal square root).  The arc angles come from one call of
  * arc_ends (errors below 5e-12 rad); the arcs are widened by 1e-6 rad and
  * the index bounds by 1e-6 steps.  The ranges of rotation indices [i0, i1]
- * land in six fixed slots (two arcs x three periods) and are disjoint, in
- * no particular order.  Returns the bit mask of the slots in use (at most
- * four) or -1 when more would be needed (the caller then scans every
- * event). */
+ * land in four fixed slots (two arcs x two periods) and are disjoint, in
+ * no particular order.  Returns the bit mask of the slots in use or -1 when
+ * more would be needed (the caller then scans every event). */
 __device__ __forceinline__ int om_ranges(const grs_dgeo *g, double g0, double g1, double gn, double lo_cb,
                                          double hi_cb, int32_t nrot, double idom, int32_t *i0, int32_t *i1) {
   const double twopi = 2.0 * GRS_PI, eps = 1e-6;
@@ -859,37 +858,31 @@ __device__ __forceinline__ int om_ranges(const grs_dgeo *g, double g0, double g1
     i1[0] = nrot - 1;
     return 1;
   }
-  /* slot 3 k + j: arc k in period m + j.  The arcs and their periods are
-   * more than 1e-5 steps apart, so the ranges are disjoint as they come;
-   * their order does not matter to the caller */
+  /* slot 2 k + j: arc k in its first period that ends at or after om0 and in
+   * the next.  The arcs and their periods are more than 1e-5 steps apart, so
+   * the ranges are disjoint as they come; their order does not matter to the
+   * caller.  The subtraction of 1e-9 keeps a period whose arc ends next to
+   * om0 (its range may be empty); an arc that would reach into a third period
+   * makes the caller scan every event. */
   uint32_t mask = 0;
 #pragma unroll
   for (int k = 0; k < 2; k++) {
     if (k >= niv) break;
-    /* the last period whose arc ends at or before om0.  The product rounds
-     * differently from the quotient only next to an integer, where m may be
-     * one less (that arc ends 2 pi below om0 and is skipped; the periods
-     * the scan can need, m..m+2 then, are still within the four steps) or
-     * one more (the period passed over ends about 2 pi below om0) */
-    const double m = __builtin_floor((g->om0 - hi[k]) * (1.0 / twopi));
+    const double m = __builtin_ceil((g->om0 - hi[k]) * (1.0 / twopi) - 1e-9);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < 2; j++) {
       const double L = lo[k] + twopi * (m + (double)j), U = hi[k] + twopi * (m + (double)j);
       double f0 = __builtin_ceil((L - g->om0) * idom - 1e-6);
       double f1 = __builtin_floor((U - g->om0) * idom + 1e-6);
       f0 = f0 > 0.0 ? f0 : 0.0;
       f1 = f1 < (double)(nrot - 1) ? f1 : (double)(nrot - 1);
       const bool ok = L <= g->om_last + 1e-9 && U >= g->om0 - 1e-9 && f0 <= f1;
-      if (j == 3) {
-        if (ok) return -1; /* a scan longer than the periods kept here */
-      } else {
-        i0[3 * k + j] = (int32_t)f0;
-        i1[3 * k + j] = (int32_t)f1;
-        mask |= (ok ? 1u : 0u) << (3 * k + j);
-      }
+      i0[2 * k + j] = (int32_t)f0;
+      i1[2 * k + j] = (int32_t)f1;
+      mask |= (ok ? 1u : 0u) << (2 * k + j);
     }
+    if (lo[k] + twopi * (m + 2.0) <= g->om_last + 1e-9) return -1;
   }
-  if (__popc(mask) > 4) return -1;
   return (int)mask;
 }
 
@@ -983,7 +976,7 @@ __device__ __forceinline__ void score_events(const grs_eval_args &a, const grs_d
   for (int hb = hlo; hb < hend; hb += 64) {
     const int h = hb + lane;
     int nr_h = 0; /* bit mask of the valid slots of ri0/ri1, or -1 */
-    int32_t ri0[6], ri1[6];
+    int32_t ri0[4], ri1[4];
     if (h < hend) {
       double gw[3];
       grs_Gw(sbuf, a.hkl + 3 * h, gw);
@@ -1035,7 +1028,7 @@ __device__ __forceinline__ void score_events(const grs_eval_args &a, const grs_d
       }
       uint32_t pos = R + (uint32_t)(incl - cnt);
 #pragma unroll
-      for (int k = 0; k < 6; k++) {
+      for (int k = 0; k < 4; k++) {
         if ((msk >> k) & 1u) {
           rstart[pos] = ((uint32_t)ri0[k] << 8) | (uint32_t)h;
           rcum[pos] = (uint32_t)(ri1[k] - ri0[k] + 1);
