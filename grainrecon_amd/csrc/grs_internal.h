@@ -65,6 +65,7 @@ typedef struct grs_eval_args {
   int32_t nrot;            /* rotation angles (must equal the geometry's); 0 turns the one-voxel beam table off */
   const uint32_t *hit_tbits; /* counts-only kernels: the hit mask in 32 x 32 pixel tiles (grs_tiled_bit) */
   int32_t bits_tiled;      /* counts-only kernels with count_keys = 0: 1 = test hit_tbits, 0 = hit_bits */
+  const double *beam;      /* V x nrot x GRS_BT beam table of the voxels (grs_launch_beam), or nullptr: terms computed per candidate */
   int32_t xcd_map;         /* 1 = consecutive waves of the evaluation order on one XCD (grid a multiple of 8 blocks) */
 } grs_eval_args;
 
@@ -95,11 +96,16 @@ __host__ __device__ inline uint32_t grs_tiled_bit(uint32_t om, uint32_t dy, uint
 #define GRS_KEY_MAX_EVENTS 23170
 /* largest k of the device top-k (sortrows + first rows) */
 #define GRS_TOPK_MAX 4096
+/* doubles per (voxel, omega) of the beam table: the omega_terms (10), cos, sin */
+#define GRS_BT 12
 /* doubles per voxel of the omega-solve bounds (k_voxel_bounds) */
 #define GRS_VB 14
 
 /* Launchers (return hipError_t). */
 /* d_vb: GRS_VB doubles per voxel, the omega-solve bounds */
+/* d_beam: V x nrot x GRS_BT */
+hipError_t grs_launch_beam(const grs_dgeo *d_g, const double *d_pos, int64_t V, const double *d_cs, int32_t nrot,
+                           double *d_beam, hipStream_t st);
 hipError_t grs_launch_voxel_bounds(const grs_dgeo *d_g, const double *d_pos, int64_t V, const double *d_cs,
                                    int32_t nrot, double *d_vb, hipStream_t st);
 hipError_t grs_launch_voxel_pos(const double *d_rows, int64_t M, int32_t row_stride, const double *d_p1,

@@ -47,7 +47,6 @@
 #define GRS_RING_DOUBLES (3 * GRS_QCAP * 4 / 8) /* three u32 rings per wave */
 #define GRS_RANGE_DOUBLES(H) (4 * (int64_t)(H) + 1) /* 8H + 2 u32: omega-solve ranges */
 #define GRS_REG_KEYS 16 /* keys per lane kept in registers for the median */
-#define GRS_BT 12       /* doubles per omega of the beam table: the omega_terms (10), cos, sin */
 
 /* LDS doubles of one wave's region of k_fast: the G table, the rings, the
  * omega-solve ranges, S*pos of the voxel (4) and S*U*B (9) */
@@ -500,6 +499,41 @@ __global__ void k_sub_from_q(const grs_dgeo *g, const double *q, int64_t N, doub
   if (ok) grs_SUB(g, U, SUB + 9 * i);
   else
     for (int k = 0; k < 9; k++) SUB[9 * i + k] = 0.0;
+}
+
+/* One row of the beam table: every term of the spot construction that depends
+ * on (voxel, omega) alone. */
+__device__ __forceinline__ void beam_row(const grs_dgeo *g, const double *P, double c, double s, double *r) {
+  om_terms w;
+  omega_terms(g, P, c, s, &w);
+  r[0] = w.u0;
+  r[1] = w.u1;
+  r[2] = w.u2;
+  r[3] = w.k0;
+  r[4] = w.d1;
+  r[5] = w.d2;
+  r[6] = w.L2;
+  r[7] = w.tnum;
+  r[8] = w.ov1;
+  r[9] = w.ov2;
+  r[10] = c;
+  r[11] = s;
+}
+
+/* The beam table of V voxels in device memory, for launches whose voxels have
+ * many evaluations each: k_fast then loads the terms of a candidate (six
+ * 16-byte loads from L1/L2) instead of 45 operations with two reciprocals.
+ * 343 x 7.9 samples of 1,024 voxels: 27.6 -> 26.7 ms; 24 orientation fits:
+ * 1.47 -> 1.39 ms. */
+__global__ __launch_bounds__(256) void k_beam(const grs_dgeo *g, const double *pos, int64_t V, const double *cs,
+                                              int32_t nrot, double *beam) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t >= V * nrot) return;
+  const int64_t v = t / nrot;
+  const int32_t om = (int32_t)(t - v * nrot);
+  double P[3];
+  voxel_P(g, pos + 3 * v, P);
+  beam_row(g, P, cs[2 * om], cs[2 * om + 1], beam + GRS_BT * t);
 }
 
 /* What a one-voxel launch needs beside the stack, in one kernel: block 0
@@ -1319,21 +1353,7 @@ __global__ __launch_bounds__(64 * GRS_WPB, GRS_FAST_MIN_WAVES) void k_fast(grs_e
     double P[3];
     voxel_P(g, a.pos, P);
     for (int32_t om = (int32_t)threadIdx.x; om < g->nrot; om += (int32_t)blockDim.x) {
-      om_terms w;
-      omega_terms(g, P, a.cs[2 * om], a.cs[2 * om + 1], &w);
-      double *r = bt + GRS_BT * om;
-      r[0] = w.u0;
-      r[1] = w.u1;
-      r[2] = w.u2;
-      r[3] = w.k0;
-      r[4] = w.d1;
-      r[5] = w.d2;
-      r[6] = w.L2;
-      r[7] = w.tnum;
-      r[8] = w.ov1;
-      r[9] = w.ov2;
-      r[10] = a.cs[2 * om];
-      r[11] = a.cs[2 * om + 1];
+      beam_row(g, P, a.cs[2 * om], a.cs[2 * om + 1], bt + GRS_BT * om);
     }
     __syncthreads();
     btab = bt;
@@ -1375,6 +1395,8 @@ __global__ __launch_bounds__(64 * GRS_WPB, GRS_FAST_MIN_WAVES) void k_fast(grs_e
       if (threadIdx.x == 0) team[0] = team[1] = team[2] = 0;
       __syncthreads();
     }
+    if (MAP == GRS_MAP_CSR || MAP == GRS_MAP_GRID)
+      btab = a.beam ? a.beam + (int64_t)GRS_BT * a.nrot * vi : nullptr;
     score_events<MEDIAN, AUDIT, TEAM>(a, g, b1thr, btab, L, sub, vi, hlo, hend, wlist, &team[2], &ns, &ni);
     if (TEAM) {
       if (lane == 0) {
@@ -1501,7 +1523,7 @@ __global__ __launch_bounds__(64 * GRS_FIT_TEAM * GRS_FIT_PTS, GRS_FAST_MIN_WAVES
     if (p < np && grs_U_from_q(xs[p][0], xs[p][1], xs[p][2], U)) {
       grs_SUB(a.g, U, sub);
       int32_t ns, ni;
-      score_events<false, false, true>(a, &sg, b1thr, nullptr, L, sub, m, hlo, hend, nullptr, nullptr, &ns, &ni);
+      score_events<false, false, true>(a, &sg, b1thr, a.beam + (int64_t)GRS_BT * a.nrot * m, L, sub, m, hlo, hend, nullptr, nullptr, &ns, &ni);
       if (lane == 0) {
         atomicAdd(&cnt[p][0], ns);
         atomicAdd(&cnt[p][1], ni);
@@ -1781,6 +1803,13 @@ hipError_t grs_launch_voxel_pos(const double *d_rows, int64_t M, int32_t stride,
                                 hipStream_t st) {
   if (M <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_voxel_pos, dim3(blocks_for(M, 256)), dim3(256), 0, st, d_rows, M, stride, d_p1, d_pos);
+  return hipGetLastError();
+}
+
+hipError_t grs_launch_beam(const grs_dgeo *d_g, const double *d_pos, int64_t V, const double *d_cs, int32_t nrot,
+                           double *d_beam, hipStream_t st) {
+  if (V <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_beam, dim3(blocks_for(V * nrot, 256)), dim3(256), 0, st, d_g, d_pos, V, d_cs, nrot, d_beam);
   return hipGetLastError();
 }
 

@@ -231,6 +231,33 @@ def test_grow_row_counts(engine, M):
         assert (got[mask == 1, 3] > 0).all()
 
 
+@pytest.mark.parametrize("nr, k", [(0, 255), (0, 256), (0, 257), (5, 1), (6, 1)])
+def test_compete_csr_with_and_without_the_beam_table(engine, nr, k):
+    """Evaluations per voxel around the rule for the voxels' beam table
+    (samples x candidates: 255, 256, 257, 216, 343), on uniform rotation
+    angles and on others: winners and counts equal the scores of the whole
+    lists."""
+    s = scenes.make_scene(seed=45, ngrains=2, spread_mm=0.02, nrot=13)
+    rng = np.random.default_rng(nr * 1000 + k)
+    g = 0.003
+    grid = np.arange(nr + 1) * g
+    for rot in (s.rot, np.sort(rng.uniform(0, 360, s.rot.size))):
+        engine.set_geometry(s.geo, s.hkl, rot)
+        engine.set_distance_stack(s.proj)
+        pos = np.array([s.centers[0], s.centers[1], s.centers[0] + 0.01])
+        cand = np.concatenate([np.concatenate([s.q[:1], scenes.random_quats(rng, k - 1)]) if k > 1 else s.q[:1] for _ in pos])
+        best, bq, ns, ni, C, med = engine.compete_csr(pos, np.arange(4) * k, cand, nr, g)
+        for r in range(3):
+            rows = []
+            for c in cand[r * k:(r + 1) * k]:
+                a, b, d = np.meshgrid(*[(c[1 + i] - (g * nr) / 2) + grid for i in range(3)], indexing="ij")
+                rows.append(np.stack([np.zeros(a.size), a.ravel(), b.ravel(), d.ravel()], 1))
+            rns, rni, rC, rmed = engine.forward_comp(pos[r], np.concatenate(rows), _lib.METHOD_PLAIN)
+            j = int(np.nanargmax(rC))
+            assert best[r] == j and ns[r] == rns[j] and ni[r] == rni[j]
+            assert _bits(C[r:r + 1])[0] == _bits(rC[j:j + 1])[0] and med[r] == rmed[j]
+
+
 @pytest.mark.parametrize("counts", [[0], [1], [0, 63, 64, 65, 0, 200, 2]])
 def test_compete_row_lengths(engine, counts):
     """Rows of no, one and more candidates than a wave lists at a time,
