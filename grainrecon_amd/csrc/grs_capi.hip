@@ -91,7 +91,7 @@ struct grs_ctx {
       x_bad;
   std::map<std::vector<uint64_t>, hipGraphExec_t> gi_cache;
   /* experimental spots per projection (CSR) for the spot pairing */
-  DevBuf p_fptr, p_fsp, p_flag, p_sid, p_lam, p_dyz, p_dis, p_off, p_cnt, p_rowptr, p_rows;
+  DevBuf p_hits, p_fptr, p_fsp, p_flag, p_sid, p_lam, p_dyz, p_dis, p_off, p_cnt, p_rowptr, p_rows;
   int64_t p_nframes = -1, p_n = 0, p_maxframe = 0;
   /* reconstruction volumes (completeness, mask, median distance, Nr_intersect)
    * and the region-growth buffers */
@@ -413,7 +413,7 @@ void grs_destroy(grs_ctx *c) {
                     &c->r_rows, &c->r_counts, &c->r_acc_lin, &c->r_acc_C, &c->t_pos, &c->t_proj, &c->t_units,
                     &c->t_fam, &c->t_dposs, &c->t_glen, &c->t_scratch, &c->t_out, &c->m_rows, &c->m_rptr,
                     &c->m_nm, &c->t_skey, &c->t_su, &c->t_bst, &c->t_slen, &c->t_sorig, &c->v_lin,
-                    &c->v_out, &c->f_in, &c->f_cnt, &c->m_cs, &c->m_dis, &c->t_band, &c->d_beam, &c->c_off, &c->c_pack, &c->c_ind};
+                    &c->v_out, &c->f_in, &c->f_cnt, &c->m_cs, &c->m_dis, &c->t_band, &c->d_beam, &c->p_hits, &c->c_off, &c->c_pack, &c->c_ind};
   if (c->g_exec) hipGraphExecDestroy(c->g_exec);
   for (auto &kv : c->gi_cache) hipGraphExecDestroy(kv.second);
   for (hipEvent_t e : c->tev) hipEventDestroy(e);
@@ -2114,13 +2114,16 @@ grs_status grs_pair_spots(grs_ctx *c, const double *pos, const double *U, int64_
     ENSURE(c, c->p_dyz, sizeof(int32_t) * 2 * me);
     ENSURE(c, c->p_dis, sizeof(float) * me);
     ENSURE(c, c->p_off, sizeof(int32_t) * me);
+    ENSURE(c, c->p_hits, sizeof(int64_t) * me);
+    ENSURE(c, c->d_bad, sizeof(uint32_t));
     ENSURE(c, c->p_cnt, sizeof(int64_t) * (m + 1));
     ENSURE(c, c->p_rowptr, sizeof(int64_t) * (m + 1));
     HIPCHK(c, grs_launch_pair_events(P<grs_dgeo>(c->d_geo), P<double>(c->d_hkl), P<double>(c->d_cs),
                                      P<uint32_t>(c->d_keys), P<double>(c->d_pos) + 3 * m0,
                                      P<double>(c->d_sub) + 9 * m0, m, E, P<int64_t>(c->p_fptr), P<double>(c->p_fsp),
                                      P<int32_t>(c->p_flag), P<int64_t>(c->p_sid), P<double>(c->p_lam),
-                                     P<int32_t>(c->p_dyz), P<float>(c->p_dis), c->st));
+                                     P<int32_t>(c->p_dyz), P<float>(c->p_dis), P<int64_t>(c->p_hits),
+                                     P<uint32_t>(c->d_bad), c->st));
     HIPCHK(c, grs_launch_pair_scan(P<int32_t>(c->p_flag), m, E, P<int32_t>(c->p_off), P<int64_t>(c->p_cnt), c->st));
     cnt.resize((size_t)m);
     HIPCHK(c, hipMemcpyAsync(cnt.data(), c->p_cnt.p, sizeof(int64_t) * m, hipMemcpyDeviceToHost, c->st));

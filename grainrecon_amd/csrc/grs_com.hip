@@ -179,13 +179,9 @@ __global__ __launch_bounds__(COM_THREADS) void k_com_nm(const grs_dgeo *g, const
     }
     __syncthreads();
     if (t < 64) { /* the first wave steps the method */
-      nm_lanes L{nm, t, t < nm->n};
-      const bool refl = nm->st == grs_nm::REFLECT;
-      L.feed(fs);
-      if (refl) {
-        const int q = nm->st == grs_nm::EXPAND ? 1 : nm->st == grs_nm::CONTRACT_OUT ? 2 : nm->st == grs_nm::CONTRACT_IN ? 3 : 0;
-        if (q > 0) L.feed(fs + q);
-      }
+      nm_lanes<6> L(nm, t);
+      L.step(fs);
+      L.store();
     }
     __syncthreads();
   }

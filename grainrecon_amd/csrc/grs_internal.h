@@ -231,7 +231,8 @@ hipError_t grs_launch_seed_out(const unsigned long long *d_topkey, const int32_t
 hipError_t grs_launch_pair_events(const grs_dgeo *d_g, const double *d_hkl, const double *d_cs,
                                   const uint32_t *d_keys, const double *d_pos, const double *d_SUB, int64_t M,
                                   int64_t E, const int64_t *d_fptr, const double *d_fsp, int32_t *d_flag,
-                                  int64_t *d_sid, double *d_lam, int32_t *d_dyz, float *d_dis, hipStream_t st);
+                                  int64_t *d_sid, double *d_lam, int32_t *d_dyz, float *d_dis, int64_t *d_hits,
+                                  uint32_t *d_nhits, hipStream_t st);
 hipError_t grs_launch_pair_scan(const int32_t *d_flag, int64_t M, int64_t E, int32_t *d_off, int64_t *d_count,
                                 hipStream_t st);
 hipError_t grs_launch_pair_rows(const grs_dgeo *d_g, const double *d_hkl, const double *d_rot, const double *d_pos,

@@ -1467,6 +1467,7 @@ __global__ __launch_bounds__(64 * GRS_FIT_TEAM * GRS_FIT_PTS, GRS_FAST_MIN_WAVES
   __shared__ grs_dgeo sg;
   __shared__ double b1thr[12];
   __shared__ int32_t cnt[GRS_FIT_PTS][2];
+  __shared__ double fs[GRS_FIT_PTS];
   __shared__ int npts;
   grs_nm *nm = reinterpret_cast<grs_nm *>(nm_buf);
   const int t = threadIdx.x, lane = t & 63, wib = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -1532,16 +1533,11 @@ __global__ __launch_bounds__(64 * GRS_FIT_TEAM * GRS_FIT_PTS, GRS_FAST_MIN_WAVES
     __syncthreads();
     if (wib == 0) {
       /* fit_OR_fun_local.m:98; 0/0 (no event, or |q_vec| > 1) is NaN */
-      double f[GRS_FIT_PTS];
-#pragma unroll
-      for (int q = 0; q < GRS_FIT_PTS; q++) f[q] = 1.0 - (double)cnt[q][1] / (double)cnt[q][0];
-      nm_lanes S{nm, t, t < nm->n};
-      const bool refl = nm->st == grs_nm::REFLECT;
-      S.feed(f);
-      if (refl) {
-        const int q = nm->st == grs_nm::EXPAND ? 1 : nm->st == grs_nm::CONTRACT_OUT ? 2 : nm->st == grs_nm::CONTRACT_IN ? 3 : 0;
-        if (q > 0) S.feed(&f[q]);
-      }
+      if (t < GRS_FIT_PTS) fs[t] = 1.0 - (double)cnt[t][1] / (double)cnt[t][0];
+      wave_sync();
+      nm_lanes<3> S(nm, t);
+      S.step(fs);
+      S.store();
     }
     __syncthreads();
   }

@@ -287,11 +287,18 @@ class Engine:
         med = np.zeros(M, np.float32)
         rp = np.zeros(M + 1, np.int64)
         i64p = ctypes.POINTER(ctypes.c_int64)
-        self._chk(self._lib.grs_pair_spots(self._h, _ptr(pos, _dp), _ptr(U, _dp), M, _ptr(ns, _ip), _ptr(ni, _ip),
-                                           _ptr(med, _fp), rp.ctypes.data_as(i64p), None, 0))
-        rows = np.zeros((max(int(rp[-1]), 1), 23))
-        self._chk(self._lib.grs_pair_spots(self._h, _ptr(pos, _dp), _ptr(U, _dp), M, _ptr(ns, _ip), _ptr(ni, _ip),
-                                           _ptr(med, _fp), rp.ctypes.data_as(i64p), _ptr(rows, _dp), rows.shape[0]))
+
+        def call(rows, cap):
+            return self._lib.grs_pair_spots(self._h, _ptr(pos, _dp), _ptr(U, _dp), M, _ptr(ns, _ip), _ptr(ni, _ip),
+                                            _ptr(med, _fp), rp.ctypes.data_as(i64p), rows, cap)
+
+        # a grain pairs a few hundred spots: one call with room for 1024 each,
+        # and where that is not enough one for the counts and one for the rows
+        rows = np.empty((max(1024 * M, 1), 23))
+        if call(_ptr(rows, _dp), rows.shape[0]) != L.GRS_OK:
+            self._chk(call(None, 0))
+            rows = np.zeros((max(int(rp[-1]), 1), 23))
+            self._chk(call(_ptr(rows, _dp), rows.shape[0]))
         return ns, ni, med, [rows[rp[m]:rp[m + 1]].copy() for m in range(M)]
 
     # -- grain centre-of-mass fit -----------------------------------------------------

@@ -78,3 +78,62 @@ def test_pair_spots_equals_oracle(engine, scene):
         np.testing.assert_array_equal(rows[m], rrows)
         total += rrows.shape[0]
     assert total > 50
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("per_frame, repeat", [(0, 1), (1, 1), (63, 1), (65, 1), (700, 1), (40, 40)])
+def test_pair_spots_list_lengths(engine, scene, per_frame, repeat):
+    """Projections without spots, with less and more than a wave reads at a
+    time, spots repeated (the first one counts) or without a position (NaN),
+    every selected event a hit; reflections repeated."""
+    s = scene
+    hkl = np.concatenate([s.hkl[:min(len(s.hkl), 240 // repeat)]] * repeat) if repeat > 1 else s.hkl
+    engine.set_geometry(s.geo, hkl, s.rot)
+    proj = np.zeros_like(s.proj)
+    engine.set_distance_stack(proj)
+    import oracle
+
+    stack = oracle.Stack(proj)
+    rng = np.random.default_rng(per_frame + repeat)
+    _, _, _, ev = oracle.forward_comp(s.geo, stack, s.U[0], s.centers[0], s.rot, hkl, events=True)
+    frames = [[] for _ in range(s.rot.size)]
+    for e in ev:
+        if per_frame and len(frames[int(e[0])]) < per_frame:
+            frames[int(e[0])].append([e[2] + rng.uniform(-3, 3), e[3] + rng.uniform(-3, 3), rng.uniform(1, 300)])
+    det = float(s.geo.detysize)
+    full = []
+    for f in frames:
+        f = np.array(f, float).reshape(-1, 3)
+        f = np.concatenate([f, f[:per_frame // 3]])[:per_frame]
+        more = np.column_stack([rng.uniform(1, det, (per_frame - len(f), 2)), np.full(per_frame - len(f), 100.0)])
+        f = np.concatenate([f, more])
+        if len(f) > 2:
+            f[1, 0] = np.nan
+        full.append(f)
+    engine.set_frame_spots(full)
+    ns, ni, med, rows = engine.pair_spots(s.centers[:1], s.U[0][None])
+    rns, rni, rmed, rrows = pair_spots(s.geo, stack, s.U[0], s.centers[0], s.rot, hkl, full)
+    assert (ns[0], ni[0], med[0]) == (rns, rni, np.float32(rmed))
+    np.testing.assert_array_equal(rows[0], rrows.reshape(-1, 23))
+
+
+@pytest.mark.gpu
+def test_pair_spots_of_more_rows_than_the_first_call_holds(engine):
+    """A dense set of events (181 angles, 240 reflections, every selected
+    event a hit with a spot of its own) pairs more than 1024 spots."""
+    import oracle
+
+    s = scenes.make_scene(seed=84, ngrains=1, spread_mm=0.02, nrot=181)
+    hkl = np.concatenate([s.hkl, s.hkl, s.hkl])[:240]
+    proj = np.zeros_like(s.proj)
+    engine.set_geometry(s.geo, hkl, s.rot)
+    engine.set_distance_stack(proj)
+    stack = oracle.Stack(proj)
+    _, _, _, ev = oracle.forward_comp(s.geo, stack, s.U[0], s.centers[0], s.rot, hkl, events=True)
+    assert len(ev) > 1024
+    frames = _frames_at_events(s, ev)
+    engine.set_frame_spots(frames)
+    ns, ni, med, rows = engine.pair_spots(s.centers[:1], s.U[0][None])
+    rns, rni, rmed, rrows = pair_spots(s.geo, stack, s.U[0], s.centers[0], s.rot, hkl, frames)
+    assert rows[0].shape[0] == len(ev) == ns[0]
+    np.testing.assert_array_equal(rows[0], rrows)
