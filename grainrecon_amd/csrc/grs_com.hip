@@ -66,7 +66,7 @@ __device__ __forceinline__ double com_pair_dist(const grs_dgeo *g, const double 
   const double g2 = __builtin_fma(gw[0], gw[0], __builtin_fma(gw[1], gw[1], gw[2] * gw[2]));
   const double cb = __builtin_fma(w.u0, G0, __builtin_fma(w.u1, G1, w.u2 * G2)) * fast_rsq(g2);
   double ry, rz, ky, kz;
-  if (__builtin_fabs(cb) <= 0.99 && b1_spot(g, w, G1, G2, cb, g2, thr, &ry, &rz) && __builtin_fabs(ry) <= 1e5 &&
+  if (__builtin_fabs(cb) <= 0.99 && b1_spot<true>(g, w, G1, G2, cb, g2, thr, &ry, &rz) && __builtin_fabs(ry) <= 1e5 &&
       __builtin_fabs(rz) <= 1e5 && com_round(ry, &ky) && com_round(rz, &kz)) {
     GRS_NO_CONTRACT
     const double ey = ky - r[17], ez = kz - r[18];

@@ -372,7 +372,7 @@ __global__ __launch_bounds__(256, 4) void k_gt_score(const grs_dgeo *g, const do
           const double gn2 = (gw[0] * gw[0] + gw[1] * gw[1]) + gw[2] * gw[2];
           const double t5[5] = {gw[0], gw[1], gw[2], fast_rsq(gn2), gn2};
           b1_out bo;
-          int st = b1_classify(g, P[0], P[1], nullptr, bt, t5, thr, &bo);
+          int st = b1_classify<false>(g, P[0], P[1], nullptr, bt, t5, thr, &bo);
           if (st == 2) {
             grs_vw v;
             gt_vw(P, &v);

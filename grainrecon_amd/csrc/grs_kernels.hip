@@ -1175,7 +1175,7 @@ __device__ __forceinline__ void score_events(const grs_eval_args &a, const grs_d
       o.win = 0;
       const double *brow = btab ? btab + GRS_BT * om : nullptr;
       const double cc = brow ? brow[10] : a.cs[2 * om], ss = brow ? brow[11] : a.cs[2 * om + 1];
-      st = b1_classify(g, cc, ss, Pw, brow, t, b1thr, &o);
+      st = b1_classify<true>(g, cc, ss, Pw, brow, t, b1thr, &o);
       if (st == 1)
         idx = tiled ? grs_tiled_bit((uint32_t)om, (uint32_t)o.dy, (uint32_t)o.dz, ntz, nty)
                     : (uint32_t)(o.dz - 1) + (uint32_t)(o.dy - 1) * nz32 + (uint32_t)om * nzny32;

@@ -53,7 +53,7 @@ __global__ __launch_bounds__(256) void k_pair_events(const grs_dgeo *g, const do
   const double g2 = (gw[0] * gw[0] + gw[1] * gw[1]) + gw[2] * gw[2];
   const double t5[5] = {gw[0], gw[1], gw[2], fast_rsq(g2), g2};
   b1_out bo;
-  const int st = b1_classify(g, c, s, P, nullptr, t5, thr, &bo);
+  const int st = b1_classify<true>(g, c, s, P, nullptr, t5, thr, &bo);
   if (st == 0) return;
   grs_vw v;
   double Gt[3], Glen, beta;
