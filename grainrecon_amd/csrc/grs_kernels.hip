@@ -1075,7 +1075,10 @@ __device__ __forceinline__ void score_events(const grs_eval_args &a, const grs_d
   wave_sync();
   uint32_t total = 0;
   if (solve && !overflow) {
-    /* lengths -> exclusive prefix sums */
+    /* lengths -> exclusive prefix sums; the first candidate of each range
+     * sets its bit in ring1, a bitmap of the first GRS_QCAP * 32 candidates
+     * (unused otherwise on this path) */
+    for (int k = lane; k < GRS_QCAP; k += 64) ring1[k] = 0u;
     for (uint32_t cb = 0; cb < R; cb += 64) {
       const uint32_t r = cb + lane;
       const uint32_t len = r < R ? rcum[r] : 0u;
@@ -1085,7 +1088,11 @@ __device__ __forceinline__ void score_events(const grs_eval_args &a, const grs_d
         if (lane >= off) incl += v;
       }
       wave_sync();
-      if (r < R) rcum[r] = total + incl - len;
+      const uint32_t first = total + incl - len;
+      if (r < R) {
+        rcum[r] = first;
+        if (first < GRS_QCAP * 32u) atomicOr(&ring1[first >> 5], 1u << (first & 31u));
+      }
       total += (uint32_t)__shfl((int)incl, 63, 64);
       wave_sync();
     }
@@ -1224,26 +1231,30 @@ __device__ __forceinline__ void score_events(const grs_eval_args &a, const grs_d
   if (solve && !overflow) {
     /* candidates of the omega solve, 64 per step, straight to phase B1.
      * Ranges are non-empty and rcum is their exclusive prefix, so the range
-     * of candidate base + l is rb plus the number of later ranges that
-     * start at or before base + l, where rb is the last range starting
-     * before base (0 at base 0).  Those starts lie in the next 64 ranges;
-     * each marks its position in ring1 (unused on this path) and a ballot
-     * turns the marks into a bit mask. */
-    uint32_t rb = 0;
+     * of a candidate is the number of set bits up to its own in the bitmap
+     * of first candidates, less one.  (Marks written and read back on every
+     * step: 27.0 instead of 26.7 ms for 1,024 voxels x 343 x 7.9 samples; the
+     * range looked up one step ahead: 27.0.) */
+    uint32_t rb = 0xFFFFFFFFu; /* set bits before base, less one */
     for (uint32_t base = 0; base < total; base += 64) {
+      const uint32_t at = base & (GRS_QCAP * 32u - 1u);
+      if (base > 0 && at == 0) {
+        /* the next GRS_QCAP * 32 candidates */
+        wave_sync();
+        for (int k = lane; k < GRS_QCAP; k += 64) ring1[k] = 0u;
+        wave_sync();
+        for (uint32_t r = lane; r < R; r += 64) {
+          const uint32_t p = rcum[r] - base;
+          if (p < GRS_QCAP * 32u) atomicOr(&ring1[p >> 5], 1u << (p & 31u));
+        }
+        wave_sync();
+      }
       const uint32_t idx = base + (uint32_t)lane;
       const bool valid = idx < total;
-      ring1[lane] = 0u;
-      wave_sync();
-      const uint32_t rn = rb + 1u + (uint32_t)lane;
-      if (rn < R) {
-        const uint32_t p = rcum[rn] - base;
-        if (p < 64u) ring1[p] = 1u;
-      }
-      wave_sync();
-      const uint64_t starts = __ballot(ring1[lane] != 0u);
-      const uint64_t upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
-      const uint32_t r = rb + (uint32_t)__popcll(starts & upto);
+      const uint32_t m0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)ring1[at >> 5]);
+      const uint32_t m1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)ring1[(at >> 5) + 1]);
+      const uint64_t starts = ((uint64_t)m1 << 32) | m0;
+      const uint32_t r = rb + lane_prefix(starts) + (uint32_t)((starts >> lane) & 1ull);
       rb += (uint32_t)__popcll(starts);
       uint32_t ev = 0;
       if (valid) {

@@ -107,7 +107,7 @@ __device__ __forceinline__ void omega_terms(const grs_dgeo *g, const double *P, 
  * the exact pipeline.  STRAIGHT: no branches at the guards, which nearly
  * always hold; a branch at each keeps the loads and products behind it from
  * starting early (without them 1,024 voxels x 343 x 7.9 samples: 26.7 ->
- * 26.0 ms, 10,000 orientations of a voxel: 2.82 -> 2.73 ms, 24 fits: 1.39 ->
+ * 26.0 ms, 262,144 orientations of a voxel: 2.82 -> 2.73 ms, 24 fits: 1.39 ->
  * 1.27 ms).  It holds more registers, which costs a kernel that spills them
  * (k_gt_score: 3.4 -> 4.3 ms). */
 template <bool STRAIGHT>

@@ -209,6 +209,28 @@ def test_small_launches_share_evaluations(engine, H):
                 assert np.array_equal(_bits(x), _bits(y[:n])), n
 
 
+@pytest.mark.parametrize("nrot", [1701, 1851, 2001, 3841])
+def test_many_candidates_per_evaluation(engine, nrot):
+    """Rotation counts whose evaluations have about 3,800, 4,100, 4,500 and
+    8,600 selected events, so that the candidates of a wave end before, near
+    and after one or two fills of its bitmap of first candidates (4,096
+    bits): one wave and four waves per evaluation equal the plain kernel, and
+    the oracle on three orientations."""
+    s = scenes.make_scene(seed=51, det=64, pixel_mm=6.72e-3 * 16, nrot=7)
+    rng = np.random.default_rng(nrot)
+    rot = np.linspace(0.0, 360.0, nrot)
+    proj = rng.integers(0, 40, (64, 64, nrot)).astype(np.float32)
+    engine.set_geometry(s.geo, s.hkl, rot)
+    engine.set_distance_stack(proj)
+    q = np.concatenate([s.q, scenes.random_quats(rng, 2597)])
+    ref = engine.forward_comp(s.centers[0], q, _lib.METHOD_PLAIN)
+    for n in (3, 2600):
+        for x, y in zip(engine.forward_comp(s.centers[0], q[:n]), ref):
+            assert np.array_equal(_bits(x), _bits(y[:n])), n
+    want = oracle.or_space_comp(s.geo, oracle.Stack(proj), s.centers[0], q[:3], rot, s.hkl)
+    assert np.array_equal(ref[0][:3], want[:, 0]) and np.array_equal(_bits(ref[2][:3]), _bits(want[:, 2].copy()))
+
+
 @pytest.mark.parametrize("M", [1, 255, 257, 1023, 1024, 16384, 16385, 32768, 262145])
 def test_grow_row_counts(engine, M):
     """Row counts around the blocks of the row listing and around the rules
