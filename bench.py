@@ -53,7 +53,7 @@ def flop_per_eval(nrot: int, H: int) -> int:
 # kernel source (grs_kernels.hip; + - * / sqrt rsq rcp acos atan2 = 1 each, a
 # fused multiply-add = 2; comparisons and integer work are not counted):
 F_SETUP = 136    # per evaluation: q0, U(q), S*U*B (k_sub_from_q)
-F_SOLVE = 182    # per (evaluation, reflection): G, |G|, thresholds, the cos(beta) window with the detector
+F_SOLVE = 150    # per (evaluation, reflection): G, |G|, thresholds, the cos(beta) window with the detector
                  # rows and columns bound, om_ranges (a refined rcp/rsq counts its Newton step: 4 and 6)
 F_CAND = 20      # per candidate event: Gt, cos(beta), lambda and the window tests (b1_classify; the
                  # thresholds come precomputed per block)
@@ -69,8 +69,8 @@ def pruned_flop_per_eval(H, cand, in_window, exact):
     return F_SETUP + F_SOLVE * H + F_CAND * cand + F_SPOT * in_window + F_EXACT * exact
 
 
-# the translation unit of k_fast: its counters change only with these files
-KFAST_SOURCES = ("grs_geom.h", "grs_internal.h", "grs_kernels.hip", "grs_math.h")
+# the sources of k_fast's translation unit that its counters change with
+KFAST_SOURCES = ("grs_geom.h", "grs_internal.h", "grs_kernels.hip", "grs_math.h", "grs_nm_lanes.h", "grs_resolve.h")
 
 
 def kernel_sources_sha():

@@ -5,8 +5,9 @@
  * Euler angles (degrees)]: for every paired spot of the grain the event of
  * its (hkl, omega) is forward-simulated from pos = [x1, x2-RotAxisOffset,
  * x3] and U = euler2u(x(4:6)) through the forward_comp.m statements
- * (grs_event_pixel), its pixel rounded, and the distance to the measured
- * centroid (columns 19:20 of the pair row) taken; ErrMean is the mean.
+ * (grs_event_pixel; its shortcut b1_spot where that rounds to the same
+ * pixel), its pixel rounded, and the distance to the measured centroid
+ * (columns 19:20 of the pair row) taken; ErrMean is the mean.
  * k_com_nm runs fminsearchbnd's Nelder-Mead for each grain inside the
  * kernel (one block per grain, its first wave stepping the method with one
  * lane per coordinate), so a fit costs no host round trip per simplex step.
@@ -82,7 +83,7 @@ __device__ __forceinline__ double com_pair_dist(const grs_dgeo *g, const double 
 #define COM_LDS_DIST 6144
 
 /* One block per fit m: the first wave steps the Nelder-Mead state machine
- * (started on the host) in LDS (nm_lanes); for the requested points - a
+ * (started on the host) in registers (nm_lanes); for the requested points - a
  * reflection together with the three points its value can lead to
  * (grs_nm::follow_ups), so that an iteration is one round - the point
  * coordinates and the six cosines and sines of each point's angles are
@@ -91,9 +92,9 @@ __device__ __forceinline__ double com_pair_dist(const grs_dgeo *g, const double 
  * p's distances in pair order, so ErrMean is the sequential sum over the
  * count.  Bound: the chain of one round (trigonometry, distances, the
  * sequential sum of a few hundred values, the simplex step).  Three grains of
- * about 400 pairs: 1.6 ms for the launch; with the exact pipeline for every
- * distance, the distances in device memory and a round per requested point
- * it took 2.4 ms.  The state machine ends after at most max_iter iterations,
+ * about 400 pairs: 1.2 ms for the launch; 1.6 with the simplex stepped in
+ * LDS; 2.4 with also the exact pipeline for every distance, the distances
+ * in device memory and a round per requested point.  The state machine ends after at most max_iter iterations,
  * so every block exits. */
 __global__ __launch_bounds__(COM_THREADS) void k_com_nm(const grs_dgeo *g, const double *rows, const int64_t *rptr,
                                                         const double *cs, double *dis, grs_nm *nms) {

@@ -7,8 +7,11 @@
  * (forward_comp.m:69-72) and reduce the integer counts and the median
  * distance (forward_comp.m:67, 86-90).
  *
- * k_fast  -- one 64-wide wavefront per evaluation.
- *   phase A: lanes walk the flattened (omega, hkl) event space 64 events at a
+ * k_fast  -- one 64-wide wavefront per evaluation (two or four share one in
+ *            small launches).
+ *   solve:   with uniform rotation angles each reflection's candidate ranges
+ *            of omega are solved for (om_ranges) and go straight to phase B1.
+ *   phase A: otherwise lanes walk the flattened (omega, hkl) event space 64 events at a
  *            time and apply a conservative Bragg/wavelength filter that only
  *            needs 4 multiplies and 3 FMAs per event; it rejects an event only
  *            when the exact test is proven to fail (margins 1e-12 on cos(beta),
@@ -1462,7 +1465,7 @@ __global__ __launch_bounds__(64 * GRS_WPB, GRS_FAST_MIN_WAVES) void k_fast(grs_e
  * of the simplex and the barriers between).  A launch, two copies and a
  * synchronisation per iteration took 3.3 ms for 24 fits of 64 iterations
  * (52 us each, 36 of them one wave's walk through all events); this takes
- * 1.5 ms.  GRS_FIT_SLICE requests end a launch, so that it ends whatever max_iter
+ * 1.3 ms.  GRS_FIT_SLICE requests end a launch, so that it ends whatever max_iter
  * is; the host launches again while fits are left. */
 #define GRS_FIT_TEAM 4
 #define GRS_FIT_PTS 4

@@ -1,6 +1,7 @@
 /*
  * grs_resolve.h -- deciding an event without the exact FP64 pipeline where
- * that is safe (device code of k_fast and k_gt_score).
+ * that is safe (device code of the scoring, pairing, G-vector matching and
+ * centre-of-mass kernels).
  */
 #ifndef GRS_RESOLVE_H
 #define GRS_RESOLVE_H

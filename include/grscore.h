@@ -427,7 +427,7 @@ grs_status grs_grow_region(grs_ctx *ctx, const int32_t *seed, double indexed_com
  * default 1e-4) minimises fit_grain_COM_fun: the mean over the pairs of the
  * distance between the rounded simulated pixel of the pair's (hkl, omega)
  * and its measured centroid.  Each fit runs its whole Nelder-Mead on the
- * device, one wave per grain, all grains in one launch.  x_out (M x 6) =
+ * device, one block per grain, all grains in one launch.  x_out (M x 6) =
  * FitOutput, fval, the evaluation and iteration counts.  max_iter is at most
  * 100000 (it bounds a wave's run time). */
 grs_status grs_fit_grain_com(grs_ctx *ctx, const double *rows, const int64_t *row_ptr, int64_t M,
