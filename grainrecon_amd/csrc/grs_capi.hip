@@ -695,17 +695,23 @@ static bool tune_pending(const grs_ctx *c, int kind, int64_t E, int64_t waves) {
   return E >= (int64_t)(2 * ncfg + 1) * tune_part_min(c);
 }
 
-/* The beam table of V voxels that share E evaluations: from 256 evaluations a
- * voxel on, while it takes at most 1.5 GB; *beam stays nullptr otherwise.
- * With 2,700 evaluations a voxel (batched compete, 1,024 voxels) the waves
- * at work share a few tables in L2 and a call goes from 27.6 to 26.7 ms, the seed indexing
- * from 13.3 to 12.9; with 30 a voxel (compete of 30,000) they do not fit,
- * 22.1 -> 27.4 ms. */
-static const int64_t kBeamBytes = (int64_t)3 << 29;
+/* The beam table of V voxels that share E evaluations (the seed indexing;
+ * *beam stays nullptr where the terms are computed per candidate): from 256
+ * evaluations a voxel on (a few hundred make no difference), while the tables
+ * stay in cache, in an XCD's 4 MB L2 and, voxel by voxel, in a CU's 32 KB L1,
+ * or while they are few (512 KB).  Times with and without, 20,000 orientations
+ * and 50 groups of 729 a voxel, in ms: 181 angles (17 KB a voxel), 3 voxels
+ * 2.98 and 3.10, 60 voxels 29.7 and 31.3, 120 (2 MB) 58.8 and 61.3; 361 angles
+ * (35 KB), 3 voxels 4.02 and 4.00, 10 voxels 9.23 and 9.20 (with 100,000
+ * orientations 32.0 and 34.0), 60 (2 MB) 49.0 and 44.3, 300 voxels 201 and 168.
+ * Batched compete has no table: 2,744 evaluations of 960 voxels each took
+ * 45.3 ms with and 35.5 without at 361 angles, 24.0 and 24.4 (86 reflections)
+ * or 21.1 and 20.4 (64) at 181. */
+static const int64_t kBeamL2 = (int64_t)4 << 20, kBeamL1 = 32 << 10, kBeamFew = 512 << 10;
 static grs_status ensure_beam(grs_ctx *c, int64_t V, int64_t E, const double **beam) {
   *beam = nullptr;
-  const int64_t bytes = (int64_t)sizeof(double) * GRS_BT * c->nrot * V;
-  if (E < 256 * V || bytes > kBeamBytes) return GRS_OK;
+  const int64_t one = (int64_t)sizeof(double) * GRS_BT * c->nrot, bytes = one * V;
+  if (E < 256 * V || bytes > (one <= kBeamL1 ? kBeamL2 : kBeamFew)) return GRS_OK;
   ENSURE(c, c->d_beam, (size_t)bytes);
   *beam = P<double>(c->d_beam);
   return GRS_OK;
@@ -1192,8 +1198,6 @@ grs_status grs_compete_csr(grs_ctx *c, const double *pos, int64_t M, const int64
     a.out_ni = P<int32_t>(c->d_ni);
     a.out_C = P<double>(c->d_C);
     a.out_med = P<float>(c->d_med);
-    a.nrot = c->nrot;
-    if ((s = ensure_beam(c, m, E, &a.beam)) != GRS_OK) return s;
     /* the whole chunk on the device: clear keys, bounds, counts-only scoring
      * of every expanded candidate, winners, median re-scoring of the winners,
      * winner index and quaternion */
@@ -1201,9 +1205,6 @@ grs_status grs_compete_csr(grs_ctx *c, const double *pos, int64_t M, const int64
       HIPCHK(c, grs_launch_fill_u64(P<unsigned long long>(c->d_rowbest), m, 0ull, c->st));
       HIPCHK(c, grs_launch_voxel_bounds(P<grs_dgeo>(c->d_geo), P<double>(c->d_pos), m, P<double>(c->d_cs), c->nrot,
                                         P<double>(c->d_vb), c->st));
-      if (a.beam)
-        HIPCHK(c, grs_launch_beam(P<grs_dgeo>(c->d_geo), P<double>(c->d_pos), m, P<double>(c->d_cs), c->nrot,
-                                  P<double>(c->d_beam), c->st));
       grs_status ls;
       if (E > 0) {
         grs_eval_args a1 = a;
@@ -1232,8 +1233,7 @@ grs_status grs_compete_csr(grs_ctx *c, const double *pos, int64_t M, const int64
       std::memcpy(&gbits, &gs, sizeof(gbits));
       std::vector<uint64_t> key = {(uint64_t)m, (uint64_t)E, (uint64_t)S, (uint64_t)nr, gbits, (uint64_t)c->H,
                                    (uint64_t)c->nrot, (uint64_t)w1, (uint64_t)w2, (uint64_t)stride,
-                                   tune_code(c, 1), tune_code(c, 0), (uint64_t)c->autotune,
-                                   (uint64_t)(uintptr_t)a.beam};
+                                   tune_code(c, 1), tune_code(c, 0), (uint64_t)c->autotune};
       for (const DevBuf *bp : {&c->d_geo, &c->d_hkl, &c->d_cs, &c->d_vb, &c->d_pos, &c->d_keys, &c->d_bits,
                                &c->d_tbits, &c->d_scratch, &c->d_rowptr, &c->d_roweoff, &c->d_candq, &c->d_rowbest, &c->d_elist,
                                &c->d_ns, &c->d_ni, &c->d_C, &c->d_med, &c->d_bestidx, &c->d_bestq})

@@ -524,10 +524,10 @@ __device__ __forceinline__ void beam_row(const grs_dgeo *g, const double *P, dou
 }
 
 /* The beam table of V voxels in device memory, for launches whose voxels have
- * many evaluations each: k_fast then loads the terms of a candidate (six
- * 16-byte loads from L1/L2) instead of 45 operations with two reciprocals.
- * 343 x 7.9 samples of 1,024 voxels: 27.6 -> 26.7 ms; 24 orientation fits:
- * 1.47 -> 1.39 ms. */
+ * many evaluations each and whose tables stay in cache: the scoring kernel then loads the terms of a
+ * candidate (six 16-byte loads from L1/L2) instead of 45 operations with two
+ * reciprocals.  262,144 orientations and 500 groups of 729 at two voxels: 13.0 -> 12.3 ms;
+ * 24 orientation fits: 1.47 -> 1.39 ms. */
 __global__ __launch_bounds__(256) void k_beam(const grs_dgeo *g, const double *pos, int64_t V, const double *cs,
                                               int32_t nrot, double *beam) {
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -1409,7 +1409,7 @@ __global__ __launch_bounds__(64 * GRS_WPB, GRS_FAST_MIN_WAVES) void k_fast(grs_e
       if (threadIdx.x == 0) team[0] = team[1] = team[2] = 0;
       __syncthreads();
     }
-    if (MAP == GRS_MAP_CSR || MAP == GRS_MAP_GRID)
+    if (MAP == GRS_MAP_GRID)
       btab = a.beam ? a.beam + (int64_t)GRS_BT * a.nrot * vi : nullptr;
     score_events<MEDIAN, AUDIT, TEAM>(a, g, b1thr, btab, L, sub, vi, hlo, hend, wlist, &team[2], &ns, &ni);
     if (TEAM) {

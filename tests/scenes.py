@@ -7,6 +7,7 @@ Sizes are chosen so the oracle finishes in seconds.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 
 import numpy as np
@@ -35,6 +36,13 @@ def U_from_qvec(q1, q2, q3):
         [2.0 * (q1 * q2 + q0 * q3), 2.0 * (q0 * q0 + q2 * q2) - 1.0, 2.0 * (q2 * q3 - q0 * q1)],
         [2.0 * (q1 * q3 - q0 * q2), 2.0 * (q2 * q3 + q0 * q1), 2.0 * (q0 * q0 + q3 * q3) - 1.0],
     ])
+
+
+def free_device_memory(engine):
+    """Bytes free on the device, from the HIP runtime the engine's library is linked to."""
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert engine._lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
 
 
 class Scene:

@@ -254,11 +254,10 @@ def test_grow_row_counts(engine, M):
 
 
 @pytest.mark.parametrize("nr, k", [(0, 255), (0, 256), (0, 257), (5, 1), (6, 1)])
-def test_compete_csr_with_and_without_the_beam_table(engine, nr, k):
-    """Evaluations per voxel around the rule for the voxels' beam table
-    (samples x candidates: 255, 256, 257, 216, 343), on uniform rotation
-    angles and on others: winners and counts equal the scores of the whole
-    lists."""
+def test_compete_csr_evaluations_per_voxel(engine, nr, k):
+    """255, 256, 257, 216 and 343 evaluations (samples x candidates) of each
+    voxel, on uniform rotation angles and on others: winners and counts equal
+    the scores of the whole lists."""
     s = scenes.make_scene(seed=45, ngrains=2, spread_mm=0.02, nrot=13)
     rng = np.random.default_rng(nr * 1000 + k)
     g = 0.003
@@ -278,6 +277,26 @@ def test_compete_csr_with_and_without_the_beam_table(engine, nr, k):
             j = int(np.nanargmax(rC))
             assert best[r] == j and ns[r] == rns[j] and ni[r] == rni[j]
             assert _bits(C[r:r + 1])[0] == _bits(rC[j:j + 1])[0] and med[r] == rmed[j]
+
+
+def test_compete_csr_holds_no_beam_table():
+    """4,000 voxels of 343 samples take no more device memory than of 216: a
+    beam table of theirs (361 angles: 139 MB) made such calls slower."""
+    from grainrecon_amd import Engine
+
+    s = scenes.make_scene(seed=45, ngrains=1, spread_mm=0.02, nrot=361, det=64, pixel_mm=6.72e-3 * 16)
+    rng = np.random.default_rng(3)
+    pos = np.tile(s.centers[:1], (4000, 1)) + rng.uniform(-0.01, 0.01, (4000, 3))
+    e = Engine(0)
+    try:
+        e.set_geometry(s.geo, s.hkl[:60], s.rot)
+        e.set_distance_stack(s.proj)
+        e.compete_csr(pos, np.arange(4001), np.tile(s.q, (4000, 1)), 5, 0.003)
+        free = scenes.free_device_memory(e)
+        e.compete_csr(pos, np.arange(4001), np.tile(s.q, (4000, 1)), 6, 0.003)
+        assert free - scenes.free_device_memory(e) < 32 << 20
+    finally:
+        e.close()
 
 
 @pytest.mark.parametrize("counts", [[0], [1], [0, 63, 64, 65, 0, 200, 2]])

@@ -192,3 +192,25 @@ def test_index_seeds_small_set_and_more_fits_than_seeds(engine):
         row = ref["indexing"].copy()
         row[0] = p + 1
         assert _same(got["indexing"][p], row) and got["candidate"][p] == ref["candidate"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nrot, count", [(181, 241), (181, 242), (341, 128), (341, 129), (342, 15), (342, 16)])
+def test_index_seeds_with_and_without_the_beam_table(engine, nrot, count):
+    """Numbers of voxels around the rule for their beam tables (4 MB in all
+    while one is at most 32 KB, 512 KB otherwise): a call equals the calls of
+    its voxels in tens, which have the tables."""
+    s = scenes.make_scene(seed=88, ngrains=2, spread_mm=0.03, nrot=nrot, det=64, pixel_mm=6.72e-3 * 16)
+    rng = np.random.default_rng(nrot + count)
+    qs = scenes.random_quats(rng, 2000)
+    qs = np.concatenate([s.q, qs[qs[:, 0] >= 0.5]])[:300]
+    engine.set_geometry(s.geo, s.hkl[:64], s.rot)
+    engine.set_distance_stack(s.proj)
+    engine.set_orientation_set(qs)
+    pos = s.centers[rng.integers(0, 2, count)] + rng.uniform(-0.01, 0.01, (count, 3))
+    lim = dict(nr_seed=2, nr=2, max_fun_evals=6)
+    got = engine.index_seeds(pos, **lim)
+    parts = [engine.index_seeds(pos[k:k + 10], **lim) for k in range(0, count, 10)]
+    for key in ("candidate", "x0", "x", "fval", "n_fun_evals", "n_iter", "seed_idx", "seed_C"):
+        assert _same(got[key], np.concatenate([p[key] for p in parts])), key
+    assert _same(got["indexing"][:, 1:], np.concatenate([p["indexing"] for p in parts])[:, 1:])
