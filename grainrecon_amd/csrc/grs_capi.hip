@@ -102,7 +102,7 @@ struct grs_ctx {
   DevBuf v_lin, v_out; /* grs_get_volume_at */
   /* grain centre-of-mass fit buffers */
   DevBuf m_rows, m_rptr, m_nm, m_cs, m_dis;
-  DevBuf f_in, f_cnt; /* fit_batch: packed per-step inputs and counts */
+  DevBuf f_in, f_cnt; /* fit_batch: packed positions and starts, results */
   void *h_pin = nullptr; /* pinned memory of small calls (ensure_pin) */
   size_t h_pin_cap = 0;
   unsigned char *h_stage = nullptr; /* pinned staging of large transfers (staged_copy) */
@@ -1627,7 +1627,10 @@ static grs_status fit_batch(grs_ctx *c, const double *pos, const double *x0, int
                             double *fval, int32_t *n_fun_evals, int32_t *n_iter) {
   if (M > INT32_MAX / 4) return fail(c, GRS_ERR_ARG, "too many fits");
   if (c->H > 240) return fail(c, GRS_ERR_ARG, "the fast method supports at most 240 reflections (got %d)", c->H);
-  const int64_t most = 16384; /* fits per launch (a block each) */
+  /* fits per launch (a block each): their state, and 512 MB of beam tables
+   * (15,000 fits at 361 rotation angles, 155 at 36,001) */
+  int64_t most = ((int64_t)512 << 20) / ((int64_t)sizeof(double) * GRS_BT * c->nrot);
+  most = most < 1 ? 1 : most > 16384 ? 16384 : most;
   if (M > most) {
     for (int64_t b = 0; b < M; b += most) {
       const grs_status s = fit_batch(c, pos + 3 * b, x0 + 3 * b, M - b < most ? M - b : most, half_width, max_fun_evals,

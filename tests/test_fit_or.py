@@ -92,3 +92,30 @@ def test_fit_longer_than_one_launch(engine, scene):
     rx, rf, rnf, rit = fit_or_local(s.geo, s.stack, pos[0], x0[0], s.rot, s.hkl, max_fun_evals=20000, max_iter=1000000)
     np.testing.assert_array_equal(x[0], rx)
     assert fv[0] == rf and nf[0] == rnf and it[0] == rit
+
+
+@pytest.mark.gpu
+def test_large_batches_bound_their_tables():
+    """8,000 fits at 1,441 angles run in launches whose beam tables take at
+    most 512 MB (1.1 GB in one launch), with the results of small calls around
+    the launches' ends."""
+    from grainrecon_amd import Engine
+
+    s = scenes.make_scene(seed=61, ngrains=2, spread_mm=0.03, nrot=1441, det=64, pixel_mm=6.72e-3 * 16)
+    rng = np.random.default_rng(7)
+    pos = s.centers[rng.integers(0, 2, 8000)] + rng.uniform(-0.01, 0.01, (8000, 3))
+    x0 = s.q[rng.integers(0, 2, 8000), 1:] + rng.normal(scale=2e-3, size=(8000, 3))
+    e = Engine(0)
+    try:
+        e.set_geometry(s.geo, s.hkl[:8], s.rot)
+        e.set_distance_stack(s.proj)
+        e.fit_or_local(pos[:5], x0[:5], max_fun_evals=10)
+        free = scenes.free_device_memory(e)
+        got = e.fit_or_local(pos, x0, max_fun_evals=10)
+        assert free - scenes.free_device_memory(e) < 700 << 20
+        most = (512 << 20) // (96 * 1441)
+        for part in (slice(0, 5), slice(most - 3, most + 3), slice(2 * most - 3, 2 * most + 3), slice(7995, 8000)):
+            for a, b in zip(got, e.fit_or_local(pos[part], x0[part], max_fun_evals=10)):
+                np.testing.assert_array_equal(a[part], b)
+    finally:
+        e.close()
