@@ -1,4 +1,6 @@
 """GPU input preparation: spot rendering and the exact distance transform."""
+import ctypes
+
 import numpy as np
 import pytest
 from scipy import ndimage
@@ -75,6 +77,43 @@ def test_large_transfers_keep_every_byte(engine, extra):
     m = rng.random((48 + extra, ny, nz)) < 0.5
     engine.set_binary_stack(m.transpose(2, 1, 0))
     assert np.array_equal(engine.get_mask((nz, ny, 48 + extra)), m.transpose(2, 1, 0))
+
+
+def test_pinned_host_memory_is_copied_directly():
+    """A stack in memory that the caller pinned goes to the device in one
+    copy: no staging buffers (64 MB) and threads, which made it slower (15.4
+    instead of 13.5 ms for 759 MB); one in pageable memory still has them."""
+    from grainrecon_amd import Engine
+
+    nz, ny, nrot = 1024, 1024, 16
+
+    def address_space():
+        return next(int(x.split()[1]) << 10 for x in open("/proc/self/status") if x.startswith("VmSize"))
+
+    e = Engine(0)
+    p = ctypes.c_void_p()
+    assert e._lib.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(4 * nz * ny * nrot), 0) == 0
+    try:
+        pinned = np.frombuffer((ctypes.c_float * (nz * ny * nrot)).from_address(p.value), np.float32)
+        rng = np.random.default_rng(9)
+        pinned[:] = rng.random(pinned.size, dtype=np.float32)
+        pageable = pinned + 1
+        mask = np.zeros((nz, ny, nrot), bool)
+        mask[3, 4] = True
+        e.set_binary_stack(mask)  # the stack's buffer, and what the first copies allocate
+        e.distance_from_mask()
+        e.set_distance_stack(pinned[:nz * ny].reshape(1, ny, nz).transpose(2, 1, 0))
+        shape = (nz, ny, nrot)
+        for src, low, high in ((pinned, -(1 << 30), 32 << 20), (pageable, 60 << 20, 1 << 40)):
+            used = address_space()
+            e.set_distance_stack(src.reshape(shape[::-1]).transpose(2, 1, 0))
+            assert low < address_space() - used < high
+        assert np.array_equal(e.get_distance_stack(shape).ravel(order="F"), pageable)
+        e.set_distance_stack(pinned.reshape(shape[::-1]).transpose(2, 1, 0))
+        assert np.array_equal(e.get_distance_stack(shape).ravel(order="F"), pinned)
+    finally:
+        e.close()
+        assert e._lib.hipHostFree(p) == 0
 
 
 def test_rendered_scene_scores_one_at_truth(engine):
