@@ -2122,6 +2122,7 @@ grs_status grs_pair_spots(grs_ctx *c, const double *pos, const double *U, int64_
   int64_t chunk = ((int64_t)1 << 26) / E;
   if (chunk < 1) chunk = 1;
   std::vector<int64_t> cnt;
+  bool over = false;
   for (int64_t m0 = 0; m0 < M; m0 += chunk) {
     const int64_t m = M - m0 < chunk ? M - m0 : chunk;
     const int64_t me = m * E;
@@ -2150,10 +2151,8 @@ grs_status grs_pair_spots(grs_ctx *c, const double *pos, const double *U, int64_
       rp[k + 1] = rp[k] + cnt[k];
       row_ptr[m0 + k + 1] = row_ptr[m0 + k] + cnt[k];
     }
-    if (!rows || rp[m] == 0) continue;
-    if (row_ptr[m0 + m] > cap)
-      return fail(c, GRS_ERR_ARG, "%lld pair rows do not fit the capacity %lld", (long long)row_ptr[m0 + m],
-                  (long long)cap);
+    over = over || (rows && row_ptr[m0 + m] > cap); /* the rest is counted only */
+    if (!rows || over || rp[m] == 0) continue;
     ENSURE(c, c->p_rows, sizeof(double) * 23 * rp[m]);
     HIPCHK(c, hipMemcpyAsync(c->p_rowptr.p, rp.data(), sizeof(int64_t) * (m + 1), hipMemcpyHostToDevice, c->st));
     HIPCHK(c, grs_launch_pair_rows(P<grs_dgeo>(c->d_geo), P<double>(c->d_hkl), P<double>(c->d_rot),
@@ -2166,6 +2165,8 @@ grs_status grs_pair_spots(grs_ctx *c, const double *pos, const double *U, int64_
     HIPCHK(c, hipStreamSynchronize(c->st));
   }
   HIPCHK(c, hipStreamSynchronize(c->st));
+  if (over)
+    return fail(c, GRS_ERR_ARG, "%lld pair rows do not fit the capacity %lld", (long long)row_ptr[M], (long long)cap);
   return GRS_OK;
 }
 

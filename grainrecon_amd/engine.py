@@ -292,13 +292,14 @@ class Engine:
             return self._lib.grs_pair_spots(self._h, _ptr(pos, _dp), _ptr(U, _dp), M, _ptr(ns, _ip), _ptr(ni, _ip),
                                             _ptr(med, _fp), rp.ctypes.data_as(i64p), rows, cap)
 
-        # a grain pairs a few hundred spots: one call with room for 1024 each,
-        # and where that is not enough one for the counts and one for the rows
-        rows = np.empty((max(1024 * M, 1), 23))
-        if call(_ptr(rows, _dp), rows.shape[0]) != L.GRS_OK:
-            self._chk(call(None, 0))
-            rows = np.zeros((max(int(rp[-1]), 1), 23))
-            self._chk(call(_ptr(rows, _dp), rows.shape[0]))
+        # a grain pairs a few hundred spots: one call with room for 1024 each (up to 193 MB in
+        # all), and where that is not enough a second one, whose row count the first returned
+        rows = np.empty((max(min(1024 * M, 1 << 20), 1), 23))
+        code = call(_ptr(rows, _dp), rows.shape[0])
+        if code == L.GRS_ERR_ARG and rp[-1] > rows.shape[0]:
+            rows = np.empty((int(rp[-1]), 23))
+            code = call(_ptr(rows, _dp), rows.shape[0])
+        self._chk(code)
         return ns, ni, med, [rows[rp[m]:rp[m + 1]].copy() for m in range(M)]
 
     # -- grain centre-of-mass fit -----------------------------------------------------

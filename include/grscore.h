@@ -369,8 +369,9 @@ grs_status grs_set_frame_spots(grs_ctx *ctx, const int64_t *frame_ptr, int64_t n
  * rounded to single precision as MATLAB's concatenation with the single dis
  * does.  A hit is paired with the nearest spot of its projection (first
  * minimum) when that distance is below min(sqrt(area), 15).  rows = NULL
- * returns row_ptr only; GRS_ERR_ARG when the rows exceed cap.  Replaces the
- * host loop of forward_comp_pair_spots.m (called from
+ * returns row_ptr only; GRS_ERR_ARG when the rows exceed cap (row_ptr is
+ * complete then, rows is not).  Replaces the host loop of
+ * forward_comp_pair_spots.m (called from
  * fit_OR_constrain_with_local_comp_cuda.m:89,151). */
 grs_status grs_pair_spots(grs_ctx *ctx, const double *pos, const double *U, int64_t M, int32_t *ns, int32_t *ni,
                           float *med, int64_t *row_ptr, double *rows, int64_t cap);

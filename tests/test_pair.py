@@ -1,5 +1,7 @@
 """Spot pairing (forward_comp_pair_spots.m:3-93): the oracle pinned on
 constructed spot lists, the GPU (grs_pair_spots) against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -137,3 +139,74 @@ def test_pair_spots_of_more_rows_than_the_first_call_holds(engine):
     rns, rni, rmed, rrows = pair_spots(s.geo, stack, s.U[0], s.centers[0], s.rot, hkl, frames)
     assert rows[0].shape[0] == len(ev) == ns[0]
     np.testing.assert_array_equal(rows[0], rrows)
+
+
+class _PairLib:
+    """grs_pair_spots with `per` rows an orientation, or with an error."""
+
+    def __init__(self, per, error=0):
+        self.per, self.error, self.caps = per, error, []
+
+    def grs_pair_spots(self, h, pos, U, M, ns, ni, med, rp, rows, cap):
+        self.caps.append(cap)
+        rp[0] = 0
+        if self.error:
+            return self.error
+        for m in range(M):
+            rp[m + 1] = rp[m] + self.per
+        return -1 if rp[M] > cap else 0
+
+
+def _pair_engine(lib):
+    from grainrecon_amd import Engine
+
+    class Stub(Engine):
+        def __init__(self):
+            self._lib, self._h = lib, None
+
+        def _chk(self, code):
+            assert code == 0, code
+
+    return Stub()
+
+
+@pytest.mark.parametrize("per, M, calls", [(1024, 3, 1), (1025, 3, 2), (5, 2000, 1), (600, 2000, 2)])
+def test_pair_spots_calls(per, M, calls):
+    """One call where the first buffer (1024 rows an orientation, at most 2^20)
+    holds the pairs, else a second one for exactly as many as there are."""
+    lib = _PairLib(per)
+    _, _, _, rows = _pair_engine(lib).pair_spots(np.zeros((M, 3)), np.zeros((M, 9)))
+    assert len(lib.caps) == calls and lib.caps[0] == min(1024 * M, 1 << 20)
+    assert calls == 1 or lib.caps[1] == per * M
+    assert [r.shape for r in rows] == [(per, 23)] * M
+
+
+@pytest.mark.parametrize("error", [-1, -3, -4])
+def test_pair_spots_reports_an_error_at_once(error):
+    lib = _PairLib(5, error)
+    with pytest.raises(AssertionError, match=str(error)):
+        _pair_engine(lib).pair_spots(np.zeros((3, 3)), np.zeros((3, 9)))
+    assert len(lib.caps) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nrot, M", [(37, 3), (6001, 131)])
+def test_pair_spots_counts_beyond_the_capacity(engine, nrot, M):
+    """A call whose rows do not fit still returns every row count, in one
+    chunk of orientations and in two (2^26 / (6001 x 86) = 130 a chunk)."""
+    from grainrecon_amd import _lib as L
+
+    s = scenes.make_scene(seed=85, ngrains=1, spread_mm=0.02, nrot=nrot, det=32, pixel_mm=6.72e-3 * 32)
+    engine.set_geometry(s.geo, s.hkl, s.rot)
+    engine.set_distance_stack(np.zeros_like(s.proj))
+    engine.set_frame_spots([np.array([[16.0, 16.0, 81.0]])] * nrot)
+    pos, U = np.repeat(s.centers[:1], M, 0), np.repeat(np.reshape(s.U[0], (1, 9)), M, 0)
+    _, _, _, rows = engine.pair_spots(pos, U)
+    n = rows[0].shape[0]
+    assert n > 0 and all(np.array_equal(r, rows[0]) for r in rows)
+    out, rp = np.zeros((n, 23)), np.zeros(M + 1, np.int64)
+    ns, ni, med = np.zeros(M, np.int32), np.zeros(M, np.int32), np.zeros(M, np.float32)
+    p = lambda a: a.ctypes.data_as(ctypes.POINTER(np.ctypeslib.as_ctypes_type(a.dtype)))  # noqa: E731
+    code = engine._lib.grs_pair_spots(engine._h, p(pos), p(U), M, p(ns), p(ni), p(med), p(rp), p(out), n)
+    assert code == L.GRS_ERR_ARG and np.array_equal(rp, n * np.arange(M + 1))
+    assert f"{M * n} pair rows do not fit" in engine._lib.grs_last_error(engine._h).decode()
