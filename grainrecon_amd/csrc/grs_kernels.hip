@@ -57,13 +57,17 @@ __host__ __device__ inline int64_t fast_wave_doubles(int32_t H) {
   return (int64_t)H * GRS_GWT + GRS_RING_DOUBLES + GRS_RANGE_DOUBLES(H) + 4 + 9;
 }
 
+/* k_fast's static LDS: the geometry, the thresholds of b1_classify and a
+ * team's counters, rounded up */
+#define GRS_FAST_STATIC_LDS ((int64_t)((sizeof(grs_dgeo) + 12 * sizeof(double) + 3 * sizeof(int32_t) + 127) / 128 * 128))
+
 /* LDS doubles of the one-voxel beam table behind the wave regions: the
- * table is kept when the block's dynamic LDS stays within 160 KB (one CU's
+ * table is kept when the block's LDS stays within 160 KB (one CU's
  * LDS; with 8 waves per block two blocks, 16 waves, share a CU) */
 __host__ __device__ inline int64_t fast_tab_doubles(int32_t map, int32_t nrot, int32_t H, int wpb) {
   if (map != GRS_MAP_ONE_VOXEL || nrot <= 0) return 0;
   const int64_t t = (int64_t)GRS_BT * nrot;
-  return ((int64_t)wpb * fast_wave_doubles(H) + t) * (int64_t)sizeof(double) <= 163840 ? t : 0;
+  return ((int64_t)wpb * fast_wave_doubles(H) + t) * (int64_t)sizeof(double) <= 163840 - GRS_FAST_STATIC_LDS ? t : 0;
 }
 
 __device__ __forceinline__ void wave_sync() {

@@ -209,6 +209,29 @@ def test_small_launches_share_evaluations(engine, H):
                 assert np.array_equal(_bits(x), _bits(y[:n])), n
 
 
+@pytest.mark.parametrize("H, wpb, nrots", [(86, 8, (1044, 1045, 1046, 1047, 1053, 1054)), (86, 1, (1616, 1617, 1618, 1625)),
+                                           (240, 4, (908, 909, 910, 918))])
+def test_beam_table_next_to_static_lds(engine, H, wpb, nrots):
+    """Rotation counts around the largest beam table that a one-voxel launch
+    keeps in LDS beside its waves' regions and the kernel's static LDS (one
+    that fits only without the latter was refused at the launch)."""
+    s = scenes.make_scene(seed=52, det=64, pixel_mm=6.72e-3 * 16, nrot=7)
+    rng = np.random.default_rng(H)
+    hkl = np.concatenate([s.hkl, 2 * s.hkl, 3 * s.hkl])[:H]
+    q = np.concatenate([s.q, scenes.random_quats(rng, 2558)])
+    assert q.shape[0] == 2561  # more than the launches that share evaluations
+    for nrot in nrots:
+        engine.set_geometry(s.geo, hkl, np.linspace(0.0, 360.0, nrot))
+        engine.set_distance_stack(rng.integers(0, 40, (64, 64, nrot)).astype(np.float32))
+        engine.set_launch_config(0, wpb, _lib.MASK_BITS, False)
+        try:
+            got = engine.forward_comp(s.centers[0], q)
+        finally:
+            engine.set_launch_config(0, 0)
+        for x, y in zip(got, engine.forward_comp(s.centers[0], q, _lib.METHOD_PLAIN)):
+            assert np.array_equal(_bits(x), _bits(y)), nrot
+
+
 @pytest.mark.parametrize("nrot", [1701, 1851, 2001, 3841])
 def test_many_candidates_per_evaluation(engine, nrot):
     """Rotation counts whose evaluations have about 3,800, 4,100, 4,500 and
