@@ -85,7 +85,7 @@ __device__ __forceinline__ double com_pair_dist(const grs_dgeo *g, const double 
 /* One block per fit m: the first wave steps the Nelder-Mead state machine
  * (started on the host) in registers (nm_lanes); for the requested points - a
  * reflection together with the three points its value can lead to
- * (grs_nm::follow_ups), so that an iteration is one round - the point
+ * (grs_nm::points), so that an iteration is one round - the point
  * coordinates and the six cosines and sines of each point's angles are
  * computed one per thread, the first threads build each point's U and SUB,
  * all threads compute the (point, pair) distances, and thread p adds point
@@ -121,7 +121,7 @@ __global__ __launch_bounds__(COM_THREADS) void k_com_nm(const grs_dgeo *g, const
   }
   __syncthreads();
   for (;;) {
-    if (t == 0) npts = nm->done() ? 0 : (nm->st == grs_nm::REFLECT ? 4 : nm->npend);
+    if (t == 0) npts = nm->points();
     __syncthreads();
     const int np = npts;
     if (np == 0) break;
@@ -129,9 +129,8 @@ __global__ __launch_bounds__(COM_THREADS) void k_com_nm(const grs_dgeo *g, const
       const int p = t / 6, k = t - 6 * p;
       double u = nm->pend[p][k];
       if (nm->st == grs_nm::REFLECT && p > 0) {
-        /* grs_nm::follow_ups, coordinate k */
         const double xb = nm->xbar[k], vn = nm->v[nm->n][k];
-        u = p == 1 ? (1.0 + 2.0) * xb - 2.0 * vn : p == 2 ? (1.0 + 0.5) * xb - 0.5 * vn : (1.0 - 0.5) * xb + 0.5 * vn;
+        u = GRS_NM_FOLLOW_UP(p, xb, vn);
       }
       double u6[6], x;
       u6[k] = u;

@@ -1462,7 +1462,7 @@ __global__ __launch_bounds__(64 * GRS_WPB, GRS_FAST_MIN_WAVES) void k_fast(grs_e
  * fminsearchbnd on the device.  The block's 16 waves are four teams of four
  * (score_events with the reflections split four ways), one team per point: a
  * requested reflection is scored together with the three points that its
- * value can lead to (grs_nm::follow_ups), the initial simplex and a shrink
+ * value can lead to (grs_nm::points), the initial simplex and a shrink
  * have at most four points.  The first wave steps the method
  * (nm_lanes).  The points, values and counts are the sequential method's.
  * Bound: one iteration's chain (a wave's events of 22 of 86 reflections, the step
@@ -1520,18 +1520,17 @@ __global__ __launch_bounds__(64 * GRS_FIT_TEAM * GRS_FIT_PTS, GRS_FAST_MIN_WAVES
   __syncthreads();
   int32_t step = 0;
   for (; step < GRS_FIT_SLICE; step++) {
-    if (t == 0) npts = nm->done() ? 0 : (nm->st == grs_nm::REFLECT ? 4 : nm->npend);
+    if (t == 0) npts = nm->points();
     if (t < 2 * GRS_FIT_PTS) cnt[t >> 1][t & 1] = 0;
     __syncthreads();
     const int np = npts;
     if (np == 0) break;
     if (t < 3 * np) {
       const int q = t / 3, k = t - 3 * q;
-      /* a reflection's follow-ups: grs_nm::follow_ups, coordinate k */
       double u = nm->pend[q][k];
       if (nm->st == grs_nm::REFLECT && q > 0) {
         const double xb = nm->xbar[k], vn = nm->v[nm->n][k];
-        u = q == 1 ? (1.0 + 2.0) * xb - 2.0 * vn : q == 2 ? (1.0 + 0.5) * xb - 0.5 * vn : (1.0 - 0.5) * xb + 0.5 * vn;
+        u = GRS_NM_FOLLOW_UP(q, xb, vn);
       }
       double u3[3];
       u3[k] = u;

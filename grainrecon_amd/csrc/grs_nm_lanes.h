@@ -1,22 +1,30 @@
 /*
  * grs_nm_lanes.h -- the Nelder-Mead of grs_nm.h stepped by one wave inside a
- * kernel (k_com_nm, k_fit_nm).
+ * kernel (k_com_nm, k_fit_nm).  Outside of HIP, __shfl and __shfl_xor are the
+ * includer's (the tests run a wave's lanes as threads).
  */
 #ifndef GRS_NM_LANES_H
 #define GRS_NM_LANES_H
 
 #include "grs_nm.h"
 
-/* grs_nm::feed for N coordinates, stepped by the 64 lanes of one wave in
+#ifdef __HIPCC__
+#define GRS_NM_LANES_FN __device__ __forceinline__
+#else
+#define GRS_NM_LANES_FN inline
+#endif
+
+/* The steps of the method for N coordinates, taken by the 64 lanes of one wave in
  * registers: lane k holds coordinate k of the simplex, xbar and xr, and every
  * lane holds the values, counts and state and takes the method's decisions
- * on them.  load() and store() move the state between the registers and the
+ * on them.  The constructor and store() move the state between the registers and the
  * grs_nm in LDS around a step (so that it costs no registers between steps),
  * each one round of independent accesses; all loops are unrolled over N.  The
- * state afterwards is grs_nm::feed's, bit for bit: grs_nm's statements for the
+ * results are the sequential method's, bit for bit: its statements for the
  * coordinate, the stopping test's largest vertex distance and largest
  * coordinate reduced across the lanes (a maximum is exact), and the stable
- * insertion sort as exchanges of neighbours.  Stepped on the grs_nm in LDS, one dependent access
+ * insertion sort as exchanges of neighbours.  Stepped by one lane on the grs_nm in
+ * LDS, one dependent access
  * after the other, a step of six coordinates with its follow-up took 11,900
  * cycles; three fits of six coordinates went from 1.61 to 1.22 ms with this. */
 template <int N>
@@ -29,7 +37,7 @@ struct nm_lanes {
   double tol_f, tol_x;
   grs_nm::State st;
 
-  __device__ __forceinline__ nm_lanes(grs_nm *nm, int lane) : s(nm), k(lane < N ? lane : N - 1), on(lane < N) {
+  GRS_NM_LANES_FN nm_lanes(grs_nm *nm, int lane) : s(nm), k(lane < N ? lane : N - 1), on(lane < N) {
 #pragma unroll
     for (int j = 0; j <= N; j++) {
       v[j] = s->v[j][k];
@@ -49,7 +57,7 @@ struct nm_lanes {
     st = s->st;
   }
 
-  __device__ __forceinline__ void store() {
+  GRS_NM_LANES_FN void store() {
     if (on) {
 #pragma unroll
       for (int j = 0; j <= N; j++) s->v[j][k] = v[j];
@@ -71,14 +79,14 @@ struct nm_lanes {
   }
 
   /* largest of the N lanes' values (the lanes beyond repeat lane N - 1's) */
-  __device__ __forceinline__ static double lanes_max(double x) {
+  GRS_NM_LANES_FN static double lanes_max(double x) {
     for (int off = 4; off > 0; off >>= 1) x = grs_nm_max(x, __shfl_xor(x, off, 64));
     return __shfl(x, 0, 64);
   }
 
   /* entry i into the sorted entries 0 .. i - 1 (stable, NaN last) */
   template <int I>
-  __device__ __forceinline__ void insert() {
+  GRS_NM_LANES_FN void insert() {
 #pragma unroll
     for (int j = I - 1; j >= 0; j--) {
       const double a = fv[j], b = fv[j + 1];
@@ -92,12 +100,12 @@ struct nm_lanes {
   }
 
   template <int I = 1>
-  __device__ __forceinline__ void sort() {
+  GRS_NM_LANES_FN void sort() {
     insert<I>();
     if constexpr (I < N) sort<I + 1>();
   }
 
-  __device__ __forceinline__ void begin() {
+  GRS_NM_LANES_FN void begin() {
     GRS_NO_CONTRACT
     if (!(nf < max_fe && it < max_it)) {
       st = grs_nm::DONE;
@@ -128,13 +136,13 @@ struct nm_lanes {
   }
 
   /* the last entry replaced: it alone can be out of order */
-  __device__ __forceinline__ void end_iter() {
+  GRS_NM_LANES_FN void end_iter() {
     insert<N>();
     it += 1;
     begin();
   }
 
-  __device__ __forceinline__ void shrink() {
+  GRS_NM_LANES_FN void shrink() {
     GRS_NO_CONTRACT
 #pragma unroll
     for (int j = 1; j <= N; j++) v[j] = v[0] + 0.5 * (v[j] - v[0]);
@@ -142,7 +150,7 @@ struct nm_lanes {
     st = grs_nm::SHRINK;
   }
 
-  __device__ __forceinline__ void feed(const double *f) {
+  GRS_NM_LANES_FN void feed(const double *f) {
     GRS_NO_CONTRACT
     switch (st) {
       case grs_nm::INIT:
@@ -160,7 +168,7 @@ struct nm_lanes {
         fxr = f[0];
         nf += 1;
         if (fxr < fv[0]) {
-          pend0 = (1.0 + 2.0) * xbar - 2.0 * v[N];
+          pend0 = GRS_NM_FOLLOW_UP(1, xbar, v[N]);
           npend = 1;
           st = grs_nm::EXPAND;
           return;
@@ -172,10 +180,10 @@ struct nm_lanes {
           return;
         }
         if (fxr < fv[N]) {
-          pend0 = (1.0 + 0.5) * xbar - 0.5 * v[N];
+          pend0 = GRS_NM_FOLLOW_UP(2, xbar, v[N]);
           st = grs_nm::CONTRACT_OUT;
         } else {
-          pend0 = (1.0 - 0.5) * xbar + 0.5 * v[N];
+          pend0 = GRS_NM_FOLLOW_UP(3, xbar, v[N]);
           st = grs_nm::CONTRACT_IN;
         }
         npend = 1;
@@ -215,10 +223,10 @@ struct nm_lanes {
     }
   }
 
-  /* a step with the values f (in LDS) of the requested points; a reflection's
-   * follow-ups (grs_nm::follow_ups) stand behind its own value.  One call
+  /* a step with the values f (in LDS) of grs_nm's points: a reflection's
+   * follow-ups stand behind its own value.  One call
    * site of feed, so that it is inlined and the state stays in registers. */
-  __device__ __forceinline__ void step(const double *f) {
+  GRS_NM_LANES_FN void step(const double *f) {
     for (int q = 0;;) {
       const bool refl = st == grs_nm::REFLECT;
       feed(f + q);

@@ -1,6 +1,6 @@
 """Known-answer pins of the Nelder-Mead restatements: the oracle's
-(oracle/fminsearch.py) and the engine's state machine (grs_nm.h, driven on
-the host through tests/nm_harness.hip).
+(oracle/fminsearch.py) and the engine's (the state of grs_nm.h stepped by
+nm_lanes as in the kernels, a wave's lanes as threads of tests/nm_harness.cpp).
 
 The hand-derived sequence below starts from a dyadic simplex, so every trial
 point is exact in binary, and visits one branch of fminsearch's iteration
@@ -74,14 +74,12 @@ START = [[0.0, 0.0], [4.0, 0.0], [0.0, 4.0]]
 
 @pytest.fixture(scope="module")
 def harness(tmp_path_factory):
-    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
-    if not os.path.exists(hipcc):
-        pytest.skip("hipcc not available")
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("g++ not available")
     out = str(tmp_path_factory.mktemp("nm") / "libnmh.so")
-    subprocess.run([hipcc, "-O2", "-std=c++17", "-fPIC", "-shared", "--offload-arch=gfx950", "-ffp-contract=off",
-                    "-fno-fast-math", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-                    "-Wno-unused-command-line-argument", "-I", CSRC, "-o", out, os.path.join(HERE, "nm_harness.hip")],
-                   check=True, capture_output=True)
+    subprocess.run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-pthread", "-ffp-contract=off", "-I", CSRC, "-o", out,
+                    os.path.join(HERE, "nm_harness.cpp")], check=True, capture_output=True)
     L = ctypes.CDLL(out)
     dp = ctypes.POINTER(ctypes.c_double)
     ip = ctypes.POINTER(ctypes.c_int)
@@ -180,7 +178,7 @@ def _run_follow_ups(harness, f, sim0, max_it, tol_f, tol_x, cap=4096):
 
 def test_follow_ups_feed_the_derived_sequence(harness):
     """The engine's fits evaluate each reflection's three follow-ups
-    (grs_nm::follow_ups) in the same launch and feed the expansion or
+    (grs_nm::points) in the same round and feed the expansion or
     contraction the method requests from them.  On the derived sequence
     (off-table points are NaN, which only a wrongly fed follow-up would
     reach) the points fed, the counts and the final simplex are the known
@@ -219,6 +217,38 @@ def test_follow_ups_equal_the_plain_drive_bit_for_bit(harness):
     assert fed == visited
     assert np.array_equal(sim2.reshape(-1), sim) and np.array_equal(fv2, fv) and (nf2, it2) == (nf.value, it.value)
     assert min(hits) > 0 and nf.value > 200
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 6, 8])
+def test_lanes_follow_the_oracle_with_ties_and_nan(harness, n):
+    """An objective of plateaus (ties in every sort) that is NaN in a corner:
+    the points, values, counts and final simplex are the oracle's."""
+    def f(u):
+        r = sum((u[k] - 0.3 * k) ** 2 * (1 + k) for k in range(n))
+        return math.nan if u[0] > 1.5 else math.floor(8.0 * r) / 8.0
+
+    rng = np.random.default_rng(n)
+    sim0 = np.concatenate([rng.uniform(-1.0, 2.0, (n + 1, n))])
+    seen = []
+    _, _, nf, it, sim, fv = nelder_mead(lambda u: (seen.append(tuple(u)), f(u))[1], sim0.tolist(), max_fun_evals=400,
+                                        max_iter=60, tol_fun=0.0, tol_x=1e-6)
+    esim, efv, enf, eit, fed, hits = _run_follow_ups(harness, f, sim0, 60, 0.0, 1e-6)
+    assert fed == seen and (enf, eit) == (nf, it)
+    assert np.array_equal(esim, np.array(sim)) and np.array_equal(efv, np.array(fv), equal_nan=True)
+    assert nf > 2 * n + 10
+
+
+@pytest.mark.parametrize("n", [1, 3, 6, 8])
+def test_stopping_test_sees_every_coordinate(harness, n):
+    """A spread of 1 in any one coordinate of any vertex keeps the method
+    going at TolX = 0.5, one of 0.25 ends it before its first iteration."""
+    for c in range(n):
+        for spread, iterations in ((1.0, 2), (0.25, 1)):
+            sim0 = np.zeros((n + 1, n))
+            sim0[1 + (c + 1) % n, c] = spread
+            _, _, nf, it, fed, _ = _run_follow_ups(harness, lambda u: 0.0, sim0, 2, 1.0, 0.5)
+            _, _, onf, oit, _, _ = nelder_mead(lambda u: 0.0, sim0.tolist(), max_iter=2, tol_fun=1.0, tol_x=0.5)
+            assert (nf, it) == (onf, oit) and it == iterations, (c, spread)
 
 
 def test_nan_vertex_sorts_last(harness):
