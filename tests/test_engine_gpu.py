@@ -632,9 +632,10 @@ def test_every_pinned_launch_configuration_gives_identical_results(engine):
     """Each launch configuration the autotuner can choose, pinned in turn:
     waves per block x XCD mapping for the median kernel, and also x bit mask /
     distance keys / tiled bit mask for the counts-only CSR and grid kernels;
-    every one equals the default configuration bit for bit (forward_comp,
-    compete_csr and index_seeds on a 256^2 x 19 scene, including a stack whose
-    sides are not multiples of the 32-pixel tile)."""
+    every one equals the default configuration (forward_comp: the plain kernel)
+    bit for bit (forward_comp, compete_csr and index_seeds on a 256^2 x 19
+    scene, including a stack whose sides are not multiples of the 32-pixel
+    tile)."""
     from grainrecon_amd import _lib as L
 
     for det in (256, 250):
@@ -653,15 +654,18 @@ def test_every_pinned_launch_configuration_gives_identical_results(engine):
         try:
             for k in range(3):
                 engine.set_launch_config(k, 4, L.MASK_BITS, False)
-            ref = engine.forward_comp(pos, q)
+            # up to 2560 evaluations are shared among a block's waves whatever is pinned
+            q_fc = np.vstack([q, scenes.random_quats(rng, 2000)])
+            ref = engine.forward_comp(pos, q_fc, L.METHOD_PLAIN)
             ref_c = engine.compete_csr(cpos, rows, cands, 8, 0.002)
             ref_i = engine.index_seeds(seeds, nr_seed=6)
             print(f"det {det}: default configuration done", flush=True)
             for xcd in (False, True):
                 for wpb in (8, 4, 2, 1):
                     engine.set_launch_config(0, wpb, L.MASK_BITS, xcd)
-                    for x, y in zip(engine.forward_comp(pos, q), ref):
-                        np.testing.assert_array_equal(x, y)
+                    for n in (2000, 2561, len(q_fc)):
+                        for x, y in zip(engine.forward_comp(pos, q_fc[:n]), ref):
+                            np.testing.assert_array_equal(x, y[:n])
                     for mask in (L.MASK_BITS, L.MASK_KEYS, L.MASK_TILED):
                         engine.set_launch_config(1, wpb, mask, xcd)
                         engine.set_launch_config(2, wpb, mask, xcd)
@@ -678,9 +682,11 @@ def test_every_pinned_launch_configuration_gives_identical_results(engine):
 
 def test_small_launches_take_smaller_blocks(engine):
     """With 8 waves per block pinned, launches of fewer evaluations than a
-    block has waves (1 to 9 orientations: 4 or 12 scratch slots) run in
-    smaller blocks; every result equals the oracle, for the one-voxel median
-    kernel, its allocation-free entry and the counts-only CSR kernel."""
+    block has waves (1 to 9 orientations): every result equals the oracle, for
+    the one-voxel median kernel and its allocation-free entry, which share
+    each evaluation among four waves, and the counts-only CSR kernel, which
+    runs one wave per block.  (Blocks made smaller for want of scratch slots:
+    test_noalloc_with_four_key_lists.)"""
     from grainrecon_amd import _lib as L
 
     s = scenes.make_scene(seed=87, ngrains=2, spread_mm=0.03, nrot=19, det=128, pixel_mm=6.72e-3 * 8)

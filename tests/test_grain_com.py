@@ -1,6 +1,8 @@
 """Grain centre-of-mass fit (fit_grain_COM.m): u2euler_corr and the
 objective pinned on the CPU, the batched GPU fit (grs_fit_grain_com) against
 the sequential oracle fit."""
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -83,3 +85,54 @@ def test_fit_grain_com_equals_oracle(engine, scene):
 
     with pytest.raises(GrsError):
         engine.fit_grain_com(sets, max_iter=100001)
+
+
+def _half_integer_geometry(s, rows, x):
+    """The geometry with the detector centre moved so that pair 0's spot at x
+    lies on a half-integer of dety and pair 1's on one of detz (to the last
+    bits: found by bisection on the rounded pixel's distance)."""
+    def moved(dy, dz):
+        return dataclasses.replace(s.geo, dety0=s.geo.dety0 + dy, detz0=s.geo.detz0 + dz)
+
+    def edge(f):
+        lo, hi = 0.0, 1.0  # one step of the rounded pixel lies between
+        a = f(lo)
+        assert f(hi) != a
+        while (lo + hi) / 2 not in (lo, hi):
+            mid = (lo + hi) / 2
+            if f(mid) == a:
+                lo = mid
+            else:
+                hi = mid
+        return hi
+
+    far = rows[:2].copy()
+    far[:, 17:19] = 1e4  # the distance moves with every step
+    dy = edge(lambda t: GC.objective(moved(t, 0.0), far[:1], x))
+    dz = edge(lambda t: GC.objective(moved(dy, t), far[1:2], x))
+    return moved(dy, dz)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("exact", [False, True])
+def test_fit_grain_com_pair_counts(engine, scene, exact):
+    """Pair counts around those up to which the distances of 7, 6 and 4
+    points stay in LDS (877, 1024 and 1536 of 6144), so that a fit changes
+    between LDS and device memory; with `exact` also spots on half-integers at
+    the start, whose rounding the exact pipeline decides."""
+    s = scene
+    rows = np.concatenate([_rows(s, 0, _frames_at_pixels(s, 0))] * 100)
+    geo = s.geo
+    if exact:
+        x0 = np.concatenate([rows[0, 9:12], GC.u2euler_corr(rows[0, 0:9].reshape(3, 3, order="F"))])
+        geo = _half_integer_geometry(s, rows, x0)
+    engine.set_geometry(geo, s.hkl, s.rot)
+    engine.set_distance_stack(s.proj)
+    counts = (1, 2, 877, 878, 1024, 1025, 1536, 1537)
+    assert rows.shape[0] >= counts[-1]
+    sets = [rows[:n] for n in counts]
+    x, fv, nf, it = engine.fit_grain_com(sets, max_fun_evals=60)
+    for m, r in enumerate(sets):
+        rx, rf, rnf, rit = GC.fit_grain_com(geo, r, max_fun_evals=60)
+        np.testing.assert_array_equal(x[m], rx)
+        assert fv[m] == rf and nf[m] == rnf and it[m] == rit, counts[m]

@@ -8,7 +8,7 @@ leak into the second.  The scene selects ~4,000 events per evaluation (512^2
 detector of 27 um pixels, 361 omega, 140 reflections), so every wave keeps
 its median keys in its scratch key list.  A geometry whose events per
 evaluation leave room for fewer than 4 key lists is rejected before any
-launch.
+launch; with room for just 4 of them blocks of 8 waves are made smaller.
 """
 import numpy as np
 import pytest
@@ -92,3 +92,36 @@ def test_noalloc_rejects_geometry_beyond_scratch(engine):
     finally:
         for d in bufs + [d_q]:
             engine.device_free(d)
+
+
+@pytest.mark.parametrize("nrot, lists", [(17_000, 4), (13_000, 4), (8_000, 8)])
+def test_noalloc_with_four_key_lists(engine, nrot, lists):
+    """240 reflections x 17,000 or 13,000 omega leave room for 4 waves' key
+    lists (5 with the rest unused), 8,000 for 8: with 8 waves per block pinned,
+    2,561 orientations (more than are shared among waves) run in one block of
+    4 or 8 waves; every row equals the oracle's of its orientation."""
+    geo = labdct_geometry(a=2.8665, lattice="I", det_pixels=16, pixel_mm=6.72e-3 * 64)
+    hkl = np.concatenate([k * cubic_hkl("I", 6) for k in (1, 2, 3)])[:240]
+    rot = np.linspace(0.0, 360.0, nrot)
+    rng = np.random.default_rng(nrot)
+    key_bytes = (64 << 20) - ((512 + 76 * 16384 + 255) & ~255)
+    assert key_bytes // (4 * 240 * nrot) // 4 * 4 == lists
+    engine.set_geometry(geo, hkl, rot)
+    proj = rng.integers(0, 40, (16, 16, nrot)).astype(np.float32)
+    engine.set_distance_stack(proj)
+    pos, q9 = [0.01, -0.02, 0.005], scenes.random_quats(rng, 9)
+    q9[4, 1:] = [0.8, 0.6, 0.3]
+    ora = oracle.or_space_comp(geo, oracle.Stack(proj), pos, q9, rot, hkl, nthreads=8)
+    ref = (ora[:, 0].astype(np.int32), ora[:, 1].astype(np.int32), ora[:, 2], ora[:, 3].astype(np.float32))
+    assert ref[0].max() > 4096 and ref[0][4] == 0
+    N = 2561
+    pick = np.where(np.arange(N) % 40 < 2, np.arange(N) % 9, 4)  # most are skipped rows: the others take long
+    d_q = engine.to_device(q9[pick])
+    engine.set_launch_config(0, 8, _lib.MASK_BITS, False)
+    try:
+        got = _run(engine, engine.forward_comp_device_noalloc, pos, d_q, N, N)
+    finally:
+        engine.set_launch_config(0, 0)
+        engine.device_free(d_q)
+    for r, g in zip(ref, got):
+        assert np.array_equal(_bits(r)[pick], _bits(g))
