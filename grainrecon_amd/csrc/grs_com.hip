@@ -82,11 +82,19 @@ __device__ __forceinline__ double com_pair_dist(const grs_dgeo *g, const double 
  * waits on every load of them); more pairs than fit use device memory */
 #define COM_LDS_DIST 6144
 
+/* pairs up to which a reflection is evaluated together with its follow-ups:
+ * a round then takes about as long for four points as for one; beyond, the
+ * distances of the two or three points that the method does not request cost more
+ * than the rounds saved.  Three fits, with and without, in ms: 373 pairs 1.61
+ * and 1.76, 724 2.80 and 2.84, 746 2.43 and 2.49, 1,119 3.42 and 3.25, 1,448 5.77 and
+ * 4.52, 2,984 9.74 and 7.16; one of 20,000 474 and 240. */
+#define COM_FOLLOW_PAIRS 1024
+
 /* One block per fit m: the first wave steps the Nelder-Mead state machine
- * (started on the host) in registers (nm_lanes); for the requested points - a
- * reflection together with the three points its value can lead to
- * (grs_nm::points), so that an iteration is one round - the point
- * coordinates and the six cosines and sines of each point's angles are
+ * (started on the host) in registers (nm_lanes); for the requested points - up
+ * to COM_FOLLOW_PAIRS pairs a reflection together with the three points its
+ * value can lead to (grs_nm::points), so that an iteration is one round - the
+ * point coordinates and the six cosines and sines of each point's angles are
  * computed one per thread, the first threads build each point's U and SUB,
  * all threads compute the (point, pair) distances, and thread p adds point
  * p's distances in pair order, so ErrMean is the sequential sum over the
@@ -94,8 +102,8 @@ __device__ __forceinline__ double com_pair_dist(const grs_dgeo *g, const double 
  * sequential sum of a few hundred values, the simplex step).  Three grains of
  * about 400 pairs: 1.2 ms for the launch; 1.6 with the simplex stepped in
  * LDS; 2.4 with also the exact pipeline for every distance, the distances
- * in device memory and a round per requested point.  The state machine ends after at most max_iter iterations,
- * so every block exits. */
+ * in device memory and a round per requested point.  The state machine ends
+ * after at most max_iter iterations, so every block exits. */
 __global__ __launch_bounds__(COM_THREADS) void k_com_nm(const grs_dgeo *g, const double *rows, const int64_t *rptr,
                                                         const double *cs, double *dis, grs_nm *nms) {
   GRS_NO_CONTRACT
@@ -114,6 +122,7 @@ __global__ __launch_bounds__(COM_THREADS) void k_com_nm(const grs_dgeo *g, const
   const int64_t m = blockIdx.x;
   const int64_t r0 = rptr[m];
   const int n = (int)(rptr[m + 1] - r0);
+  const bool follow_ups = n <= COM_FOLLOW_PAIRS;
   if (t == 0) {
     *nm = nms[m];
     sg = *g;
@@ -121,7 +130,7 @@ __global__ __launch_bounds__(COM_THREADS) void k_com_nm(const grs_dgeo *g, const
   }
   __syncthreads();
   for (;;) {
-    if (t == 0) npts = nm->points();
+    if (t == 0) npts = follow_ups ? nm->points() : nm->npend;
     __syncthreads();
     const int np = npts;
     if (np == 0) break;
@@ -180,7 +189,7 @@ __global__ __launch_bounds__(COM_THREADS) void k_com_nm(const grs_dgeo *g, const
     __syncthreads();
     if (t < 64) { /* the first wave steps the method */
       nm_lanes<6> L(nm, t);
-      L.step(fs);
+      L.step(fs, follow_ups);
       L.store();
     }
     __syncthreads();

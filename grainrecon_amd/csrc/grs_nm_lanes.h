@@ -14,19 +14,19 @@
 #define GRS_NM_LANES_FN inline
 #endif
 
-/* The steps of the method for N coordinates, taken by the 64 lanes of one wave in
- * registers: lane k holds coordinate k of the simplex, xbar and xr, and every
- * lane holds the values, counts and state and takes the method's decisions
- * on them.  The constructor and store() move the state between the registers and the
- * grs_nm in LDS around a step (so that it costs no registers between steps),
- * each one round of independent accesses; all loops are unrolled over N.  The
- * results are the sequential method's, bit for bit: its statements for the
- * coordinate, the stopping test's largest vertex distance and largest
- * coordinate reduced across the lanes (a maximum is exact), and the stable
- * insertion sort as exchanges of neighbours.  Stepped by one lane on the grs_nm in
- * LDS, one dependent access
- * after the other, a step of six coordinates with its follow-up took 11,900
- * cycles; three fits of six coordinates went from 1.61 to 1.22 ms with this. */
+/* The steps of the method for N coordinates, taken by the 64 lanes of one
+ * wave in registers: lane k holds coordinate k of the simplex, xbar and xr,
+ * and every lane holds the values, counts and state and takes the method's
+ * decisions on them.  The constructor and store() move the state between the
+ * registers and the grs_nm in LDS around a step (so that it costs no registers
+ * between steps), each one round of independent accesses; all loops are
+ * unrolled over N.  The results are the sequential method's, bit for bit: its
+ * statements for the coordinate, the stopping test's largest vertex distance
+ * and largest coordinate reduced across the lanes (a maximum is exact), and
+ * the stable insertion sort as exchanges of neighbours.  Stepped by one lane
+ * on the grs_nm in LDS, one dependent access after the other, a step of six
+ * coordinates with its follow-up took 11,900 cycles; three fits of six
+ * coordinates went from 1.61 to 1.22 ms with this. */
 template <int N>
 struct nm_lanes {
   grs_nm *s;
@@ -224,13 +224,14 @@ struct nm_lanes {
   }
 
   /* a step with the values f (in LDS) of grs_nm's points: a reflection's
-   * follow-ups stand behind its own value.  One call
-   * site of feed, so that it is inlined and the state stays in registers. */
-  GRS_NM_LANES_FN void step(const double *f) {
+   * follow-ups stand behind its own value (without follow_ups: of the
+   * requested points alone).  One call site of feed, so that it is inlined
+   * and the state stays in registers. */
+  GRS_NM_LANES_FN void step(const double *f, bool follow_ups = true) {
     for (int q = 0;;) {
       const bool refl = st == grs_nm::REFLECT;
       feed(f + q);
-      if (!refl) return;
+      if (!refl || !follow_ups) return;
       q = st == grs_nm::EXPAND ? 1 : st == grs_nm::CONTRACT_OUT ? 2 : st == grs_nm::CONTRACT_IN ? 3 : 0;
       if (q == 0) return;
     }

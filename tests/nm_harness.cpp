@@ -33,8 +33,8 @@ static double __shfl(double x, int lane, int) { return exchange(x, lane); }
 
 typedef double (*nm_objective)(const double *u, int n);
 
-/* one step of the wave: step() takes the values of all points, feed() those
- * of the requested ones alone */
+/* one step of the wave on the values of all points, or of the requested ones
+ * alone */
 template <int N>
 static void wave_step(grs_nm *s, const double *f, bool follow_ups) {
   pthread_barrier_init(&g_meet, nullptr, LANES);
@@ -43,8 +43,7 @@ static void wave_step(grs_nm *s, const double *f, bool follow_ups) {
     lane[l] = std::thread([=]() {
       g_lane = l;
       nm_lanes<N> L(s, l);
-      if (follow_ups) L.step(f);
-      else L.feed(f);
+      L.step(f, follow_ups);
       /* the lanes store one after the other */
       for (int t = 0; t < LANES; t++) {
         pthread_barrier_wait(&g_meet);

@@ -116,9 +116,10 @@ def _half_integer_geometry(s, rows, x):
 @pytest.mark.gpu
 @pytest.mark.parametrize("exact", [False, True])
 def test_fit_grain_com_pair_counts(engine, scene, exact):
-    """Pair counts around those up to which the distances of 7, 6 and 4
-    points stay in LDS (877, 1024 and 1536 of 6144), so that a fit changes
-    between LDS and device memory; with `exact` also spots on half-integers at
+    """Pair counts around those up to which the distances of 7, 6, 4 and one
+    points stay in LDS (877, 1024, 1536 and 6144), so that a fit changes
+    between LDS and device memory, and up to which a reflection's follow-ups
+    are evaluated with it (1024); with `exact` also spots on half-integers at
     the start, whose rounding the exact pipeline decides."""
     s = scene
     rows = np.concatenate([_rows(s, 0, _frames_at_pixels(s, 0))] * 100)
@@ -128,7 +129,7 @@ def test_fit_grain_com_pair_counts(engine, scene, exact):
         geo = _half_integer_geometry(s, rows, x0)
     engine.set_geometry(geo, s.hkl, s.rot)
     engine.set_distance_stack(s.proj)
-    counts = (1, 2, 877, 878, 1024, 1025, 1536, 1537)
+    counts = (1, 2, 877, 878, 1024, 1025, 1536, 1537, 6144, 6145)
     assert rows.shape[0] >= counts[-1]
     sets = [rows[:n] for n in counts]
     x, fv, nf, it = engine.fit_grain_com(sets, max_fun_evals=60)
