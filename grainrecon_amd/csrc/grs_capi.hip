@@ -985,24 +985,37 @@ grs_status grs_grow_indexed_region(grs_ctx *c, const double *vox, int64_t M, con
   grs_status s = check_ready(c);
   if (s != GRS_OK) return s;
   if (M == 0) return GRS_OK;
-  ENSURE(c, c->d_sub, sizeof(double) * 9);
-  ENSURE(c, c->d_valid, sizeof(int32_t));
-  ENSURE(c, c->d_p1, sizeof(double) * (14 + 9)); /* param1, then U */
-  double p1U[14 + 9];
+  double p1U[14 + 9]; /* param1, then U */
   std::memcpy(p1U, p1, sizeof(double) * 14);
   std::memcpy(p1U + 14, U, sizeof(double) * 9);
-  HIPCHK(c, hipMemcpyAsync(c->d_p1.p, p1U, sizeof(p1U), hipMemcpyHostToDevice, c->st));
-  HIPCHK(c, grs_launch_sub_from_U(P<grs_dgeo>(c->d_geo), P<double>(c->d_p1) + 14, 1, P<double>(c->d_sub),
-                                  P<int32_t>(c->d_valid), c->st));
+  bool up = false;
   const int64_t chunk = voxel_chunk(c);
   for (int64_t b = 0; b < M; b += chunk) {
     const int64_t m = M - b < chunk ? M - b : chunk;
-    /* only voxels inside the mask are scored: counted here while that is
+    /* only voxels inside the mask are scored: the rows before the first of
+     * them are written here (rows without any need no device: 0.1 ms for
+     * 100,000 instead of 0.6), the others are counted here while that is
      * quicker than a round trip (a pass over the rows' mask column) */
+    int64_t in = b;
+    for (; in < b + m && !(vox[6 * in + 4] > 0.0); in++) {
+      double *o = out + 7 * in;
+      for (int j = 0; j < 3; j++) o[j] = vox[6 * in + j];
+      for (int j = 3; j < 7; j++) o[j] = 0.0;
+    }
+    if (in == b + m) continue;
+    if (!up) {
+      ENSURE(c, c->d_sub, sizeof(double) * 9);
+      ENSURE(c, c->d_valid, sizeof(int32_t));
+      ENSURE(c, c->d_p1, sizeof(p1U));
+      HIPCHK(c, hipMemcpyAsync(c->d_p1.p, p1U, sizeof(p1U), hipMemcpyHostToDevice, c->st));
+      HIPCHK(c, grs_launch_sub_from_U(P<grs_dgeo>(c->d_geo), P<double>(c->d_p1) + 14, 1, P<double>(c->d_sub),
+                                      P<int32_t>(c->d_valid), c->st));
+      up = true;
+    }
     int64_t E = -1;
     if (m <= 16384) {
       E = 0;
-      for (int64_t i = b; i < b + m; i++) E += vox[6 * i + 4] > 0.0 ? 1 : 0;
+      for (int64_t i = in; i < b + m; i++) E += vox[6 * i + 4] > 0.0 ? 1 : 0;
     }
     const int64_t nb = grs_grow_blocks(m);
     ENSURE(c, c->d_rows, sizeof(double) * 6 * m);

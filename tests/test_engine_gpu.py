@@ -276,6 +276,34 @@ def test_grow_row_counts(engine, M):
         assert (got[mask == 1, 3] > 0).all()
 
 
+@pytest.mark.parametrize("last", [False, True])
+def test_grow_rows_outside_the_mask(last):
+    """Rows of which none is inside the mask take no device memory (they went
+    up and down for nothing); with the last one inside, all are listed."""
+    from grainrecon_amd import Engine
+
+    s = scenes.make_scene(seed=41, ngrains=2, spread_mm=0.02)
+    rng = np.random.default_rng(5)
+    M = 200_000
+    vox = np.column_stack([rng.integers(14, 27, (M, 2)), rng.integers(16, 25, M), rng.uniform(0, 0.6, M), np.zeros(M),
+                           rng.uniform(0, 30, M)]).astype(float)
+    vox[::3, 4] = -1.0
+    vox[1::3, 4] = np.nan
+    vox[-1, 4] = float(last)
+    e = Engine(0)
+    try:
+        e.set_geometry(s.geo, s.hkl, s.rot)
+        e.set_distance_stack(s.proj)
+        free = scenes.free_device_memory(e)
+        got = e.grow_indexed_region(vox, s.U[0], _p1())
+        taken = free - scenes.free_device_memory(e)
+        assert taken > 20 << 20 if last else taken < 4 << 20
+    finally:
+        e.close()
+    assert np.array_equal(got[:, :3], vox[:, :3]) and not got[:-1, 3:].any()
+    assert np.array_equal(_bits(got[-2:]), _bits(oracle.grow(s.geo, s.stack, vox[-2:], s.U[0], s.rot, s.hkl, _p1())))
+
+
 @pytest.mark.parametrize("nr, k", [(0, 255), (0, 256), (0, 257), (5, 1), (6, 1)])
 def test_compete_csr_evaluations_per_voxel(engine, nr, k):
     """255, 256, 257, 216 and 343 evaluations (samples x candidates) of each
