@@ -2831,7 +2831,7 @@ grs_status grs_distance_from_mask(grs_ctx *c) {
   const int64_t nz = c->mnz, ny = c->mny, nr = c->mnrot, n = nz * ny * nr;
   ENSURE(c, c->d_keys, sizeof(float) * n);
   if (grs_edt_tile_width(nz, ny, nr) > 0) {
-    ENSURE(c, c->d_g1, (size_t)grs_edt_work_bytes(nz, ny * nr));
+    ENSURE(c, c->d_g1, (size_t)grs_edt_work_bytes(nz, ny, nr));
     HIPCHK(c, grs_launch_edt(P<uint8_t>(c->d_mask), nz, ny, nr, c->d_g1.p, P<float>(c->d_keys), c->st));
   } else {
     ENSURE(c, c->d_g1, sizeof(int32_t) * n);

@@ -184,7 +184,7 @@ hipError_t grs_launch_sim_events(const grs_dgeo *d_g, const double *d_pos, const
 /* exact distance transform at the sides grs_edt_tile_width accepts (nonzero);
  * d_work holds grs_edt_work_bytes */
 int grs_edt_tile_width(int64_t nz, int64_t ny, int64_t nslices);
-int64_t grs_edt_work_bytes(int64_t nz, int64_t nlines);
+int64_t grs_edt_work_bytes(int64_t nz, int64_t ny, int64_t nslices);
 hipError_t grs_launch_edt(const uint8_t *d_mask, int64_t nz, int64_t ny, int64_t nslices, void *d_work, float *d_out,
                           hipStream_t st);
 hipError_t grs_launch_edt_cols(const uint8_t *d_mask, int64_t nz, int64_t ncols, int32_t *d_g1, hipStream_t st);
