@@ -1,4 +1,6 @@
 """Candidate generation: ori_local_sampling.m and find_neighbor_ORs.m."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -160,6 +162,27 @@ def test_engine_find_neighbor_ors_matches_oracle(engine):
         ids2, ind2 = oracle.find_neighbor_ors(gid, vox, radius, nr_max)
         np.testing.assert_array_equal(ids, ids2)
         np.testing.assert_array_equal(ind, ind2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 4228, 4229])
+def test_engine_find_neighbor_ors_list_sizes(engine, M):
+    """Lists packed by the host (up to 512 KB: 4,228 voxels of 30 ids and a
+    count) and on the device; the caller's memory behind the ids stays as it
+    was."""
+    rng = np.random.default_rng(M)
+    gid = _volume(rng, (30, 23, 19), 0.05, 400)
+    vox = np.stack([rng.integers(1, n + 1, M) for n in gid.shape], axis=1)
+    want = oracle.find_neighbor_ors(gid, vox, 3, 30)
+    for a, b in zip(engine.find_neighbor_ors(gid, vox, 3), want):
+        np.testing.assert_array_equal(a, b)
+    ids, ind, n = np.full(30 * M, -7, np.int32), np.zeros((M, 2), np.int64), ctypes.c_int64()
+    flat, v = np.ascontiguousarray(gid.reshape(-1, order="F")), np.ascontiguousarray(vox, dtype=np.int32)
+    p = lambda a: a.ctypes.data_as(ctypes.POINTER(np.ctypeslib.as_ctypes_type(a.dtype)))  # noqa: E731
+    engine._chk(engine._lib.grs_find_neighbor_ors(engine._h, p(flat), *gid.shape, p(v), M, 3, 30, p(ids), p(ind),
+                                                  ctypes.byref(n)))
+    assert n.value == want[0].size and np.array_equal(ids[:n.value], want[0]) and (ids[n.value:] == -7).all()
+    np.testing.assert_array_equal(ind, want[1])
 
 
 @pytest.mark.gpu
