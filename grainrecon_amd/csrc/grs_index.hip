@@ -36,11 +36,6 @@
 
 #define GRS_CLS_NAN (1ull << 31)
 
-__global__ void k_fill_u32(uint32_t *p, int64_t n, uint32_t v) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-
 /* ---------------------------------------------------------------------- */
 /* k_topk: the k largest of n unique keys per segment, sorted descending    */
 
@@ -285,12 +280,6 @@ __global__ void k_seed_out(const unsigned long long *topkey, const int32_t *ns1,
 /* launchers                                                               */
 
 static unsigned grid_for(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
-
-hipError_t grs_launch_fill_u32(uint32_t *d_p, int64_t n, uint32_t v, hipStream_t st) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(n, 256)), dim3(256), 0, st, d_p, n, v);
-  return hipGetLastError();
-}
 
 hipError_t grs_launch_topk(const unsigned long long *d_keys, int64_t segs, int64_t n, int64_t seg_stride, int32_t k,
                            unsigned long long *d_out, hipStream_t st) {

@@ -1571,6 +1571,11 @@ __global__ __launch_bounds__(64 * GRS_FIT_TEAM * GRS_FIT_PTS, GRS_FAST_MIN_WAVES
 /* ---------------------------------------------------------------------- */
 /* batched compete: device-side steps between and after the two launches   */
 
+__global__ void k_fill_u32(uint32_t *p, int64_t n, uint32_t v) {
+  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = v;
+}
+
 __global__ void k_fill_u64(unsigned long long *p, int64_t n, unsigned long long v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -1740,6 +1745,90 @@ __global__ __launch_bounds__(256) void k_plain(grs_eval_args a, int64_t T) {
     a.out_C[e] = (double)ni / (double)ns;
     a.out_med[e] = med;
   }
+}
+
+/* ---------------------------------------------------------------------- */
+/* voxel rows of cuda_grow_indexed_region                                  */
+
+/* The rows [x y z C mask DisMedian] stay on the device as they came: block b
+ * of GROW_T rows counts its rows inside the mask, k_grow_list gives row i its
+ * place among the scored ones (slot, -1 outside the mask) and writes the
+ * position there, k_grow_out forms the 7 output values and the growth flag.
+ * Bound: 48 bytes in and 56 out per row; on the host the same loops and their
+ * copies took about 40 ms for 3.2M rows, the three kernels take 0.28 ms.
+ * They stand in this file because a process loads each file's kernels at the
+ * first launch of one of them, 0.8 ms of its first growth call. */
+#define GROW_T 256
+
+__device__ __forceinline__ int64_t grow_block_sum(int32_t v, int32_t *part) {
+  const uint64_t lanes = 64;
+  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, (int)lanes);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  int64_t s = 0;
+  for (int k = 0; k < GROW_T / 64; k++) s += part[k];
+  __syncthreads();
+  return s;
+}
+
+__global__ __launch_bounds__(GROW_T) void k_grow_count(const double *rows, int64_t M, int32_t *count) {
+  __shared__ int32_t part[GROW_T / 64];
+  const int64_t i = (int64_t)blockIdx.x * GROW_T + threadIdx.x;
+  const int64_t n = grow_block_sum(i < M && rows[6 * i + 4] > 0.0 ? 1 : 0, part);
+  if (threadIdx.x == 0) count[blockIdx.x] = (int32_t)n;
+}
+
+/* count: rows inside the mask per block, or nullptr when every row is inside;
+ * total receives their sum */
+__global__ __launch_bounds__(GROW_T) void k_grow_list(const double *rows, int64_t M, const double *p1,
+                                                      const int32_t *count, double *pos, int32_t *slot,
+                                                      int64_t *total) {
+  __shared__ int32_t part[GROW_T / 64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t b = blockIdx.x, i = b * GROW_T + threadIdx.x;
+  int64_t k = i;
+  bool in = i < M;
+  if (count) {
+    int32_t before = 0;
+    for (int64_t j = threadIdx.x; j < b; j += GROW_T) before += count[j];
+    const int64_t base = grow_block_sum(before, part);
+    in = in && rows[6 * i + 4] > 0.0;
+    const uint64_t m = __ballot(in);
+    if (lane == 0) part[wv] = (int32_t)__popcll(m);
+    __syncthreads();
+    k = base + __popcll(lane == 0 ? 0ull : m & (~0ull >> (64 - lane)));
+    for (int w = 0; w < wv; w++) k += part[w];
+    if (total && b == (int64_t)gridDim.x - 1 && threadIdx.x == 0) *total = base + count[b];
+  }
+  if (i < M) slot[i] = in ? (int32_t)k : -1;
+  if (in) grs_voxel_pos(rows[6 * i], rows[6 * i + 1], rows[6 * i + 2], p1, pos + 3 * k);
+}
+
+__global__ __launch_bounds__(GROW_T) void k_grow_out(const double *rows, int64_t M, const double *p1,
+                                                     const int32_t *slot, const int32_t *ns, const int32_t *ni,
+                                                     const double *C, const float *med, double *out) {
+  GRS_NO_CONTRACT
+  const int64_t i = (int64_t)blockIdx.x * GROW_T + threadIdx.x;
+  if (i >= M) return;
+  const double *v = rows + 6 * i;
+  double *o = out + 7 * i;
+  o[0] = v[0];
+  o[1] = v[1];
+  o[2] = v[2];
+  const int32_t k = slot[i];
+  if (k < 0) {
+    o[3] = o[4] = o[5] = o[6] = 0.0;
+    return;
+  }
+  const double Cn = C[k], dm = (double)med[k];
+  /* min([DisMedian maxDmedian]) with MATLAB's NaN rule */
+  const double a = v[5], b = p1[13];
+  const double lim = a != a ? b : (b != b ? a : (b < a ? b : a));
+  const bool flag = (Cn > v[3] && dm <= lim) && (Cn >= p1[11] * (1.0 - p1[12]));
+  o[3] = (double)ns[k];
+  o[4] = (double)ni[k];
+  o[5] = dm;
+  o[6] = flag ? 1.0 : 0.0;
 }
 
 /* ---------------------------------------------------------------------- */
@@ -1937,7 +2026,11 @@ static hipError_t launch_fast_impl(const grs_eval_args *a, int32_t H, int64_t n_
  * lose.  A one-voxel call of 100, 300, 729, 1500, 2187, 4000 orientations (86
  * reflections, 181 angles; whole call on resident buffers, us): a wave each
  * 44, 73, 69, 78, 75, 71; two 37, 40, 44, 54, 70, 86; four 35, 38, 44, 66, 81,
- * 118; eight 34, 41, 58, 86, 112, 179.  The order is the same with 64 x 361. */
+ * 118; eight 34, 41, 58, 86, 112, 179.  The order is the same with 64 x 361.
+ * Growth, compete pairs and CSR winners, which have no beam table in LDS,
+ * cross near 2,000: calls of 1,500 take 139, 152 and 271 with two waves, 145,
+ * 165 and 293 with a wave each, of 2,560 160, 182 and 313 against 148, 169
+ * and 295. */
 static int fast_team(int64_t n) { return n <= 512 ? 4 : n <= 2560 ? 2 : 1; }
 
 template <int MAP>
@@ -2012,6 +2105,26 @@ hipError_t grs_launch_plain(const grs_eval_args *a, int64_t T, hipStream_t st) {
   return hipGetLastError();
 }
 
+int64_t grs_grow_blocks(int64_t M) { return (M + GROW_T - 1) / GROW_T; }
+
+hipError_t grs_launch_grow_list(const double *d_rows, int64_t M, const double *d_p1, int32_t *d_count, double *d_pos,
+                                int32_t *d_slot, int64_t *d_total, hipStream_t st) {
+  if (M <= 0) return hipSuccess;
+  const dim3 grid((unsigned)grs_grow_blocks(M));
+  if (d_count) hipLaunchKernelGGL(k_grow_count, grid, dim3(GROW_T), 0, st, d_rows, M, d_count);
+  hipLaunchKernelGGL(k_grow_list, grid, dim3(GROW_T), 0, st, d_rows, M, d_p1, d_count, d_pos, d_slot, d_total);
+  return hipGetLastError();
+}
+
+hipError_t grs_launch_grow_out(const double *d_rows, int64_t M, const double *d_p1, const int32_t *d_slot,
+                               const int32_t *d_ns, const int32_t *d_ni, const double *d_C, const float *d_med,
+                               double *d_out, hipStream_t st) {
+  if (M <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_grow_out, dim3((unsigned)grs_grow_blocks(M)), dim3(GROW_T), 0, st, d_rows, M, d_p1, d_slot,
+                     d_ns, d_ni, d_C, d_med, d_out);
+  return hipGetLastError();
+}
+
 hipError_t grs_launch_compete_list(const double *d_vox, int64_t M, const int64_t *d_rs, const double *d_ids,
                                    int64_t n_id, int64_t G, const double *d_p1, double *d_pos, int32_t *d_evox,
                                    int32_t *d_eu, unsigned long long *d_bad, hipStream_t st) {
@@ -2057,9 +2170,15 @@ hipError_t grs_launch_check_keys(const uint32_t *d_keys, int64_t n, uint32_t *d_
 
 int64_t grs_fast_wave_slots(int device) {
   (void)device;
-  /* upper bound over the instantiations (at most 32 resident waves per
-   * CU): the scratch is indexed by wave */
+  /* the scratch is indexed by wave: no launch has more than this, twice the
+   * waves that a CU can hold (16 at 128 VGPRs) */
   return (int64_t)device_cus() * 64;
+}
+
+hipError_t grs_launch_fill_u32(uint32_t *d_p, int64_t n, uint32_t v, hipStream_t st) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(n, 256)), dim3(256), 0, st, d_p, n, v);
+  return hipGetLastError();
 }
 
 hipError_t grs_launch_fill_u64(unsigned long long *d_p, int64_t n, unsigned long long v, hipStream_t st) {
