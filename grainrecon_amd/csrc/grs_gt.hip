@@ -286,7 +286,12 @@ __device__ __forceinline__ void gt_vw(const double *P, grs_vw *v) {
 }
 
 #define GT_RING 128     /* candidate events queued per wave */
-#define GT_TAB_MAX 1024 /* reflections up to which a wave keeps its G table in LDS (36 bytes each) */
+/* Reflections up to which a wave keeps its G table in LDS (36 bytes each; 149 KB
+ * a block at 1024).  Four blocks, which the registers allow, share a CU up to
+ * about 270.  4,096 orientations, 181 angles, with and without the table, in ms: 86
+ * reflections 1.75 and 2.12, 172 2.9 and 3.5, 258 4.1 and 5.0, 344 7.3 and 6.3,
+ * 688 23.3 and 11.8. */
+#define GT_TAB_MAX 1024
 
 /* One wave per orientation.  About 10% of the (projection, reflection) events
  * can do anything: the expected count needs cos(beta) and lambda inside the

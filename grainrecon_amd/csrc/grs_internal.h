@@ -122,7 +122,7 @@ hipError_t grs_launch_sub_from_U(const grs_dgeo *d_g, const double *d_U, int64_t
 hipError_t grs_launch_sub_from_euler(const grs_dgeo *d_g, const double *d_euler, int64_t N, double *d_SUB,
                                      int32_t *d_valid, hipStream_t st);
 hipError_t grs_launch_omega_cs(const double *d_rot, int32_t nrot, double *d_cs, hipStream_t st);
-/* wpb: waves per block, 1, 2 or 4; n_waves: a multiple of 4 (wave slots of the scratch) */
+/* wpb: waves per block, 1, 2, 4 or 8; n_waves: a multiple of 4 (wave slots of the scratch) */
 hipError_t grs_launch_fast(const grs_eval_args *a, int32_t H, int64_t n_waves, int32_t wpb, hipStream_t st);
 hipError_t grs_launch_fast_counts(const grs_eval_args *a, int32_t H, int64_t n_waves, int32_t wpb, hipStream_t st);
 /* M orientation fits, a block each (k_fit_nm): a describes the voxels (pos,
